@@ -628,127 +628,238 @@ __global__ __launch_bounds__(256) void k_post_learned(SgDevView d, SgDevView dq,
 }
 
 // ---------------------------------------------------------------------------
-// Training (FP32).  One workgroup = TB samples: forward, loss, backward with LDS
-// activations; per-workgroup gradient written to its own slot, then reduced in a
-// fixed order and applied with Adam (deterministic).
+// Training (FP32).  One workgroup = TB samples: forward, loss, backward; per-workgroup
+// gradient written to its own slot, then reduced in a fixed order and applied with Adam
+// (deterministic).
+//
+// Every product runs on v_mfma_f32_16x16x4_f32 (FP32 operands and accumulators; lane
+// L = 16 g + c holds A[c][g], B[g][c] and D[4 g + r][c], r < 4).  Wave w owns the hidden
+// columns j = 16 w + c: its weight fragments load into registers at once, beside the
+// gathered rows, and its pre-activations stay in registers in the D layout, where they
+// are also the B operand (and, for dW3, the A operand) of the weight gradients when the
+// sum over samples takes sample 16 mt + 4 g + r as step (mt, r)'s index g.  Bound by the
+// chain of four products each way, not by FLOPs (1.2 MFLOP per workgroup): 256
+// workgroups take 15.4 us, where scalar loops over LDS took 30.8.
 // ---------------------------------------------------------------------------
 #define TB 32
+#define TRN_XP 34  // row pitches = 2 mod 32 floats: the 16 rows x 2 columns a half wave reads are 32 banks
+#define TRN_HP 66
+
+__device__ __forceinline__ sg_float4 mfma_f32(float a, float b, sg_float4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// sum over the four lane groups of a wave (lanes c, c + 16, c + 32, c + 48)
+__device__ __forceinline__ float sum_groups(float v) {
+  v += __shfl_xor(v, 16);
+  return v + __shfl_xor(v, 32);
+}
+
 __global__ __launch_bounds__(256) void k_mlp_train(const float *w, const float *X, const float *T, const int *idx,
                                                   int n_valid, int base, float inv_count, const float *norm,
                                                   float *grad_part, float *loss_part) {
-  __shared__ float sX[TB][28], sZ1[TB][64], sA1[TB][64], sZ2[TB][64], sA2[TB][64], sD[TB][4];
-  __shared__ float sLoss[256];
-  const int tid = threadIdx.x;
+  __shared__ float sX[TB][TRN_XP], sA1[TB][TRN_HP], sA2[TB][TRN_HP], sZ[TB][TRN_HP];
+  __shared__ float sD[TB][4];
+  __shared__ float sLoss[2];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int j = wv * 16 + c;
   const int s0 = base + blockIdx.x * TB;
-  for (int q = tid; q < TB * 28; q += 256) {
-    const int s = q / 28, i = q % 28;
-    const int gs = s0 + s;
-    const float raw = gs < n_valid ? X[(size_t)idx[gs] * 28 + i] : 0.0f;
-    sX[s][i] = (raw - norm[i]) * norm[28 + i];
-  }
-  __syncthreads();
   const float *W1 = w + SG_OFF_W1, *B1 = w + SG_OFF_B1, *W2 = w + SG_OFF_W2, *B2 = w + SG_OFF_B2;
   const float *W3 = w + SG_OFF_W3, *B3 = w + SG_OFF_B3;
-  for (int o = tid; o < TB * 64; o += 256) {
-    const int s = o / 64, j = o % 64;
-    float z = B1[j];
-    for (int i = 0; i < 28; i++) z += sX[s][i] * W1[i * 64 + j];
-    sZ1[s][j] = z;
-    sA1[s][j] = sg_silu(z);
+  // rows: thread q < 224 one float4 of row q / 7 (a row is 7 of them); the rest clear
+  // the pad columns
+  const int xs = tid < 224 ? tid / 7 : tid - 224, xq = tid < 224 ? tid % 7 : 0;
+  const int xr = s0 + xs < n_valid ? idx[s0 + xs] : -1;
+  // weights of this lane's hidden column
+  float w1[7], w2[16], w2t[16], w3b[16], w3r[3];
+#pragma unroll
+  for (int k = 0; k < 7; k++) w1[k] = W1[(4 * k + g) * 64 + j];
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    w2[k] = W2[(4 * k + g) * 64 + j];
+    w2t[k] = W2[j * 64 + 4 * k + g];
+    const float v = W3[(4 * k + g) * 3 + (c < 3 ? c : 0)];
+    w3b[k] = c < 3 ? v : 0.0f;
   }
-  __syncthreads();
-  for (int o = tid; o < TB * 64; o += 256) {
-    const int s = o / 64, j = o % 64;
-    float z = B2[j];
-    for (int i = 0; i < 64; i++) z += sA1[s][i] * W2[i * 64 + j];
-    sZ2[s][j] = z;
-    sA2[s][j] = sg_silu(z);
-  }
-  __syncthreads();
-  float lsum = 0.0f;
-  if (tid < TB * 3) {
-    const int s = tid / 3, o = tid % 3;
-    const int gs = s0 + s;
-    float yv = B3[o];
-    for (int j = 0; j < 64; j++) yv += sA2[s][j] * W3[j * 3 + o];
-    float dv = 0.0f;
-    if (gs < n_valid) {
-      const float t = T[(size_t)idx[gs] * 3 + o] / norm[56 + o];
-      const float e = yv - t;
-      lsum = e * e;
-      dv = 2.0f * e * inv_count;
+#pragma unroll
+  for (int o = 0; o < 3; o++) w3r[o] = W3[j * 3 + o];
+  const float b1 = B1[j], b2 = B2[j], b3 = B3[c < 3 ? c : 0];
+  const float4 xraw = ((const float4 *)X)[(size_t)(xr < 0 ? 0 : xr) * 7 + xq];
+  float4 mu, sc;
+  mu = make_float4(norm[4 * xq], norm[4 * xq + 1], norm[4 * xq + 2], norm[4 * xq + 3]);
+  sc = make_float4(norm[28 + 4 * xq], norm[29 + 4 * xq], norm[30 + 4 * xq], norm[31 + 4 * xq]);
+  // targets: waves 0 and 1 own the output tile's rows, lanes c < 3 its columns
+  float tv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (wv < 2 && c < 3) {
+    const float os = norm[56 + c];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int gs = s0 + wv * 16 + 4 * g + r;
+      if (gs < n_valid) tv[r] = T[(size_t)idx[gs] * 3 + c] / os;
     }
-    sD[s][o] = dv;
   }
-  sLoss[tid] = lsum;
+  if (tid < 224) {
+    const bool ok = xr >= 0;
+    float *q = &sX[xs][4 * xq];
+    q[0] = ((ok ? xraw.x : 0.0f) - mu.x) * sc.x;
+    q[1] = ((ok ? xraw.y : 0.0f) - mu.y) * sc.y;
+    q[2] = ((ok ? xraw.z : 0.0f) - mu.z) * sc.z;
+    q[3] = ((ok ? xraw.w : 0.0f) - mu.w) * sc.w;
+  } else {
+    sX[xs][28] = sX[xs][29] = sX[xs][30] = sX[xs][31] = 0.0f;
+  }
   __syncthreads();
+  const sg_float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // forward
+  float z1[2][4], z2[2][4], a2[2][4];
+#pragma unroll
+  for (int mt = 0; mt < 2; mt++) {
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int k = 0; k < 7; k++) acc = mfma_f32(sX[mt * 16 + c][4 * k + g], w1[k], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      z1[mt][r] = acc[r] + b1;
+      sA1[mt * 16 + 4 * g + r][j] = sg_silu(z1[mt][r]);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int mt = 0; mt < 2; mt++) {
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int k = 0; k < 16; k++) acc = mfma_f32(sA1[mt * 16 + c][4 * k + g], w2[k], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      z2[mt][r] = acc[r] + b2;
+      a2[mt][r] = sg_silu(z2[mt][r]);
+      sA2[mt * 16 + 4 * g + r][j] = a2[mt][r];
+    }
+  }
+  __syncthreads();
+  if (wv < 2) {  // output layer and loss: rows 16 wv .. 16 wv + 15
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int k = 0; k < 16; k++) acc = mfma_f32(sA2[wv * 16 + c][4 * k + g], w3b[k], acc);
+    float lsum = 0.0f;
+    if (c < 4) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int s = wv * 16 + 4 * g + r;
+        const float e = c < 3 && s0 + s < n_valid ? acc[r] + b3 - tv[r] : 0.0f;
+        lsum += e * e;
+        sD[s][c] = 2.0f * e * inv_count;
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) lsum += __shfl_xor(lsum, off);
+    if (lane == 0) sLoss[wv] = lsum;
+  }
+  __syncthreads();
+  // backward
   float *G = grad_part + (size_t)blockIdx.x * SG_MLP_NPARAM;
-  // dW3, db3
-  for (int q = tid; q < 64 * 3; q += 256) {
-    const int j = q / 3, o = q % 3;
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sA2[s][j] * sD[s][o];
-    G[SG_OFF_W3 + q] = g;
-  }
-  if (tid < 3) {
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sD[s][tid];
-    G[SG_OFF_B3 + tid] = g;
-  }
-  __syncthreads();
-  // dZ2 in place
-  for (int q = tid; q < TB * 64; q += 256) {
-    const int s = q / 64, j = q % 64;
-    const float da = sD[s][0] * W3[j * 3 + 0] + sD[s][1] * W3[j * 3 + 1] + sD[s][2] * W3[j * 3 + 2];
-    sZ2[s][j] = da * sg_silu_grad(sZ2[s][j]);
-  }
-  __syncthreads();
-  for (int q = tid; q < 64 * 64; q += 256) {
-    const int i = q / 64, j = q % 64;
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sA1[s][i] * sZ2[s][j];
-    G[SG_OFF_W2 + q] = g;
-  }
-  if (tid < 64) {
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sZ2[s][tid];
-    G[SG_OFF_B2 + tid] = g;
-  }
-  __syncthreads();  // dW2 above still reads A1
-  // dZ1 in place
-  for (int q = tid; q < TB * 64; q += 256) {
-    const int s = q / 64, i = q % 64;
-    float da = 0.0f;
-    for (int j = 0; j < 64; j++) da += sZ2[s][j] * W2[i * 64 + j];
-    sA1[s][i] = da * sg_silu_grad(sZ1[s][i]);  // (A1 no longer needed)
+  if (tid == 0) loss_part[blockIdx.x] = sLoss[0] + sLoss[1];
+  sg_float4 gw3 = zero;
+  float gb3 = 0.0f, gb2 = 0.0f, gb1 = 0.0f, dz[2][4];
+#pragma unroll
+  for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int s = mt * 16 + 4 * g + r;
+      const float4 e = *(const float4 *)sD[s];
+      const float eo = c == 0 ? e.x : (c == 1 ? e.y : (c == 2 ? e.z : 0.0f));
+      gw3 = mfma_f32(a2[mt][r], eo, gw3);
+      gb3 += eo;
+      dz[mt][r] = (e.x * w3r[0] + e.y * w3r[1] + e.z * w3r[2]) * sg_silu_grad(z2[mt][r]);
+      gb2 += dz[mt][r];
+      sZ[s][j] = dz[mt][r];
+    }
+#pragma unroll
+  for (int r = 0; r < 4; r++)
+    if (c < 3) G[SG_OFF_W3 + (wv * 16 + 4 * g + r) * 3 + c] = gw3[r];
+  gb3 = sum_groups(gb3);
+  if (tid < 3) G[SG_OFF_B3 + tid] = gb3;
+  gb2 = sum_groups(gb2);
+  if (g == 0) G[SG_OFF_B2 + j] = gb2;
+#pragma unroll
+  for (int it = 0; it < 4; it++) {
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc = mfma_f32(sA1[mt * 16 + 4 * g + r][it * 16 + c], dz[mt][r], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) G[SG_OFF_W2 + (it * 16 + 4 * g + r) * 64 + j] = acc[r];
   }
   __syncthreads();
-  for (int q = tid; q < 28 * 64; q += 256) {
-    const int i = q / 64, j = q % 64;
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sX[s][i] * sA1[s][j];
-    G[SG_OFF_W1 + q] = g;
+#pragma unroll
+  for (int mt = 0; mt < 2; mt++) {
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int k = 0; k < 16; k++) acc = mfma_f32(sZ[mt * 16 + c][4 * k + g], w2t[k], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      dz[mt][r] = acc[r] * sg_silu_grad(z1[mt][r]);
+      gb1 += dz[mt][r];
+    }
   }
-  if (tid < 64) {
-    float g = 0.0f;
-    for (int s = 0; s < TB; s++) g += sA1[s][tid];
-    G[SG_OFF_B1 + tid] = g;
+  gb1 = sum_groups(gb1);
+  if (g == 0) G[SG_OFF_B1 + j] = gb1;
+#pragma unroll
+  for (int it = 0; it < 2; it++) {
+    sg_float4 acc = zero;
+#pragma unroll
+    for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) acc = mfma_f32(sX[mt * 16 + 4 * g + r][it * 16 + c], dz[mt][r], acc);
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int i = it * 16 + 4 * g + r;
+      if (i < 28) G[SG_OFF_W1 + i * 64 + j] = acc[r];
+    }
   }
-  // per-workgroup loss
-  for (int off = 128; off > 0; off >>= 1) {
-    __syncthreads();
-    if (tid < off) sLoss[tid] += sLoss[tid + off];
-  }
-  if (tid == 0) loss_part[blockIdx.x] = sLoss[0];
 }
 
-__global__ __launch_bounds__(256) void k_mlp_adam(float *w, float *mo, float *ve, const float *grad_part, int nwg,
-                                                 float lr, float b1, float b2, float eps, float c1, float c2,
-                                                 float *grad_out) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= SG_MLP_NPARAM) return;
+// Sum of the workgroups' gradients, then Adam.  A workgroup takes ADAM_PAR parameters and
+// splits the partial gradients over ADAM_SEG threads each, added in segment order: one
+// thread per parameter walked all 256 partials on 25 CUs (58.3 us; now 4.4).  With `curve` an
+// extra workgroup sums the batch's loss.
+#define ADAM_PAR 32
+#define ADAM_SEG 16
+#define ADAM_BLOCKS ((SG_MLP_NPARAM + ADAM_PAR - 1) / ADAM_PAR)
+__global__ __launch_bounds__(ADAM_PAR *ADAM_SEG) void k_mlp_adam(float *w, float *mo, float *ve,
+                                                                const float *grad_part, int nwg, float lr, float b1,
+                                                                float b2, float eps, float c1, float c2,
+                                                                float *grad_out, const float *loss_part,
+                                                                double loss_scale, float *curve) {
+  if (blockIdx.x >= ADAM_BLOCKS) {
+    __shared__ double sL[ADAM_PAR * ADAM_SEG];
+    double s = 0.0;
+    for (int i = threadIdx.x; i < nwg; i += blockDim.x) s += loss_part[i];
+    sL[threadIdx.x] = s;
+    for (int off = ADAM_PAR * ADAM_SEG / 2; off > 0; off >>= 1) {
+      __syncthreads();
+      if ((int)threadIdx.x < off) sL[threadIdx.x] += sL[threadIdx.x + off];
+    }
+    if (threadIdx.x == 0) *curve = (float)(sL[0] * loss_scale);
+    return;
+  }
+  __shared__ float sG[ADAM_SEG][ADAM_PAR];
+  const int pl = threadIdx.x % ADAM_PAR, seg = threadIdx.x / ADAM_PAR;
+  const int p = min((int)(blockIdx.x * ADAM_PAR) + pl, SG_MLP_NPARAM - 1);
+  const int per = (nwg + ADAM_SEG - 1) / ADAM_SEG, i0 = seg * per, i1 = min(nwg, i0 + per);
   float g = 0.0f;
-  for (int i = 0; i < nwg; i++) g += grad_part[(size_t)i * SG_MLP_NPARAM + p];
+  for (int i = i0; i < i1; i += 16) {
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++) v[u] = grad_part[(size_t)min(i + u, i1 - 1) * SG_MLP_NPARAM + p];
+#pragma unroll
+    for (int u = 0; u < 16; u++) g += i + u < i1 ? v[u] : 0.0f;
+  }
+  sG[seg][pl] = g;
+  __syncthreads();
+  if (seg > 0 || (int)(blockIdx.x * ADAM_PAR) + pl >= SG_MLP_NPARAM) return;
+  g = 0.0f;
+#pragma unroll
+  for (int q = 0; q < ADAM_SEG; q++) g += sG[q][pl];
   if (grad_out) {
     grad_out[p] = g;
     return;  // gradient only (checks)
@@ -758,6 +869,30 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float *w, float *mo, float *ve
   mo[p] = m;
   ve[p] = v;
   w[p] -= lr * (m * c1) / (sqrtf(v * c2) + eps);
+}
+
+// The inference copy of the weights: BF16, output-major and padded (MlpLds), and the
+// biases.
+#define MLP_WB (64 * 32 + 64 * 64 + 16 * 64)
+__global__ __launch_bounds__(256) void k_mlp_export(const float *w, uint16_t *wb, float *bias) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < MLP_WB) {
+    float v = 0.0f;
+    if (i < 64 * 32) {
+      const int n = i / 32, k = i % 32;
+      if (k < 28) v = w[SG_OFF_W1 + k * 64 + n];
+    } else if (i < 64 * 32 + 64 * 64) {
+      const int n = (i - 64 * 32) / 64, k = (i - 64 * 32) % 64;
+      v = w[SG_OFF_W2 + k * 64 + n];
+    } else {
+      const int n = (i - 64 * 32 - 64 * 64) / 64, k = (i - 64 * 32 - 64 * 64) % 64;
+      if (n < 3) v = w[SG_OFF_W3 + k * 3 + n];
+    }
+    wb[i] = sg_f2bf(v);
+  } else if (i < MLP_WB + 144) {
+    const int q = i - MLP_WB;
+    bias[q] = q < 64 ? w[SG_OFF_B1 + q] : (q < 128 ? w[SG_OFF_B2 + q - 64] : (q < 131 ? w[SG_OFF_B3 + q - 128] : 0.0f));
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -771,24 +906,15 @@ SgMlpView sg_mlp_view(SgMlp *m) {
   return v;
 }
 
+static void enqueue_export(SgMlp *m) {
+  hipLaunchKernelGGL(k_mlp_export, dim3((MLP_WB + 144 + 255) / 256), dim3(256), 0, m->stream, m->w, m->wb, m->bias);
+}
+
+// After a host change of the weights or the normalisation.
 static int mlp_export(SgMlp *m) {
-  std::vector<float> w(SG_MLP_NPARAM);
-  if (sg_check_hip(hipMemcpy(w.data(), m->w, SG_MLP_NPARAM * 4, hipMemcpyDeviceToHost), "copy")) return -1;
-  std::vector<uint16_t> wb(64 * 32 + 64 * 64 + 16 * 64, 0);
-  for (int n = 0; n < 64; n++)
-    for (int k = 0; k < 28; k++) wb[n * 32 + k] = sg_f2bf(w[SG_OFF_W1 + k * 64 + n]);
-  for (int n = 0; n < 64; n++)
-    for (int k = 0; k < 64; k++) wb[64 * 32 + n * 64 + k] = sg_f2bf(w[SG_OFF_W2 + k * 64 + n]);
-  for (int n = 0; n < 3; n++)
-    for (int k = 0; k < 64; k++) wb[64 * 32 + 64 * 64 + n * 64 + k] = sg_f2bf(w[SG_OFF_W3 + k * 3 + n]);
-  std::vector<float> bias(144, 0.0f);
-  for (int j = 0; j < 64; j++) {
-    bias[j] = w[SG_OFF_B1 + j];
-    bias[64 + j] = w[SG_OFF_B2 + j];
-  }
-  for (int o = 0; o < 3; o++) bias[128 + o] = w[SG_OFF_B3 + o];
-  if (sg_check_hip(hipMemcpy(m->wb, wb.data(), wb.size() * 2, hipMemcpyHostToDevice), "copy")) return -1;
-  if (sg_check_hip(hipMemcpy(m->bias, bias.data(), bias.size() * 4, hipMemcpyHostToDevice), "copy")) return -1;
+  enqueue_export(m);
+  if (sg_check_hip(hipGetLastError(), "export launch")) return -1;
+  if (sg_check_hip(hipStreamSynchronize(m->stream), "export")) return -1;  // readers run on other streams
   return sg_check_hip(hipMemcpy(m->norm, m->host_norm, sizeof(m->host_norm), hipMemcpyHostToDevice), "copy");
 }
 
@@ -835,7 +961,7 @@ SgMlp *sg_mlp_new(uint64_t seed) {
 void sg_mlp_free(SgMlp *m) {
   if (!m) return;
   if (m->stream) hipStreamSynchronize(m->stream);
-  void *ptrs[] = {m->w, m->mo, m->ve, m->wb, m->bias, m->norm, m->grad_part, m->loss_part, m->dX, m->dT, m->perm};
+  void *ptrs[] = {m->w, m->mo, m->ve, m->wb, m->bias, m->norm, m->grad_part, m->loss_part, m->dX, m->dT, m->perm, m->curve};
   for (void *q : ptrs)
     if (q) hipFree(q);
   if (m->stream) hipStreamDestroy(m->stream);
@@ -916,8 +1042,9 @@ int sg_mlp_gradient(SgMlp *m, int n, float *grad_out, float *loss_out) {
   if (sg_check_hip(hipMalloc(&dg, SG_MLP_NPARAM * 4), "hipMalloc")) return -1;
   hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(256), 0, m->stream, m->w, m->dX, m->dT, m->perm, n, 0,
                      1.0f / (float)(n * 3), m->norm, m->grad_part, m->loss_part);
-  hipLaunchKernelGGL(k_mlp_adam, dim3((SG_MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->w, m->mo, m->ve,
-                     m->grad_part, nwg, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, dg);
+  hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_BLOCKS), dim3(ADAM_PAR * ADAM_SEG), 0, m->stream, m->w, m->mo, m->ve,
+                     m->grad_part, nwg, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, dg, (const float *)nullptr, 0.0,
+                     (float *)nullptr);
   hipMemcpyAsync(grad_out, dg, SG_MLP_NPARAM * 4, hipMemcpyDeviceToHost, m->stream);
   std::vector<float> lp(nwg);
   hipMemcpyAsync(lp.data(), m->loss_part, (size_t)nwg * 4, hipMemcpyDeviceToHost, m->stream);
@@ -936,38 +1063,52 @@ int sg_mlp_gradient(SgMlp *m, int n, float *grad_out, float *loss_out) {
 int sg_mlp_train(SgMlp *m, int epochs, int batch_wg, float lr, uint64_t seed, float *loss_curve) {
   if (!m || !m->dX || epochs <= 0 || batch_wg <= 0) return sg_set_error("bad arguments");
   if (ensure_parts(m, batch_wg)) return -1;
+  if (loss_curve && epochs > m->curve_cap) {
+    if (m->curve) hipFree(m->curve);
+    m->curve = nullptr;
+    m->curve_cap = 0;
+    if (sg_check_hip(hipMalloc(&m->curve, (size_t)epochs * 4), "hipMalloc")) return -1;
+    m->curve_cap = epochs;
+  }
   std::mt19937_64 rng(seed);
   std::vector<int> id(m->n);
-  std::vector<float> lp(batch_wg);
   const int batch = batch_wg * TB;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+  // The host shuffles an epoch while the one before runs: it waits only for the copy of
+  // that epoch's order out of `id` (each epoch's first loss is summed on the GPU).
+  hipEvent_t copied = nullptr;
+  if (sg_check_hip(hipEventCreateWithFlags(&copied, hipEventDisableTiming), "event")) return -1;
   for (int e = 0; e < epochs; e++) {
+    if (e > 0) hipEventSynchronize(copied);
     for (int i = 0; i < m->n; i++) id[i] = i;
     std::shuffle(id.begin(), id.end(), rng);
     hipMemcpyAsync(m->perm, id.data(), (size_t)m->n * 4, hipMemcpyHostToDevice, m->stream);
-    double lsum = 0.0;
+    hipEventRecord(copied, m->stream);
     // cosine-free schedule: constant, then /10 for the last quarter of the epochs
     const float lr_e = (e >= (3 * epochs) / 4) ? lr * 0.1f : lr;
     for (int base = 0; base + batch <= m->n; base += batch) {
       m->step++;
       const float c1 = 1.0f / (1.0f - powf(b1, (float)m->step));
       const float c2 = 1.0f / (1.0f - powf(b2, (float)m->step));
+      const bool curve = loss_curve && base == 0;
       hipLaunchKernelGGL(k_mlp_train, dim3(batch_wg), dim3(256), 0, m->stream, m->w, m->dX, m->dT, m->perm,
                          m->n, base, 1.0f / (float)(batch * 3), m->norm, m->grad_part, m->loss_part);
-      hipLaunchKernelGGL(k_mlp_adam, dim3((SG_MLP_NPARAM + 255) / 256), dim3(256), 0, m->stream, m->w, m->mo,
-                         m->ve, m->grad_part, batch_wg, lr_e, b1, b2, eps, c1, c2, (float *)nullptr);
-      if (loss_curve && base == 0) {
-        hipMemcpyAsync(lp.data(), m->loss_part, (size_t)batch_wg * 4, hipMemcpyDeviceToHost, m->stream);
-        hipStreamSynchronize(m->stream);
-        double s = 0.0;
-        for (float x : lp) s += x;
-        lsum = s / (double)(batch * 3);
-      }
+      hipLaunchKernelGGL(k_mlp_adam, dim3(ADAM_BLOCKS + (curve ? 1 : 0)), dim3(ADAM_PAR * ADAM_SEG), 0, m->stream,
+                         m->w, m->mo, m->ve, m->grad_part, batch_wg, lr_e, b1, b2, eps, c1, c2, (float *)nullptr,
+                         m->loss_part, 1.0 / (double)(batch * 3), curve ? m->curve + e : (float *)nullptr);
     }
-    if (loss_curve) loss_curve[e] = (float)lsum;
   }
-  if (sg_check_hip(hipStreamSynchronize(m->stream), "train")) return -1;
-  return mlp_export(m);
+  enqueue_export(m);
+  if (loss_curve) {
+    if (batch <= m->n)
+      hipMemcpyAsync(loss_curve, m->curve, (size_t)epochs * 4, hipMemcpyDeviceToHost, m->stream);
+    else  // less than one batch: no step was taken
+      std::fill(loss_curve, loss_curve + epochs, 0.0f);
+  }
+  int rc = sg_check_hip(hipGetLastError(), "train launch");
+  const int rs = sg_check_hip(hipStreamSynchronize(m->stream), "train");
+  hipEventDestroy(copied);
+  return rc ? rc : rs;
 }
 
 // Inference through the MFMA path on raw features X[n][28] -> displacement Y[n][3]

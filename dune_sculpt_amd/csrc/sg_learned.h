@@ -31,6 +31,8 @@ struct SgMlp {
   int part_cap = 0;
   float *dX = nullptr, *dT = nullptr;
   int *perm = nullptr;
+  float *curve = nullptr;  // per-epoch losses of the running training
+  int curve_cap = 0;
   int n = 0;
   int step = 0;
   float alpha = 1.0f;  // held-out RMS error / RMS displacement of the plain brush
