@@ -532,7 +532,7 @@ int sg_dab_apply(PBVH *p, const SgDabParams *dab) {
   SgDabK k = sg_make_dab(dab, g_stats ? 1 : 0);
   const int stamp = (++p->stamp) * 128;
   p->halt_live = k.learned && p->mlp;
-  int rc = sg_enqueue_clear_ctr(p);
+  int rc = sg_enqueue_clear_ctr(p, 1);
   if (!rc) rc = sg_enqueue_dab(p, k, curve, nullptr, 0, stamp, 0);
   if (!rc) rc = sg_enqueue_finish(p, 0);
   if (!rc) rc = sg_enqueue_flush(p);
@@ -655,7 +655,7 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
       int ci = 0;
       for (int i = 0; i < a0; i++)
         ci += (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table) ? 1 : 0;
-      if (sg_enqueue_clear_ctr(p)) return -1;
+      if (sg_enqueue_clear_ctr(p, n - a0)) return -1;
       for (int i = a0; i < n; i++) {
         const float *curve = nullptr;
         if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
@@ -667,7 +667,11 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
           if (int rc = enqueue_place(p, dabs, rays, p->d.place_rays, p->d.place, i, n, i - a0)) return rc;
           place = p->d.place + 8 * (size_t)i;
         }
-        if (int rc = sg_enqueue_dab(p, k, curve, log ? p->d.log : nullptr, i - a0, stamp, i - a0, nullptr, place))
+        SgDabK kn;
+        const bool next = !rays && i + 1 < n;
+        if (next) kn = sg_make_dab(&dabs[i + 1], g_stats ? 1 : 0);
+        if (int rc = sg_enqueue_dab(p, k, curve, log ? p->d.log : nullptr, i - a0, stamp, i - a0, nullptr, place,
+                                    next ? &kn : nullptr))
           return rc;
         if (flush_each && sg_enqueue_flush(p)) return -1;
       }
@@ -894,7 +898,7 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
     rc = erc ? erc : sg_check_hip(e, "end capture");
   } else if (!rc) {
     int ci = 0;
-    erc = sg_enqueue_clear_ctr(p);
+    erc = sg_enqueue_clear_ctr(p, n);
     for (int i = 0; i < n && !erc; i++) {
       const float *curve = nullptr;
       if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
@@ -905,7 +909,11 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
         erc = enqueue_place(p, dabs, rays, s->place_rays, s->place, i, n, i);
         place = s->place + 8 * (size_t)i;
       }
-      if (!erc) erc = sg_enqueue_dab(p, k, curve, log ? p->d.log : nullptr, i, 0, i, nullptr, place);
+      SgDabK kn;
+      const bool next = !rays && i + 1 < n;
+      if (next) kn = sg_make_dab(&dabs[i + 1], 0);
+      if (!erc)
+        erc = sg_enqueue_dab(p, k, curve, log ? p->d.log : nullptr, i, 0, i, nullptr, place, next ? &kn : nullptr);
       if (!erc && flush_each) erc = sg_enqueue_flush(p);
     }
     if (!erc) erc = sg_enqueue_finish(p, n - 1);
@@ -1138,7 +1146,7 @@ int sg_learned_collect(PBVH *p, const SgDabParams *dab, float *X, float *T, floa
   plain.flag &= ~SG_SMOOTH_LEARNED;
   SgDabK k = sg_make_dab(&plain, 0);
   p->halt_live = false;
-  int rc = sg_enqueue_clear_ctr(p);
+  int rc = sg_enqueue_clear_ctr(p, 1);
   if (!rc) rc = sg_enqueue_dab(p, k, nullptr, nullptr, 0, 0, 0, &col);
   if (!rc) rc = sg_enqueue_flush(p);
   long long ctr[SG_CTR_COUNT];

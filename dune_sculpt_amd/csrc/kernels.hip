@@ -54,10 +54,6 @@ int sg_check_hip(hipError_t e, const char *what) {
 // it into the reference's left->right order when asked).  A wave after the subtree
 // waves logs the previous dab's counters and clears the next dab's counter set.
 // ---------------------------------------------------------------------------
-// The last `copy_blocks` workgroups of the search bring in the results of the previous
-// dab when it was a fused dab (fused kernel below): it wrote its affected vertices'
-// positions into the shadow copy and their normals into (mx, my, mz), because its own
-// workgroups read those arrays' old values; the copy restores positions == shadow copy.
 #define COUNT_UNROLL 8
 // A wave's sum of the per-leaf affected counts aff_cnt[0, ng): the first 64 *
 // COUNT_UNROLL counts load unconditionally (clamped indices), so they are issued before
@@ -79,93 +75,47 @@ __device__ __forceinline__ int aff_count_sum(const SgDevView &d, const CountPref
   return wave_sum_i(s);
 }
 
-#define COPY_UNROLL 4
-// Caller knows a fused dab's results are pending (its record: pend[0] = its gathered
-// count).
-__device__ __forceinline__ void fused_copy_back(const SgDevView &d, int tid, int nthreads) {
-  // The first COPY_UNROLL slots of each thread load beside the pending record, and all
-  // their positions and normals load before any store: unconditional loads from clamped
-  // indices (slots below L << aff_shift are allocated; vertex 0 stands in for an unused
-  // slot), so the copies wait on two levels.
-  const int nslot = d.L << d.aff_shift, msk = (1 << d.aff_shift) - 1;
-  int cnt[COPY_UNROLL], vs[COPY_UNROLL];
-#pragma unroll
-  for (int u = 0; u < COPY_UNROLL; u++) {
-    const int i = min(tid + u * nthreads, nslot - 1);
-    cnt[u] = d.aff_cnt[i >> d.aff_shift];
-    vs[u] = d.aff_v[i];
-  }
-  const int na = d.pend[0] << d.aff_shift;
-  bool ok[COPY_UNROLL];
-  float x[COPY_UNROLL], y[COPY_UNROLL], z[COPY_UNROLL], a[COPY_UNROLL], b[COPY_UNROLL], c[COPY_UNROLL];
-#pragma unroll
-  for (int u = 0; u < COPY_UNROLL; u++) {
-    const int i = tid + u * nthreads;
-    ok[u] = i < na && (i & msk) < cnt[u];
-    const int v = ok[u] ? vs[u] : 0;
-    x[u] = d.qx[v];
-    y[u] = d.qy[v];
-    z[u] = d.qz[v];
-    a[u] = d.mx[v];
-    b[u] = d.my[v];
-    c[u] = d.mz[v];
-  }
-#pragma unroll
-  for (int u = 0; u < COPY_UNROLL; u++) {
-    if (!ok[u]) continue;
-    const int v = vs[u];
-    d.px[v] = x[u];
-    d.py[v] = y[u];
-    d.pz[v] = z[u];
-    d.nx[v] = a[u];
-    d.ny[v] = b[u];
-    d.nz[v] = c[u];
-  }
-  for (int i = tid + COPY_UNROLL * nthreads; i < na; i += nthreads) {
-    const int v = aff_slot_vertex(d, i, d.aff_cnt[i >> d.aff_shift]);
-    if (v < 0) continue;
-    const float px = d.qx[v], py = d.qy[v], pz = d.qz[v];
-    const float nx = d.mx[v], ny = d.my[v], nz = d.mz[v];
-    d.px[v] = px;
-    d.py[v] = py;
-    d.pz[v] = pz;
-    d.nx[v] = nx;
-    d.ny[v] = ny;
-    d.nz[v] = nz;
+// Appends passing leaves to dab `serial`'s chain list (whole wave; a lane per leaf, leaf
+// l = lane modulo SG_CH_SEG).  The list is SG_CH_SEG segments by leaf number, each with
+// its own counter line and room for its share of all leaves: one counter took a returning
+// atomic per gathered leaf, 12 ns each (a dab over 1250 leaves waited 15 us on it).
+__device__ __forceinline__ void chain_append(const SgDevView &d, int serial, int l, bool pass, unsigned long long m,
+                                             const int4 &r0, const int4 &r1, int stamp) {
+  const int lane = lane_id(), seg = lane % SG_CH_SEG;
+  // this lane's segment: every SG_CH_SEG-th lane
+  const unsigned long long ms = m & (0x0001000100010001ull << seg);
+  int base = 0;
+  if (lane < SG_CH_SEG && ms)
+    base = (int)atomicAdd((unsigned long long *)&d.ch_ctr[((size_t)(serial % 3) * SG_CH_SEG + seg) * SG_CH_CTR],
+                          (unsigned long long)__popcll(ms));
+  base = __shfl(base, seg);
+  if (pass) {
+    const size_t q = (size_t)(serial % 3) * d.ch_cap * SG_CH_SEG + (size_t)seg * d.ch_cap + (size_t)(base + mask_prefix(ms));
+    d.ch_leaf[q] = l;
+    d.ch_rec[2 * q] = r0;
+    d.ch_rec[2 * q + 1] = r1;
+    d.ch_gstamp[(size_t)(serial & 1) * d.L + l] = stamp;
   }
 }
 
-// Block roles, in grid order:
-//   [0, leaf_blocks)          a thread per leaf: box test, then for passing leaves the
-//                             records load beside one slot reservation per wave
-//   next cut_blocks           a wave per subtree: refresh the box of a subtree the
-//                             previous dab changed (for ray casts and the statistics);
-//                             the wave after the last subtree does the bookkeeping
-//   last copy_blocks          copy-back of a fused previous dab (copy_pending: known
-//                             when the launch is recorded)
+// Block roles, in grid order (the dispatcher starts blocks in index order, and the
+// refreshes are the longest):
+//   [0, cut_blocks)   a wave per subtree c < nrefresh: refresh the box of a subtree the
+//                     previous dab changed (for the ray casts of a placed stroke and for
+//                     the statistics; nrefresh = 0 otherwise, the deferred refit rebuilds
+//                     the boxes after the stroke); wave nrefresh does the bookkeeping
+//   the rest          a thread per leaf: box test, then for passing leaves the records
+//                     load beside one slot reservation per wave
 // No test waits on a subtree box: a leaf's own box decides, so a passing leaf's chain
 // is its box, then the reservation.
 __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long *log, int log_index,
-                                                int serial, const float *place, int leaf_blocks, int cut_blocks,
-                                                int copy_blocks, int copy_pending) {
+                                                int serial, const float *place, int cut_blocks, int nrefresh) {
   if (d.halt && d.halt[0]) return;
   const int lane = lane_id();
-  // Block roles in launch order: subtree waves, copy blocks, then leaves.  The
-  // dispatcher starts blocks in index order, and the subtree refreshes and the copy are
-  // the longest blocks, so they start first.  vb: the block's number in the order
-  // leaves, subtrees, copy.
-  const int bx = (int)blockIdx.x;
-  const int vb = bx < cut_blocks ? leaf_blocks + bx
-                                 : (bx < cut_blocks + copy_blocks ? leaf_blocks + bx : bx - cut_blocks - copy_blocks);
-  if (vb >= leaf_blocks + cut_blocks) {
-    const int cb = vb - (leaf_blocks + cut_blocks);
-    if (copy_pending) fused_copy_back(d, cb * blockDim.x + threadIdx.x, copy_blocks * blockDim.x);
-    return;
-  }
   sg_place(k, place);
   const float *leaf_bbs = k.use_orig ? d.leaf_obb : d.leaf_bb;
-  if (vb < leaf_blocks) {
-    const int l = vb * blockDim.x + threadIdx.x;
+  if ((int)blockIdx.x >= cut_blocks) {
+    const int l = ((int)blockIdx.x - cut_blocks) * blockDim.x + threadIdx.x;
     const int lc = min(l, d.L - 1);
     const BB6 b = bb_load(leaf_bbs + 8 * (size_t)lc);
     const int fl = k.hide_skip ? d.leaf_flags[lc] : 0;
@@ -184,7 +134,7 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
                      0, 0);
     }
     const int cut = d.leaf_cut[lc];
-    const int stamp = d.dstamp ? d.dstamp[serial & 1] : 0;
+    const int stamp = d.dstamp ? d.dstamp[0] + serial : 0;
     int wbase = 0;
     if (lane == 0) wbase = (int)atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], (unsigned long long)__popcll(m));
     wbase = __shfl(wbase, 0);
@@ -193,42 +143,29 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
       d.gathered[pos] = l;
       d.gl_v[pos] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
       d.gl_s[pos] = make_int2(r0.y, r0.y + (r1.x >> 16));
-      if (k.fused) {
-        d.gl_rec[2 * pos] = r0;
-        d.gl_rec[2 * pos + 1] = r1;
-        d.leaf_gstamp[l] = stamp;
-      }
       // the subtree's flags (every passing leaf of it writes the same values)
       d.cut_touch[cut] = serial;
       d.cut_dirty[cut] = 1;
       d.draw_dirty[cut] = 1;  // the subtree's leaves need new draw records (UpdateDrawBuffers)
     }
+    if (k.fused) chain_append(d, serial, l, pass, m, r0, r1, stamp);  // the first dab of a chain
     return;
   }
   // subtree waves
-  const int c = (vb - leaf_blocks) * (blockDim.x / SG_WAVE) + threadIdx.x / SG_WAVE;
-  if (c == d.C) {  // bookkeeping
-    const int stamp = d.dstamp ? d.dstamp[serial & 1] : 0;
-    if (log && log_index > 0) {
-      // a fused previous dab left its affected count as per-leaf counts: sum them
-      long long naff = -1;
-      if (copy_pending) {
-        const CountPrefetch cp = aff_count_prefetch(d, lane);
-        naff = aff_count_sum(d, cp, lane, d.pend[0]);
-      }
-      if (lane < SG_CTR_COUNT) {
-        long long prev = d.ctr_next[lane];  // the set the previous dab used
-        if (lane == SG_CTR_NAFF && naff >= 0) prev = naff;
+  const int c = (int)blockIdx.x * (blockDim.x / SG_WAVE) + threadIdx.x / SG_WAVE;
+  if (c == nrefresh) {  // bookkeeping
+    if (lane < SG_CTR_COUNT) {
+      if (log && log_index > 0) {
+        const long long prev = d.ctr_next[lane];  // the set the previous dab used
         log[(size_t)(log_index - 1) * SG_CTR_COUNT + lane] = lane == SG_CTR_NGATHER ? (prev & 0xffffffffll) : prev;
       }
+      d.ctr_next[lane] = 0;
     }
-    if (lane < SG_CTR_COUNT) d.ctr_next[lane] = 0;
-    if (lane == 0 && d.seq) d.seq[0] += 1;                                 // this dab's stamp for the later kernels
-    if (lane == 0 && d.dstamp) d.dstamp[(serial & 1) ^ 1] = stamp + 1;   // the next dab's
+    if (lane == 0 && d.seq) d.seq[0] += 1;  // this dab's stamp for the later kernels
     if (lane == 0 && undo_active(d)) atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], SG_NGATHER_UNDO);
     return;
   }
-  if (c > d.C) return;
+  if (c > nrefresh) return;
   // The previous dab changed this subtree (its leaves' boxes moved), so its box is
   // rebuilt here from its leaf boxes, both the current and the original one.  With the
   // statistics on, the wave also counts the tests a pruned search makes: the subtree
@@ -273,12 +210,20 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
   if (k.stats && lane == 0) atomicAdd((unsigned long long *)&d.ctr[SG_CTR_TESTS], (unsigned long long)ntests);
 }
 
-// zero both counter sets and the halt flag at the start of a stroke; the dab stamps
-// only grow (the first dab's stamp is above every earlier one)
-__global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp) {
+// At the start of a stroke of n dabs: zero the counter sets and the halt flag, and take
+// the stamps dstamp[0] + serial for its dabs, above every earlier one and leaving the
+// stamp before the first one unused (no staged value belongs to "the dab before" it).
+__global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp, long long *ch_ctr, int n) {
   if (threadIdx.x < 2 * SG_CTR_COUNT) ctr[threadIdx.x] = 0;
   if (threadIdx.x == 0) halt[0] = 0;
-  if (threadIdx.x == 0 && dstamp) dstamp[0] = max(dstamp[0], dstamp[1]) + 1;
+  if (dstamp) {
+    for (int i = threadIdx.x; i < 3 * SG_CH_SEG * SG_CH_CTR; i += blockDim.x) ch_ctr[i] = 0;
+    if (threadIdx.x == 0) {
+      const int b = dstamp[1] + 2;
+      dstamp[0] = b;
+      dstamp[1] = b + n;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -287,7 +232,9 @@ __global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp) {
 // and accumulated in int64 -- exact, so the atomic order cannot change the bits.
 // Positions and normals are fetched in the same load level.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_area(SgDevView d, SgDabK k, const float *place) {
+// ch: the counter lines of a chain's first dab (one per workgroup modulo SG_CH_AREA), or
+// null: the dab's counter set.
+__global__ __launch_bounds__(256) void k_area(SgDevView d, SgDabK k, const float *place, long long *ch) {
   if (d.halt && d.halt[0]) return;
   sg_place(k, place);
   const int lane = lane_id();
@@ -335,10 +282,11 @@ __global__ __launch_bounds__(256) void k_area(SgDevView d, SgDabK k, const float
     for (int i = 0; i < (int)(blockDim.x / SG_WAVE); i++)
       for (int q = 0; q < 4; q++) t[q] += s_part[i][q];
     if (t[3]) {
-      atomicAdd((unsigned long long *)&d.ctr[SG_CTR_AREA_X], as_u64(t[0]));
-      atomicAdd((unsigned long long *)&d.ctr[SG_CTR_AREA_Y], as_u64(t[1]));
-      atomicAdd((unsigned long long *)&d.ctr[SG_CTR_AREA_Z], as_u64(t[2]));
-      atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NAREA], (unsigned long long)t[3]);
+      long long *c = ch ? ch + (blockIdx.x % SG_CH_AREA) * SG_CH_CTR : d.ctr;
+      atomicAdd((unsigned long long *)&c[SG_CTR_AREA_X], as_u64(t[0]));
+      atomicAdd((unsigned long long *)&c[SG_CTR_AREA_Y], as_u64(t[1]));
+      atomicAdd((unsigned long long *)&c[SG_CTR_AREA_Z], as_u64(t[2]));
+      atomicAdd((unsigned long long *)&c[ch ? SG_CH_NAREA : SG_CTR_NAREA], (unsigned long long)t[3]);
     }
   }
 }
@@ -836,23 +784,42 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 }
 
 // ---------------------------------------------------------------------------
-// Fused dab: one workgroup per gathered leaf runs the brush, Smooth's Jacobi steps, the
-// normals of the leaf's affected vertices and the leaf's box in one pass, on the leaf's
-// halo staged in LDS (its uniq vertices, ring 0 = its shared vertices and their edge
-// neighbours' ring, and for Smooth(k) k more rings; tables from the build).  Every
+// Fused dabs, chained: one launch per dab.  Launch i does, side by side,
+//   F  a workgroup per leaf gathered by dab i: brush, Smooth's Jacobi steps, normals and
+//      leaf box on the leaf's halo staged in LDS; then the leaf's new box against dab
+//      i + 1's sphere, and its share of dab i + 1's area normal
+//   S  a thread per leaf not gathered by dab i: its box against dab i + 1's sphere (no
+//      vertex of it moves in this launch), and its share of the area normal
+//   C  copies dab i - 1's results into the mesh arrays
+// so a dab waits for one kernel boundary instead of two (three for Draw) and for no
+// search.  Bound by the chain of dependent loads, not by bytes.  As search, area normal
+// and brush kernels 240 mixed dabs on a 2.6 M-vertex mesh took 3.47 ms with the draw
+// refill after them, now 2.54; 200 Draw dabs on 41 k vertices 2.67 and 1.78; 24 dabs over
+// about 1250 leaves each 0.94 and 0.78.  The first dab of a chain has its own search (and
+// k_area).
+//
+// F works on the leaf's halo (its uniq vertices, ring 0 = its shared vertices and their
+// edge neighbours' ring, and for Smooth(k) k more rings; tables from the build).  Every
 // halo vertex's displacement is computed here from the same inputs and in the same
 // FP32 order as the vertex's own workgroup computes it (a vertex of ring j is exact
 // after k - j Jacobi steps), so the results equal the separate kernels' bit for bit.
-// Workgroups read other leaves' vertices as they were before the dab, so the results
-// go to the shadow copy (positions) and to (mx, my, mz) (normals); the next dab's
-// search, or k_dab_finish, copies them in.  A halo vertex counts as affected only when
-// its own leaf was gathered (the search stamps gathered leaves), as the search and the
-// per-leaf vertex test decide it for that leaf.
+// A halo vertex counts as affected only when its own leaf was gathered (gather stamps),
+// as the search and the per-leaf vertex test decide it for that leaf.
+//
+// Workgroups read other leaves' vertices as they were before the dab, so dab i's results
+// go to its staging arrays (by its parity): position and the dab's stamp in one float4,
+// normal in another.  Whoever reads a vertex in launch i takes the staged value when it
+// carries dab i - 1's stamp and the mesh array otherwise: C may be writing exactly those
+// vertices' mesh values.  What launch i reads and writes at the same time therefore
+// differs in its slot: staging, gather stamps and copied counts by the dab's parity,
+// leaf lists and counters by the dab modulo 3 (dab i + 1's list fills while C reads dab
+// i - 1's).
 // ---------------------------------------------------------------------------
 #define FUSED_THREADS 256
+#define FUSED_LEAD 256  // F blocks started before the S and C blocks: more leaves than most dabs gather
 #define FUSED_ROW 8  // neighbour / incidence entries per local held in registers
 
-// One workgroup per gathered leaf; each thread holds LPT locals (local i = tid + j * 256).
+// F: one workgroup per gathered leaf; each thread holds LPT locals (local i = tid + j * 256).
 // Global loads come in three dependent levels, each issued for every local at once:
 //   1  the counters and the workgroup's first gathered leaf (ranges, halo header)
 //   2  halo vertex ids, neighbour-row and incidence ranges, shared-vertex local ids
@@ -863,12 +830,176 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 #define FUSED_FPT 2              // faces per face thread whose corners load up front
 #define FUSED_FACE_THREADS 192   // the first three waves compute the face normals, the last the leaf box
 
+struct SgChainArgs {
+  int serial;
+  int f0;                    // F blocks ahead of the S and C blocks in launch order
+  int nf, ns, nc;            // F, S, C blocks
+  int cap, fcap;             // LDS: locals, faces
+  int has_next, has_prev;
+  int last;                  // the chain ends here: keep the affected list and the gathered leaves for the host
+  long long *log;            // per-dab counter rows, or null
+};
+
+// Affected vertices of dab `serial` from staging into the mesh arrays: a wave per leaf it
+// gathered (its uniq range, staged entries of that dab only).
+__device__ __forceinline__ void chain_copy_back(const SgDevView &d, int serial, int gw, int nw) {
+  const float4 *sp = d.st_pos + (size_t)(serial & 1) * d.V, *sn = d.st_nor + (size_t)(serial & 1) * d.V;
+  // wave gw takes its share of segment gw % SG_CH_SEG
+  const int seg = gw % SG_CH_SEG, i0 = gw / SG_CH_SEG;
+  const int4 *rec = d.ch_rec + 2 * ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  const int gc = min(i0, d.ch_cap - 1);
+  const int4 ra0 = rec[2 * gc], rb0 = rec[2 * gc + 1];
+  const int ng = d.pend[(serial & 1) * SG_CH_SEG + seg], stamp = d.dstamp[0] + serial;
+  for (int g = i0; g < ng; g += nw / SG_CH_SEG) {
+    const int4 ra = g == i0 ? ra0 : rec[2 * g], rb = g == i0 ? rb0 : rec[2 * g + 1];
+    const int nu = rb.x & 0xffff;
+    for (int i = lane_id(); i < nu; i += 2 * SG_WAVE) {
+      // two vertices per lane, all loads ahead of the stores
+      const int v0 = ra.x + i, v1 = i + SG_WAVE < nu ? v0 + SG_WAVE : v0;
+      const float4 a0 = sp[v0], a1 = sp[v1], b0 = sn[v0], b1 = sn[v1];
+      if (__float_as_int(a0.w) == stamp) {
+        d.px[v0] = d.qx[v0] = a0.x;
+        d.py[v0] = d.qy[v0] = a0.y;
+        d.pz[v0] = d.qz[v0] = a0.z;
+        d.nx[v0] = b0.x;
+        d.ny[v0] = b0.y;
+        d.nz[v0] = b0.z;
+      }
+      if (v1 != v0 && __float_as_int(a1.w) == stamp) {
+        d.px[v1] = d.qx[v1] = a1.x;
+        d.py[v1] = d.qy[v1] = a1.y;
+        d.pz[v1] = d.qz[v1] = a1.z;
+        d.nx[v1] = b1.x;
+        d.ny[v1] = b1.y;
+        d.nz[v1] = b1.z;
+      }
+    }
+  }
+}
+
+// Exact fixed-point sums of the area normal (see k_area); a wave's share.
+struct AreaSum {
+  long long x, y, z;
+  int n;
+};
+__device__ __forceinline__ void area_add(AreaSum &s, const SgDabK &k, float px, float py, float pz, float nx, float ny,
+                                         float nz, bool ok) {
+  const float dx = k.cx - px, dy = k.cy - py, dz = k.cz - pz;
+  if (ok && dx * dx + dy * dy + dz * dz <= k.nr2) {
+    s.x += __double2ll_rn((double)nx * 4294967296.0);
+    s.y += __double2ll_rn((double)ny * 4294967296.0);
+    s.z += __double2ll_rn((double)nz * 4294967296.0);
+    s.n++;
+  }
+}
+// whole wave active; ctr: a counter line of the dab (the first SG_CH_AREA lines hold area
+// sums: one line per leaf segment cost each Draw workgroup 1 us to add up)
+__device__ __forceinline__ void area_flush(const AreaSum &s, long long *ctr) {
+  if (!__any(s.n > 0)) return;
+  const long long x = wave_total_ll(s.x), y = wave_total_ll(s.y), z = wave_total_ll(s.z), n = wave_total_ll(s.n);
+  if (lane_id() == SG_WAVE - 1) {
+    atomicAdd((unsigned long long *)&ctr[SG_CTR_AREA_X], as_u64(x));
+    atomicAdd((unsigned long long *)&ctr[SG_CTR_AREA_Y], as_u64(y));
+    atomicAdd((unsigned long long *)&ctr[SG_CTR_AREA_Z], as_u64(z));
+    atomicAdd((unsigned long long *)&ctr[SG_CH_NAREA], as_u64(n));
+  }
+}
+
+// S: dab serial + 1's search over the leaves that dab `serial` does not touch, block b.
+__device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &kn, int serial, int b, int2 *s_q,
+                                             int *s_nq) {
+  const int lane = lane_id();
+  if (threadIdx.x == 0) *s_nq = 0;
+  const int l = b * blockDim.x + threadIdx.x, lc = min(l, d.L - 1);
+  const BB6 bb = bb_load((kn.use_orig ? d.leaf_obb : d.leaf_bb) + 8 * (size_t)lc);
+  const int gs = d.ch_gstamp[(size_t)(serial & 1) * d.L + lc];
+  const int fl = kn.hide_skip ? d.leaf_flags[lc] : 0;
+  const int stamp = d.dstamp[0] + serial;
+  const bool pass = l < d.L && gs != stamp && !(fl & kn.hide_skip) && sphere_box(bb, kn.cx, kn.cy, kn.cz, kn.r2);
+  const unsigned long long m = __ballot(pass);
+  int4 r0 = make_int4(0, 0, 0, 0), r1 = make_int4(0, 0, 0, 0);
+  if (m) {
+    r0 = d.hl_rec[2 * (size_t)lc];
+    r1 = d.hl_rec[2 * (size_t)lc + 1];
+    chain_append(d, serial + 1, l, pass, m, r0, r1, stamp + 1);
+  }
+  if (kn.tool != SG_TOOL_DRAW) return;
+  // the area normal's share of the new leaves that reach into its sphere (usually none:
+  // the dab before covered it), a wave per leaf.  A vertex with d2 <= nr2 lies in its
+  // leaf's box, whose distance, rounded the same way, is not larger.
+  float t2;
+  {
+    const float cc[3] = {kn.cx, kn.cy, kn.cz};
+    float t[3];
+    for (int i = 0; i < 3; i++) t[i] = cc[i] - (bb.mn[i] > cc[i] ? bb.mn[i] : (bb.mx[i] < cc[i] ? bb.mx[i] : cc[i]));
+    t2 = t[0] * t[0] + t[1] * t[1] + t[2] * t[2];
+  }
+  __syncthreads();
+  if (pass && t2 <= kn.nr2) s_q[atomicAdd(s_nq, 1)] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
+  __syncthreads();
+  const int nq = *s_nq;
+  const float4 *sp = d.st_pos + (size_t)((serial + 1) & 1) * d.V, *sn = d.st_nor + (size_t)((serial + 1) & 1) * d.V;
+  const bool hide = d.vhide && d.respect_hide;
+  const int *hp = hide ? d.vhide : (const int *)d.px;
+  AreaSum sum = {0, 0, 0, 0};
+  for (int q = threadIdx.x / SG_WAVE; q < nq; q += blockDim.x / SG_WAVE) {
+    const int2 vr = s_q[q];
+    for (int base = vr.x; base < vr.y; base += 2 * SG_WAVE) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int v = base + u * SG_WAVE + lane, vc = min(v, vr.y - 1);
+        const float4 a = sp[vc], nn = sn[vc];
+        const bool st = __float_as_int(a.w) == stamp - 1;  // moved by the dab before: staged
+        const float x = d.px[vc], y = d.py[vc], z = d.pz[vc], nx = d.nx[vc], ny = d.ny[vc], nz = d.nz[vc];
+        const bool ok = v < vr.y && !(hide && hp[vc] != 0);
+        area_add(sum, kn, st ? a.x : x, st ? a.y : y, st ? a.z : z, st ? nn.x : nx, st ? nn.y : ny, st ? nn.z : nz, ok);
+      }
+    }
+  }
+  area_flush(sum, d.ch_ctr + ((size_t)((serial + 1) % 3) * SG_CH_SEG + b % SG_CH_AREA) * SG_CH_CTR);
+}
+
+// Counter i (SG_CTR_*) of a chained dab: its lines summed.
+__device__ __forceinline__ long long chain_counter(const long long *lines, int i) {
+  const int f = i == SG_CTR_NAREA ? SG_CH_NAREA : i;
+  if (f > SG_CH_NAREA || i == SG_CH_NAREA) return 0;
+  long long t = 0;
+  for (int q = 0; q < SG_CH_SEG; q++) t += lines[q * SG_CH_CTR + f];
+  return t;
+}
+
 template <int LPT>
-__global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK k, const float *curve, int serial,
-                                                            int cap, int fcap) {
+__global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK k, SgDabK kn, const float *curve,
+                                                            SgChainArgs ca) {
   if (d.halt && d.halt[0]) return;
   extern __shared__ __align__(16) unsigned char fused_smem[];
-  __shared__ int s_cnt;
+  __shared__ int s_cnt, s_next;
+  __shared__ int2 s_q[FUSED_THREADS];
+  const int serial = ca.serial;
+  int g0 = (int)blockIdx.x;
+  if (g0 >= ca.f0) {
+    const int o = g0 - ca.f0;
+    if (o < ca.ns) {
+      chain_search(d, kn, serial, o, s_q, &s_cnt);
+      return;
+    }
+    if (o < ca.ns + ca.nc) {
+      chain_copy_back(d, serial - 1, ((o - ca.ns) * FUSED_THREADS + (int)threadIdx.x) / SG_WAVE,
+                      ca.nc * (FUSED_THREADS / SG_WAVE));
+      return;
+    }
+    if (o == ca.ns + ca.nc) {  // log the previous dab's counters and clear its set (dab serial + 2's)
+      long long *ctr = d.ch_ctr + (size_t)((serial + 2) % 3) * SG_CH_SEG * SG_CH_CTR;
+      if (ca.log && ca.has_prev && threadIdx.x < SG_CTR_COUNT)
+        ca.log[(size_t)(serial - 1) * SG_CTR_COUNT + threadIdx.x] = chain_counter(ctr, threadIdx.x);
+      __syncthreads();
+      if (threadIdx.x < SG_CH_SEG * SG_CH_CTR) ctr[threadIdx.x] = 0;
+      return;
+    }
+    g0 = o - ca.ns - ca.nc - 1 + ca.f0;
+  }
+  const size_t L = (size_t)d.L;
+  const int cap = ca.cap, fcap = ca.fcap;
   // positions of the locals, two buffers of `cap` (x, y, z, 0), the normals of the
   // leaf's faces (`fcap` of them), the shared vertices' local ids
   float4 *const S = (float4 *)fused_smem;
@@ -878,35 +1009,51 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
   // level 1: counters, stamp and the first gathered leaf's records together.  Loads
   // below are unconditional from clamped (always valid) indices, with the selection
   // after them: a load under a branch makes the compiler wait for it at the join.
-  const int g0 = blockIdx.x;
-  const int gc = min(g0, d.L - 1);
-  const int leaf0 = d.gathered[gc];
-  const int4 ra0 = d.gl_rec[2 * gc], rb0 = d.gl_rec[2 * gc + 1];
-  const long long ng_ctr = d.ctr[SG_CTR_NGATHER];
-  const int ng = (int)ng_ctr;
-  const int stamp = d.dstamp[serial & 1];
+  const int seg = g0 % SG_CH_SEG;
+  g0 /= SG_CH_SEG;  // the workgroup's first entry of its segment
+  const int *list = d.ch_leaf + ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  const int4 *recs = d.ch_rec + 2 * ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  long long *lines = d.ch_ctr + (size_t)(serial % 3) * SG_CH_SEG * SG_CH_CTR;
+  long long *lines1 = d.ch_ctr + (size_t)((serial + 1) % 3) * SG_CH_SEG * SG_CH_CTR;
+  const int gc = min(g0, d.ch_cap - 1);
+  const int leaf0 = list[gc];
+  const int4 ra0 = recs[2 * gc], rb0 = recs[2 * gc + 1];
+  const int ng = (int)lines[seg * SG_CH_CTR];
+  const int stamp = d.dstamp[0] + serial;
+  const bool undo = undo_active(d);
+  if (g0 == 0 && tid == 0) d.pend[(serial & 1) * SG_CH_SEG + seg] = ng;  // what the copy-back takes
+  const float4 *stp = d.st_pos + (size_t)((serial + 1) & 1) * d.V, *stn = d.st_nor + (size_t)((serial + 1) & 1) * d.V;
+  float4 *wtp = d.st_pos + (size_t)(serial & 1) * d.V, *wtn = d.st_nor + (size_t)(serial & 1) * d.V;
+  const bool next_draw = ca.has_next && kn.tool == SG_TOOL_DRAW;
   const bool smooth = k.tool == SG_TOOL_SMOOTH;
   const int K = smooth ? k.iters : 0;
-  if (blockIdx.x == 0 && tid == 0) {  // this dab's results wait for the copy-back
-    d.pend[0] = ng;
-    d.pend[1] = stamp;
-  }
   // Draw offset: (normalize(area) * r) * bstrength
   float ox = 0.0f, oy = 0.0f, oz = 0.0f;
   if (k.tool == SG_TOOL_DRAW) {
-    float ax = (float)((double)d.ctr[SG_CTR_AREA_X] * (1.0 / 4294967296.0));
-    float ay = (float)((double)d.ctr[SG_CTR_AREA_Y] * (1.0 / 4294967296.0));
-    float az = (float)((double)d.ctr[SG_CTR_AREA_Z] * (1.0 / 4294967296.0));
+    long long sx = 0, sy = 0, sz = 0;
+#pragma unroll
+    for (int q = 0; q < SG_CH_AREA; q++) {
+      sx += lines[q * SG_CH_CTR + SG_CTR_AREA_X];
+      sy += lines[q * SG_CH_CTR + SG_CTR_AREA_Y];
+      sz += lines[q * SG_CH_CTR + SG_CTR_AREA_Z];
+    }
+    float ax = (float)((double)sx * (1.0 / 4294967296.0));
+    float ay = (float)((double)sy * (1.0 / 4294967296.0));
+    float az = (float)((double)sz * (1.0 / 4294967296.0));
     sg_normalize(ax, ay, az);
     ox = (ax * k.r) * k.bstr;
     oy = (ay * k.r) * k.bstr;
     oz = (az * k.r) * k.bstr;
   }
+  // the host reads the last dab's lists by gathered leaf: entries before this segment's
+  int gbase = 0;
+  if (ca.last)
+    for (int q = 0; q < seg; q++) gbase += (int)lines[q * SG_CH_CTR];
   const bool hide = d.vhide && d.respect_hide;
-  for (int g = g0; g < ng; g += gridDim.x) {
+  for (int g = g0; g < ng; g += ca.nf / SG_CH_SEG) {
     const bool first = g == g0;
-    const int leaf = first ? leaf0 : d.gathered[g];
-    const int4 ra = first ? ra0 : d.gl_rec[2 * g], rb = first ? rb0 : d.gl_rec[2 * g + 1];
+    const int leaf = first ? leaf0 : list[g];
+    const int4 ra = first ? ra0 : recs[2 * g], rb = first ? rb0 : recs[2 * g + 1];
     const int nu = rb.x & 0xffff, ns = rb.x >> 16;
     const int2 vr = make_int2(ra.x, ra.x + nu), sr = make_int2(ra.y, ra.y + ns);
     const int ext_off = ra.z, nb_blk = ra.w;
@@ -918,8 +1065,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
     const int nloc = nu + ring_end(K);
     const int ninner = K > 0 ? nu + ring_end(K - 1) : 0;  // locals the first Jacobi step updates
     if (tid == 0) s_cnt = 0;
-    if ((ng_ctr & SG_NGATHER_UNDO) && tid < SG_WAVE) undo_save_leaf(d, leaf, vr, d.px, d.py, d.pz);
+    // A leaf saved here moves for the first time in the open step, so the mesh arrays
+    // hold its state before the dab (C writes leaves that an earlier dab saved).
+    if (undo && tid < SG_WAVE) undo_save_leaf(d, leaf, vr, d.px, d.py, d.pz);
     // level 2
+    const int cut = d.leaf_cut[leaf];
     int vid[LPT], owner[LPT], nbb[LPT], nbe[LPT];
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
@@ -956,16 +1106,19 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
     // level 3
     // stand-ins keep the loads unconditional without new traffic: a tool that needs no
     // normals, or a mesh with no mask or hidden vertices, reads the position lines again
-    const bool inflate = k.tool == SG_TOOL_INFLATE;
+    const bool need_n = k.tool == SG_TOOL_INFLATE || next_draw;
     const float *mp = d.mask ? d.mask : d.px;
     const int *hp = hide ? d.vhide : (const int *)d.px;
-    const float *nxp = inflate ? d.nx : d.px, *nyp = inflate ? d.ny : d.py, *nzp = inflate ? d.nz : d.pz;
+    const float *nxp = need_n ? d.nx : d.px, *nyp = need_n ? d.ny : d.py, *nzp = need_n ? d.nz : d.pz;
+    const float4 *snp = need_n ? stn : stp;
+    const int *gst = d.ch_gstamp + (size_t)(serial & 1) * L;
     float x[LPT], y[LPT], z[LPT], nxv[LPT], nyv[LPT], nzv[LPT], mk[LPT];
     bool own[LPT], hid[LPT];
     unsigned short nb[LPT][FUSED_ROW];
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
       const int v = vid[j] < 0 ? 0 : vid[j];
+      const float4 a = stp[v], b = snp[v];
       x[j] = d.px[v];
       y[j] = d.py[v];
       z[j] = d.pz[v];
@@ -974,7 +1127,14 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
       nzv[j] = nzp[v];
       const float m = mp[v];
       const int hv = hp[v];
-      const int gs = d.leaf_gstamp[owner[j] < 0 ? 0 : owner[j]];
+      const int gs = gst[owner[j] < 0 ? 0 : owner[j]];
+      const bool st = __float_as_int(a.w) == stamp - 1;  // moved by the dab before: staged
+      x[j] = st ? a.x : x[j];
+      y[j] = st ? a.y : y[j];
+      z[j] = st ? a.z : z[j];
+      nxv[j] = st ? b.x : nxv[j];
+      nyv[j] = st ? b.y : nyv[j];
+      nzv[j] = st ? b.z : nzv[j];
       mk[j] = d.mask ? m : 0.0f;
       hid[j] = hide && hv != 0;
       own[j] = owner[j] < 0 || gs == stamp;  // its leaf was gathered by this search
@@ -1068,6 +1228,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
     // the affected uniq vertices: normal (spec S10, incident tris in vertex->tri order),
     // position, list record
     const float4 *F = S + cur * cap;  // final positions of the locals
+    bool pass = false;
+    int slot = 0;
     if (tid < FUSED_FACE_THREADS) {
       // each face normal once (spec S10's face normal; faces in the tables' order)
       auto face_normal = [&](unsigned c0, unsigned c1, int j) {
@@ -1101,15 +1263,35 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
       if (lane == SG_WAVE - 1) {
         bb_store(d.leaf_bb + 8 * (size_t)leaf, acc);
         bb_store(d.leaf_obb + 8 * (size_t)leaf, acc);
+        d.cut_dirty[cut] = 1;
+        d.draw_dirty[cut] = 1;  // the subtree's leaves need new draw records (UpdateDrawBuffers)
+        if (ca.last) d.gathered[gbase + g] = leaf;
+        // dab i + 1's search for this leaf (visible or not is the same for both dabs)
+        pass = ca.has_next && sphere_box(acc, kn.cx, kn.cy, kn.cz, kn.r2);
+        s_next = pass ? 1 : 0;
+        if (pass) slot = (int)atomicAdd((unsigned long long *)&lines1[seg * SG_CH_CTR], 1ull);  // the leaf's segment
       }
     }
     __syncthreads();
+    if (pass) {  // (the last lane; its slot arrived during the barrier)
+      const size_t q = ((size_t)((serial + 1) % 3) * SG_CH_SEG + seg) * d.ch_cap + slot;
+      d.ch_leaf[q] = leaf;
+      d.ch_rec[2 * q] = ra;
+      d.ch_rec[2 * q + 1] = rb;
+      d.ch_gstamp[(size_t)((serial + 1) & 1) * L + leaf] = stamp + 1;
+    }
+    AreaSum area = {0, 0, 0, 0};
+    const bool area_leaf = next_draw && s_next != 0;
     // the affected uniq vertices: normal (the incident faces' normals summed in
     // vertex->tri order), position, list record
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
       const int i = tid + j * FUSED_THREADS;
-      if (i >= nu || !aff[j]) continue;
+      if (i >= nu) continue;
+      if (!aff[j]) {
+        if (area_leaf) area_add(area, kn, x[j], y[j], z[j], nxv[j], nyv[j], nzv[j], !hid[j]);
+        continue;
+      }
       const int v = vr.x + i;
       float ax = 0.0f, ay = 0.0f, az = 0.0f;
       auto add_face = [&](int f) {
@@ -1129,31 +1311,39 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_fused(SgDevView d, SgDabK
         for (int q = qb; q < qe; q++) add_face(d.hl_ti[q]);
       }
       sg_normalize(ax, ay, az);
-      d.mx[v] = ax;
-      d.my[v] = ay;
-      d.mz[v] = az;
-      d.qx[v] = x[j];
-      d.qy[v] = y[j];
-      d.qz[v] = z[j];
-      const int pos = atomicAdd(&s_cnt, 1);
-      d.aff_v[(g << d.aff_shift) + pos] = v;
+      wtp[v] = make_float4(x[j], y[j], z[j], __int_as_float(stamp));
+      wtn[v] = make_float4(ax, ay, az, 0.0f);
+      if (area_leaf) area_add(area, kn, x[j], y[j], z[j], ax, ay, az, true);
+      if (ca.last || ca.log) {
+        const int pos = atomicAdd(&s_cnt, 1);
+        if (ca.last) d.aff_v[((gbase + g) << d.aff_shift) + pos] = v;
+      }
     }
-    __syncthreads();
-    if (tid == 0) d.aff_cnt[g] = s_cnt;
-    __syncthreads();  // LDS is reused by the next leaf
+    if (area_leaf) area_flush(area, lines1 + seg % SG_CH_AREA * SG_CH_CTR);
+    __syncthreads();  // the count is complete, and LDS is reused by the next leaf
+    if (tid == 0 && ca.last) d.aff_cnt[gbase + g] = s_cnt;
+    if (tid == 0 && ca.log)
+      atomicAdd((unsigned long long *)&lines[seg * SG_CH_CTR + SG_CTR_NAFF], (unsigned long long)s_cnt);
+    if (g + ca.nf / SG_CH_SEG < ng) __syncthreads();
   }
 }
 
-// After the last dab of a stroke (or a single dab): when that dab was fused, copy its
-// results in, and give it its affected count.
+// After a chain: copy its last dab's results in, hand the dab's counters (with its
+// affected count) to the counter set of its serial, and leave the other set and the
+// chain's own sets clear for what follows.
 __global__ __launch_bounds__(256) void k_dab_finish(SgDevView d, int serial) {
-  const int stamp = d.dstamp[serial & 1];
-  if (d.pend[1] != stamp) return;
-  fused_copy_back(d, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+  if (d.halt && d.halt[0]) return;
+  chain_copy_back(d, serial, (blockIdx.x * blockDim.x + threadIdx.x) / SG_WAVE, gridDim.x * blockDim.x / SG_WAVE);
   if (blockIdx.x == 0 && threadIdx.x < SG_WAVE) {
     const CountPrefetch cp = aff_count_prefetch(d, threadIdx.x);
-    const int s = aff_count_sum(d, cp, threadIdx.x, d.pend[0]);
-    if (threadIdx.x == 0) d.ctr[SG_CTR_NAFF] = s;
+    long long *lines = d.ch_ctr + (size_t)(serial % 3) * SG_CH_SEG * SG_CH_CTR;
+    const int ng = (int)chain_counter(lines, SG_CTR_NGATHER);
+    const int s = aff_count_sum(d, cp, threadIdx.x, ng);
+    if (threadIdx.x < SG_CTR_COUNT) {
+      d.ctr[threadIdx.x] = threadIdx.x == SG_CTR_NAFF ? (long long)s : chain_counter(lines, threadIdx.x);
+      d.ctr_next[threadIdx.x] = 0;
+    }
+    for (int i = threadIdx.x; i < SG_CH_SEG * SG_CH_CTR; i += SG_WAVE) lines[i] = 0;
   }
 }
 
@@ -1599,13 +1789,15 @@ SgDevView sg_view_of(SgDev &d, bool respect_hide, bool halt_live) {
   v.hl_nbl = d.hl_nbl;
   v.hl_sh = d.hl_sh;
   v.hl_ti = d.hl_ti;
-  v.gl_rec = d.gl_rec;
-  v.leaf_gstamp = d.leaf_gstamp;
+  v.ch_leaf = d.ch_leaf;
+  v.ch_rec = d.ch_rec;
+  v.ch_gstamp = d.ch_gstamp;
+  v.ch_ctr = d.ch_ctr;
+  v.ch_cap = (d.L + SG_CH_SEG - 1) / SG_CH_SEG;
   v.dstamp = d.dstamp;
   v.pend = d.pend;
-  v.mx = d.mx;
-  v.my = d.my;
-  v.mz = d.mz;
+  v.st_pos = d.st_pos;
+  v.st_nor = d.st_nor;
   v.halt = halt_live ? d.halt : nullptr;  // no flag test in strokes without learned dabs
   v.seq = d.seq;
   v.vstamp = d.vstamp;
@@ -1716,15 +1908,39 @@ int sg_profile_collect(PBVH *p) {
   return 0;
 }
 
-int sg_enqueue_clear_ctr(PBVH *p) {
-  hipLaunchKernelGGL(k_clear_ctr, dim3(1), dim3(64), 0, p->stream, p->d.ctr, p->d.halt, p->d.dstamp);
+int sg_enqueue_clear_ctr(PBVH *p, int ndabs) {
+  p->fused_pending = p->chain_live = false;  // (a failed enqueue may have left them set)
+  hipLaunchKernelGGL(k_clear_ctr, dim3(1), dim3(128), 0, p->stream, p->d.ctr, p->d.halt, p->d.dstamp, p->d.ch_ctr,
+                     ndabs);
   return sg_check_hip(hipGetLastError(), "clear launch");
 }
 
+// LDS and locals per thread of the chain kernel for dab k; lpt 0 when the mesh has no
+// halo tables or the dab is not one it covers.
+struct FusedShape {
+  int cap = 0, fcap = 1, lpt = 0;
+  size_t lds = 0;
+};
+static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
+  FusedShape f;
+  const bool tool = k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_GRAB ||
+                    (k.tool == SG_TOOL_SMOOTH && k.iters >= 1 && k.iters <= SG_HALO_RINGS);
+  if (!p->d.halo_ok || !p->fused_enabled || !tool || k.stats || k.orig_co || (k.learned && p->mlp)) return f;
+  f.cap = p->d.halo_maxlocr[k.tool == SG_TOOL_SMOOTH ? k.iters : 0];
+  f.fcap = std::max(1, p->d.halo_maxlt);
+  f.lds = (size_t)f.cap * 2 * sizeof(float4) + (size_t)f.fcap * sizeof(float4) + (size_t)(p->d.leaf_maxsh + 2) * 2 + 16;
+  const int lpt = (f.cap + FUSED_THREADS - 1) / FUSED_THREADS;
+  // larger halos (very large leaves) take the separate kernels
+  f.lpt = lpt >= 1 && lpt <= 4 && f.lds <= 65536 - 4096 ? lpt : 0;
+  return f;
+}
+
 // One dab; `serial` is the dab's position in its stroke (selects the counter set and
-// the "touched by the previous dab" test of the search).
+// the "touched by the previous dab" test of the search).  `next`: the dab that follows it
+// at once on the stream (serial + 1, no ray placement), or null; when both are fused, this
+// dab's launch also searches for that one.
 int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index,
-                   int stamp, int serial, const SgCollect *col, const float *place) {
+                   int stamp, int serial, const SgCollect *col, const float *place, const SgDabK *next) {
   SgDevView v = sg_view(p);
   v.ctr = p->d.ctr + (size_t)(serial & 1) * SG_CTR_COUNT;
   v.ctr_next = p->d.ctr + (size_t)((serial + 1) & 1) * SG_CTR_COUNT;
@@ -1733,51 +1949,60 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
   const int GB = p->grid_brush > 0 ? p->grid_brush : G;
   const int GP = p->grid_post > 0 ? p->grid_post : G;
   const int GS = p->grid_smooth > 0 ? p->grid_smooth : G;
-  // the fused dab (one kernel after the search) when the mesh has halo tables and the
+  // the fused dab (one launch, chained to the next) when the mesh has halo tables and the
   // dab is a plain brush dab it covers
   SgDabK kk = k;
   // no leaf is fully hidden: the hidden test passes every leaf, and the search skips
   // loading the flags
   if (p->d.nhidden_leaves == 0) kk.hide_skip = 0;
-  kk.fused = 0;
-  const bool fused_tool = k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_GRAB ||
-                          (k.tool == SG_TOOL_SMOOTH && k.iters >= 1 && k.iters <= SG_HALO_RINGS);
-  int fused_cap = 0, fused_fcap = 1, lpt = 0;
-  size_t lds = 0;
-  if (p->d.halo_ok && p->fused_enabled && fused_tool && !k.stats && !k.orig_co && !(k.learned && p->mlp) && !col &&
-      !place) {
-    fused_cap = p->d.halo_maxlocr[k.tool == SG_TOOL_SMOOTH ? k.iters : 0];
-    lpt = (fused_cap + FUSED_THREADS - 1) / FUSED_THREADS;
-    fused_fcap = std::max(1, p->d.halo_maxlt);
-    lds = (size_t)fused_cap * 2 * sizeof(float4) + (size_t)fused_fcap * sizeof(float4) +
-          (size_t)(p->d.leaf_maxsh + 2) * 2 + 16;
-    // larger halos (very large leaves) take the separate kernels
-    kk.fused = lpt >= 1 && lpt <= 4 && lds <= 65536 ? 1 : 0;
-  }
-  const int copy_blocks = p->d.halo_ok ? 64 : 0;
-  {
-    ProfScope ps(p, SG_K_SEARCH);
-    const int leaf_blocks = std::max(1, (p->d.L + 255) / 256);
-    const int cut_blocks = (p->d.C + 1 + 3) / 4;  // a wave per subtree and one for the bookkeeping
-    SG_LAUNCH(ps, k_search, dim3(leaf_blocks + cut_blocks + copy_blocks), dim3(256), 0, s, v, kk, log, log_index,
-              serial, place, leaf_blocks, cut_blocks, copy_blocks, p->fused_pending ? 1 : 0);
-    p->fused_pending = kk.fused != 0;
+  FusedShape fs;
+  if (!col && !place) fs = fused_shape(p, k);
+  kk.fused = fs.lpt > 0 ? 1 : 0;
+  const int leaf_blocks = std::max(1, (p->d.L + 255) / 256);
+  const bool chained = kk.fused && p->chain_live;  // the previous dab's launch searched for this one
+  if (!kk.fused && p->fused_pending)
+    if (int rc = sg_enqueue_finish(p, serial - 1)) return rc;
+  if (!chained) {
+    {
+      ProfScope ps(p, SG_K_SEARCH);
+      const int nrefresh = place || k.stats ? p->d.C : 0;
+      const int cut_blocks = (nrefresh + 1 + 3) / 4;  // a wave per subtree and one for the bookkeeping
+      SG_LAUNCH(ps, k_search, dim3(leaf_blocks + cut_blocks), dim3(256), 0, s, v, kk, log, log_index, serial, place,
+                cut_blocks, nrefresh);
+    }
+    if (kk.fused && k.tool == SG_TOOL_DRAW) {
+      ProfScope ps(p, SG_K_AREA);
+      SG_LAUNCH(ps, k_area, dim3(GB), dim3(256), 0, s, v, k, place,
+                p->d.ch_ctr + (size_t)(serial % 3) * SG_CH_SEG * SG_CH_CTR);
+    }
   }
   if (kk.fused) {
-    if (k.tool == SG_TOOL_DRAW) {
-      ProfScope ps(p, SG_K_AREA);
-      SG_LAUNCH(ps, k_area, dim3(GB), dim3(256), 0, s, v, k, place);
-    }
+    SgDabK kn = next ? *next : k;
+    if (p->d.nhidden_leaves == 0) kn.hide_skip = 0;
+    SgChainArgs ca;
+    ca.serial = serial;
+    ca.has_next = next && fused_shape(p, *next).lpt > 0 ? 1 : 0;
+    ca.has_prev = chained ? 1 : 0;
+    ca.last = ca.has_next ? 0 : 1;
+    ca.nf = p->grid_fused;
+    ca.f0 = std::min(ca.nf, FUSED_LEAD);
+    ca.ns = ca.has_next ? leaf_blocks : 0;
+    ca.nc = ca.has_prev ? 128 : 0;
+    ca.cap = fs.cap;
+    ca.fcap = fs.fcap;
+    ca.log = log;
     ProfScope ps(p, SG_K_BRUSH);
-    const dim3 gf(p->grid_fused), bf(FUSED_THREADS);
-    if (lpt == 1)
-      SG_LAUNCH(ps, k_dab_fused<1>, gf, bf, lds, s, v, kk, curve_dev, serial, fused_cap, fused_fcap);
-    else if (lpt == 2)
-      SG_LAUNCH(ps, k_dab_fused<2>, gf, bf, lds, s, v, kk, curve_dev, serial, fused_cap, fused_fcap);
-    else if (lpt == 3)
-      SG_LAUNCH(ps, k_dab_fused<3>, gf, bf, lds, s, v, kk, curve_dev, serial, fused_cap, fused_fcap);
+    const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(FUSED_THREADS);
+    if (fs.lpt == 1)
+      SG_LAUNCH(ps, k_dab_chain<1>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+    else if (fs.lpt == 2)
+      SG_LAUNCH(ps, k_dab_chain<2>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+    else if (fs.lpt == 3)
+      SG_LAUNCH(ps, k_dab_chain<3>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
     else
-      SG_LAUNCH(ps, k_dab_fused<4>, gf, bf, lds, s, v, kk, curve_dev, serial, fused_cap, fused_fcap);
+      SG_LAUNCH(ps, k_dab_chain<4>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+    p->chain_live = ca.has_next != 0;
+    p->fused_pending = true;
     return sg_check_hip(hipGetLastError(), "dab launch");
   }
   if (k.tool == SG_TOOL_ELASTIC_DEFORM) {  // every leaf; then all normals, leaf boxes and the tree
@@ -1823,7 +2048,7 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
   }
   if (k.tool == SG_TOOL_DRAW) {
     ProfScope ps(p, SG_K_AREA);
-    SG_LAUNCH(ps, k_area, dim3(GB), dim3(256), 0, s, v, k, place);
+    SG_LAUNCH(ps, k_area, dim3(GB), dim3(256), 0, s, v, k, place, (long long *)nullptr);
   }
   if (k.orig_co) {
     ProfScope ps(p, SG_K_BRUSH);
@@ -1916,11 +2141,13 @@ int sg_enqueue_coords_apply(PBVH *p, const float *src_dev) {
 }
 
 int sg_enqueue_finish(PBVH *p, int serial_last) {
+  if (!p->fused_pending) return 0;
   p->fused_pending = false;
-  if (!p->d.halo_ok) return 0;
+  p->chain_live = false;
   SgDevView v = sg_view(p);
   v.ctr = p->d.ctr + (size_t)(serial_last & 1) * SG_CTR_COUNT;  // the last dab's counter set
-  hipLaunchKernelGGL(k_dab_finish, dim3(64), dim3(256), 0, p->stream, v, serial_last);
+  v.ctr_next = p->d.ctr + (size_t)((serial_last + 1) & 1) * SG_CTR_COUNT;
+  hipLaunchKernelGGL(k_dab_finish, dim3(128), dim3(256), 0, p->stream, v, serial_last);
   return sg_check_hip(hipGetLastError(), "finish launch");
 }
 

@@ -820,13 +820,16 @@ static bool build_halo(PBVH *p, const SgLayout &h, hipStream_t s) {
   rc |= upload(&d.hl_nbl, nbl.data(), nbl.size(), s);
   rc |= upload(&d.hl_ti, ti.data(), std::max<size_t>(ti.size(), 1), s);
   rc |= upload(&d.hl_sh, shl.data(), std::max<size_t>(shl.size(), 1), s);
-  rc |= alloc_fill(&d.leaf_gstamp, std::max(L, 1), 0xFF, s);  // -1: no dab's stamp (stamps start at 1)
-  rc |= alloc_fill(&d.dstamp, 2, 0, s);
-  rc |= alloc_fill(&d.pend, 4, 0xFF, s);  // no fused dab pending
-  rc |= alloc_fill(&d.mx, V, 0, s);
-  rc |= alloc_fill(&d.my, V, 0, s);
-  rc |= alloc_fill(&d.mz, V, 0, s);
-  rc |= alloc_fill(&d.gl_rec, 2 * std::max(L, 1), 0, s);
+  const size_t L1 = (size_t)std::max(L, 1), V1 = (size_t)std::max(V, 1);
+  rc |= alloc_fill(&d.dstamp, 2, 0, s);  // stamps start at 2: no leaf or vertex carries one yet
+  const size_t cap = (L1 + SG_CH_SEG - 1) / SG_CH_SEG;
+  rc |= alloc_fill(&d.pend, 2 * SG_CH_SEG, 0, s);
+  rc |= alloc_fill(&d.ch_leaf, 3 * SG_CH_SEG * cap, 0, s);
+  rc |= alloc_fill(&d.ch_rec, 6 * SG_CH_SEG * cap, 0, s);
+  rc |= alloc_fill(&d.ch_gstamp, 2 * L1, 0, s);
+  rc |= alloc_fill(&d.ch_ctr, 3 * SG_CH_SEG * SG_CH_CTR, 0, s);
+  rc |= alloc_fill(&d.st_pos, 2 * V1, 0, s);
+  rc |= alloc_fill(&d.st_nor, 2 * V1, 0, s);
   hipStreamSynchronize(s);  // the host tables are freed on return
   d.halo_maxloc = maxloc;
   d.halo_maxloc0 = maxloc0;
@@ -1061,8 +1064,8 @@ void sg_free_device(PBVH *p) {
                   d.draw_poly_v, d.draw_vbo, d.undo, d.undo_stamp, d.undo_slot, d.place_pair,
                   d.prox_dev, d.prox_tab, d.prox_leaves, d.prox_off, d.poly_off, d.poly_v,
                   d.poly_of_tri, d.vc_off, d.vc, d.stage, d.hl_rec, d.hl_v, d.hl_nboff,
-                  d.hl_nbl, d.hl_ti, d.hl_sh, d.leaf_gstamp, d.dstamp, d.mx, d.my, d.mz, d.pend,
-                  d.gl_rec};
+                  d.hl_nbl, d.hl_ti, d.hl_sh, d.dstamp, d.pend, d.ch_leaf, d.ch_rec, d.ch_gstamp,
+                  d.ch_ctr, d.st_pos, d.st_nor};
   for (void *q : ptrs) {
     if (q) hipFree(q);
   }

@@ -428,6 +428,21 @@ __device__ __forceinline__ long long wave_sum_ll(long long v) {
   for (int off = SG_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
   return v;
 }
+// The same total by a scan over DPP lane moves (no LDS round trips), in lane 63 only.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ long long dpp_add_ll(long long v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)as_u64(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(as_u64(v) >> 32), CTRL, ROWS, 0xf, false);
+  return v + (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ long long wave_total_ll(long long v) {
+  v = dpp_add_ll<0x111, 0xf>(v);   // row_shr:1
+  v = dpp_add_ll<0x112, 0xf>(v);   // row_shr:2
+  v = dpp_add_ll<0x114, 0xf>(v);   // row_shr:4
+  v = dpp_add_ll<0x118, 0xf>(v);   // row_shr:8
+  v = dpp_add_ll<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  return dpp_add_ll<0x143, 0xc>(v);  // row_bcast:31 into rows 2 and 3
+}
 __device__ __forceinline__ int wave_sum_i(int v) {
   for (int off = SG_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off);
   return v;

@@ -9,6 +9,10 @@
 
 #include "../../include/sculpt_gpu.h"
 
+#define SG_CH_SEG 16  // segments of a chained dab's leaf list and counters, by leaf number (divides the wave size)
+#define SG_CH_CTR 8   // counters of a segment (a 64-byte line): SG_CTR_NGATHER .. SG_CTR_AREA_Z, then SG_CH_NAREA
+#define SG_CH_NAREA 5
+#define SG_CH_AREA 4   // segments whose lines take area-normal sums
 #define SG_HALO_RINGS 4  // Smooth(k) runs fused for k <= this
 
 // Cut of the tree used by the two-level sphere search: maximal subtrees holding at
@@ -177,11 +181,16 @@ struct SgDev {
                                      // its vertex's leaf; the leaf's faces (corners as local ids, c0 | c1 << 16,
                                      // c2) follow its neighbour offsets in hl_nboff
   unsigned short *hl_sh = nullptr;   // parallel to leaf_sh: local id of each shared vertex
-  int *leaf_gstamp = nullptr;   // [L] dab stamp of the last search that gathered the leaf
-  int *dstamp = nullptr;        // [2] dab stamps by counter-set parity
-  float *mx = nullptr, *my = nullptr, *mz = nullptr;  // [V] normals the fused kernel wrote, copied in by the next search
-  int *pend = nullptr;          // [4] the fused dab whose results wait for that copy: gathered count, stamp
-  int4 *gl_rec = nullptr;                 // [2L] the gathered leaves' records (fused dabs)
+  // Chained fused dabs (k_dab_chain): per dab modulo 3 the gathered leaves, their records
+  // and the counters, each in SG_CH_SEG segments (cap = ceil(L / SG_CH_SEG) leaves); by the dab's parity the gather stamps, the gathered count and the
+  // staged results (position and stamp, normal), copied in by the next dab's launch
+  int *ch_leaf = nullptr;       // [3][SG_CH_SEG][cap]
+  int4 *ch_rec = nullptr;       // [3][SG_CH_SEG][2 cap]
+  long long *ch_ctr = nullptr;  // [3][SG_CH_SEG][SG_CH_CTR]
+  int *ch_gstamp = nullptr;     // [2 L] stamp of the last dab (of this parity) that gathered the leaf
+  int *dstamp = nullptr;        // [2] the stroke's first stamp (dab i has stamp + i), one past its last
+  int *pend = nullptr;          // [2][SG_CH_SEG] gathered leaves of the staged dab
+  float4 *st_pos = nullptr, *st_nor = nullptr;  // [2 V]
   int halo_maxnbl = 0, leaf_maxsh = 0;    // most neighbour entries / shared vertices of a leaf
   int halo_maxlt = 0;                     // most faces incident to a leaf's uniq vertices
   int halo_maxlocr[SG_HALO_RINGS + 1] = {};  // most locals of a leaf up to ring j (uniq + rings 0..j)
@@ -271,6 +280,7 @@ struct PBVH {
   int grid_fused = 1024;             // workgroups of the fused dab kernel (a leaf each)
   bool fused_enabled = true;
   bool fused_pending = false;        // the last dab enqueued was fused and no finish followed yet
+  bool chain_live = false;           // ... and its launch searches for the next one
   // device snapshot (checkpoint) of the mutable mesh state
   // slot 0: the caller's (sg_pbvh_snapshot_save/restore); slot 1: internal (autotuner, judge)
   std::vector<void *> snap[2];

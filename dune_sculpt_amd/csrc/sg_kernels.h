@@ -77,16 +77,17 @@ struct SgDevView {
   long long *ctr, *ctr_next;
   const int *vperm_old;
   int *stamp_v, *stamp_v2, *stamp_t, *stamp_a;
-  // fused dabs: per-leaf halos, the gathered leaves' halo headers, gather stamps, dab
-  // stamps, the normals the fused kernel wrote and its pending record
+  // fused dabs: per-leaf halos, and the chain's lists, stamps, counters and staged results
   const int4 *hl_rec;
   const int2 *hl_v;
   const int *hl_nboff;
   const unsigned short *hl_nbl, *hl_sh;
   const unsigned short *hl_ti;
-  int4 *gl_rec;
-  int *leaf_gstamp, *dstamp, *pend;
-  float *mx, *my, *mz;
+  int4 *ch_rec;
+  int *ch_leaf, *ch_gstamp, *dstamp, *pend;
+  long long *ch_ctr;
+  int ch_cap;  // entries per list segment
+  float4 *st_pos, *st_nor;
 };
 
 // Per-dab constants (spec S1-S9), computed on the host in the same FP32 order as the
@@ -99,7 +100,7 @@ struct SgDabK {
   int hide_skip;  // 1: the search skips fully hidden subtrees and leaves; 0: every leaf (elastic deform)
   int etype;      // elastic deform mode
   float epois, enx, eny, enz, eforce;  // Poisson ratio, sculpt normal, force (Kelvinlet parameters)
-  int fused;      // the search fills the halo headers and gather stamps for the fused kernel
+  int fused;      // the search fills the chain's list and gather stamps
 };
 
 // kernel ids for the per-kernel profile
@@ -114,8 +115,9 @@ int sg_enqueue_gather_raw(hipStream_t s, const float *x, const float *y, const f
 int sg_profile_collect(PBVH *p);
 SgDabK sg_make_dab(const SgDabParams *dab, int stats);
 int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index,
-                   int stamp, int serial, const SgCollect *col = nullptr, const float *place = nullptr);
-int sg_enqueue_clear_ctr(PBVH *p);
+                   int stamp, int serial, const SgCollect *col = nullptr, const float *place = nullptr,
+                   const SgDabK *next = nullptr);
+int sg_enqueue_clear_ctr(PBVH *p, int ndabs);
 int sg_enqueue_flush(PBVH *p);
 int sg_enqueue_log_row(PBVH *p, long long *log, int row);
 int sg_enqueue_full_normals(PBVH *p);

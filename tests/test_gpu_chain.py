@@ -1,0 +1,122 @@
+"""Chained fused dabs (one launch per dab that also searches for the next one) against the
+separate kernels, bit for bit: positions, normals, every node box, the last dab's affected
+vertices and gathered leaves, per-dab logged counts.  At the chain's own edges: every
+position of the modulo-3 lists (lengths 1..7), chains broken by dabs that are not fused,
+meshes of fewer leaves than list segments, radii that jump (the next dab's area normal
+then comes from leaves the dab before did not touch), area spheres larger than the brush,
+hidden leaves, refit after every dab, replays, undo and what reads the mesh after it."""
+import numpy as np
+import pytest
+
+from parity_util import n_bit_diff
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(p):
+    n = p.tree_info()["nodes"]
+    boxes = np.array([np.concatenate([p.node_bb(i), p.node_bb(i, original=True)]) for i in range(n)], np.float32)
+    return p.positions(), p.normals(), boxes
+
+
+def _same(a, b):
+    return all(n_bit_diff(x, y) == 0 for x, y in zip(a, b))
+
+
+def _path(sg, n, seed, radii, tools, ks=(2,), spacing=0.3, **kw):
+    """Overlapping dabs along a great circle of the unit sphere."""
+    radii = np.asarray(radii, np.float32)
+    c = sg.great_circle_centres(seed, radii, spacing_frac=spacing)
+    rng = np.random.default_rng(seed)
+    return [sg.make_dab(tool=tools[i % len(tools)], location=c[i], radius=float(radii[i]),
+                        strength=float(rng.uniform(0.2, 1.0)), smooth_iterations=int(ks[i % len(ks)]),
+                        grab_delta=rng.normal(size=3) * 0.02, **kw) for i in range(n)]
+
+
+def _check(sg, co, tris, dabs, leaf=64, hidden=None, mask=None, **how):
+    a = sg.PBVH(co, tris, leaf_limit=leaf, hidden=hidden)
+    b = sg.PBVH(co, tris, leaf_limit=leaf, hidden=hidden)
+    assert a.set_fused(True)
+    b.set_fused(False)
+    for p in (a, b):
+        if mask is not None:
+            p.set_mask(mask)
+        p.stroke(dabs, log=True, **how)
+        p.stroke(dabs[::-1], log=True, **how)  # on what the first one left
+    assert np.array_equal(a.stroke_log(len(dabs))[:, :5], b.stroke_log(len(dabs))[:, :5])
+    assert np.array_equal(a.last_affected(), b.last_affected())
+    assert np.array_equal(a.last_gathered(), b.last_gathered())
+    assert np.array_equal(a.last_stats()[:2], b.last_stats()[:2])
+    assert _same(_state(a), _state(b))
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 6, 7])
+@pytest.mark.parametrize("graph", [True, False])
+def test_lengths(sg, n, graph):
+    co, tris = sg.noisy_icosphere(5, seed=3, amplitude=0.02)
+    _check(sg, co, tris, _path(sg, n, n, np.full(n, 0.2), (1, 4, 2, 5)), graph=graph)
+
+
+@pytest.mark.parametrize("tools,ks", [((1,), (1,)), ((1, 2), (4,)), ((2,), (1, 5, 4, 9)), ((4, 5, 1), (1,)),
+                                      ((1, 2, 2), (3, 6))])
+def test_broken_chains(sg, tools, ks):
+    """Smooth with more steps than the halo covers runs the separate kernels in between."""
+    co, tris = sg.noisy_icosphere(5, seed=4, amplitude=0.02)
+    _check(sg, co, tris, _path(sg, 24, 2, np.full(24, 0.15), tools, ks))
+
+
+@pytest.mark.parametrize("level,leaf", [(1, 128), (2, 128), (2, 20), (3, 9), (4, 300)])
+def test_few_and_odd_leaves(sg, level, leaf):
+    co, tris = sg.noisy_icosphere(level, seed=5, amplitude=0.02)
+    _check(sg, co, tris, _path(sg, 12, 6, np.full(12, 0.5), (1, 2, 4, 5)), leaf=leaf)
+
+
+@pytest.mark.parametrize("factor", [0.25, 0.5, 1.0, 1.7])
+def test_area_normal_of_jumping_radii(sg, factor):
+    co, tris = sg.noisy_icosphere(6, seed=6, amplitude=0.02)
+    radii = np.tile([0.05, 0.6, 0.1, 0.02, 0.9, 0.05], 4)
+    _check(sg, co, tris, _path(sg, 24, 7, radii, (1,), normal_radius_factor=factor), leaf=32)
+
+
+def test_hidden_masked_refit_each(sg):
+    co, tris = sg.noisy_icosphere(5, seed=8, amplitude=0.02)
+    hidden = co[:, 2] > 0.55
+    mask = np.clip(co[:, 0], 0, 1).astype(np.float32)
+    dabs = _path(sg, 30, 11, np.random.default_rng(1).uniform(0.05, 0.4, 30), (1, 4, 2, 5), (1, 4))
+    _check(sg, co, tris, dabs, hidden=hidden, mask=mask, refit_each=True)
+
+
+def test_replay_undo_and_readers(sg):
+    """A captured stroke replayed over a changed mesh, an undo step around it, then the
+    draw buffers and rays: as after the separate kernels."""
+    co, tris = sg.noisy_icosphere(5, seed=9, amplitude=0.02)
+    dabs = _path(sg, 17, 13, np.random.default_rng(2).uniform(0.05, 0.3, 17), (1, 2, 4, 5), (4,))
+    dirs = np.random.default_rng(3).normal(size=(200, 3))
+    dirs = (dirs / np.linalg.norm(dirs, axis=1, keepdims=True)).astype(np.float32)
+    got = []
+    for fused in (True, False):
+        p = sg.PBVH(co, tris, leaf_limit=64)
+        p.set_fused(fused)
+        p.draw_build(np.ones(len(tris), np.int32))
+        st = p.prepare(dabs)
+        p.undo_begin()
+        st.launch()
+        p.dab(dabs[3])
+        st.launch(sync=False)
+        st.launch()
+        p.undo_end()
+        out = [*_state(p)]
+        p.draw_update()
+        leaf = [i for i in range(p.tree_info()["nodes"]) if p.node_flag(i) & sg.PBVH_Leaf]
+        out.append(np.concatenate([p.draw_leaf(i)[0].reshape(-1) for i in leaf]))
+        p.stroke_placed(dabs[:6], -3 * dirs[:6], dirs[:6])
+        h = p.raycast(-3 * dirs, dirs)
+        out += [h[f] for f in ("hit", "depth", "looptri")] + [*_state(p)]
+        p.undo()
+        out += [*_state(p)]
+        got.append(out)
+        p.close()
+    for x, y in zip(*got):
+        assert x.tobytes() == y.tobytes()
