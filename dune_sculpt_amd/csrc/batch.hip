@@ -618,6 +618,7 @@ SgBatch *sg_batch_new(int n_meshes, const float *const *co, const int *const *tr
   DevBuf<int> vt_off, vv_off, vv_idx, leaf_sh, leaf_flags, cut_lbeg, cut_lend, cut_flags, cut_mesh, vperm;
   DevBuf<float> leaf_bb, leaf_obb, cut_bb;
   DevBuf<int2> leaf_vr, leaf_shr;
+  b->density.assign(n_meshes, 0.0);
   b->vbase.assign(1, 0);
   b->lbase.assign(1, 0);
   b->cbase.assign(1, 0);
@@ -648,6 +649,19 @@ SgBatch *sg_batch_new(int n_meshes, const float *const *co, const int *const *tr
             return;
           }
         }
+        // vertex density from up to 4096 triangles spread over the mesh
+        double area = 0.0;
+        const int step = std::max(1, T / 4096), ns = (T + step - 1) / step;
+        for (int q = 0; q < T; q += step) {
+          const float *A = co[m] + 3 * (size_t)tris[m][3 * (size_t)q], *B = co[m] + 3 * (size_t)tris[m][3 * (size_t)q + 1],
+                      *Cc = co[m] + 3 * (size_t)tris[m][3 * (size_t)q + 2];
+          const double ux = B[0] - A[0], uy = B[1] - A[1], uz = B[2] - A[2];
+          const double vx = Cc[0] - A[0], vy = Cc[1] - A[1], vz = Cc[2] - A[2];
+          const double nx = uy * vz - uz * vy, ny = uz * vx - ux * vz, nz = ux * vy - uy * vx;
+          area += 0.5 * std::sqrt(nx * nx + ny * ny + nz * nz);
+        }
+        area *= (double)T / ns;
+        b->density[m] = area > 0.0 ? V / area : 0.0;
         PBVH *p = new PBVH();
         p->no_device = true;
         p->leaf_limit = leaf_limit > 0 ? leaf_limit : 10000;
@@ -818,9 +832,6 @@ SgBatch *sg_batch_new(int n_meshes, const float *const *co, const int *const *tr
   if (!rc) {
     std::vector<int> mc(b->M + 1), ml(b->M + 1), mv(b->M + 1);
     b->pm_ok = true;
-    // a workgroup per mesh: by default only when the meshes are enough to spread over
-    // the chip (the autotuner times both)
-    b->persistent = b->M >= 128;
     for (int m = 0; m <= b->M; m++) {
       mc[m] = (int)b->cbase[m];
       ml[m] = (int)b->lbase[m];
@@ -874,6 +885,30 @@ int sg_batch_info(SgBatch *b, long long *out, int out_n) {
   return 0;
 }
 
+// Whether a table runs faster as one launch with a workgroup per mesh than as a graph per
+// step.  The persistent step lasts as long as its slowest mesh: 14 us per dab and 30 ns per
+// affected vertex on that mesh's one CU.  A step graph lasts 45 us (its 7 to 10 kernels and
+// their boundaries) and 0.45 ns per affected vertex of all meshes on the whole chip.
+// Measured per step, persistent / graph: 32 meshes of 5k-60k vertices 19.5 / 51.9 us; 2
+// meshes 15.3 / 43.9; 8 of 200k-500k 37.2 / 51.3; 96 of 5k-500k 34.6 / 59.5; 64 of 1M-4M
+// (r to 0.08) 92 / 92.
+static bool persistent_pays(const SgBatch *b, const SgDabParams *dabs, int steps) {
+  double slowest = 0.0, all = 0.0;
+  for (int m = 0; m < b->M; m++) {
+    const double nv = (double)(b->vbase[m + 1] - b->vbase[m]);
+    double t = 0.0;
+    for (int s = 0; s < steps; s++) {
+      const SgDabParams &p = dabs[(size_t)s * b->M + m];
+      if (p.sculpt_tool == 0) continue;
+      const double aff = std::min(nv, 3.14159 * (double)p.radius * (double)p.radius * b->density[m]);
+      t += 14.0 + 0.030 * aff;
+      all += aff;
+    }
+    slowest = std::max(slowest, t);
+  }
+  return slowest <= 45.0 * steps + 0.00045 * all;
+}
+
 // Upload a [steps][n_meshes] dab table (tool 0 = no dab for that mesh in that step)
 // and capture the step graph for it; sg_batch_launch then runs it.
 int sg_batch_load(SgBatch *b, const SgDabParams *dabs, int steps) {
@@ -922,6 +957,7 @@ int sg_batch_load(SgBatch *b, const SgDabParams *dabs, int steps) {
   b->maxk = maxk;
   b->learned = learned;
   b->odd_k = odd_k;
+  if (b->persistent_auto) b->persistent = persistent_pays(b, dabs, steps);
   const int cfg[] = {maxk, learned ? 1 : 0, odd_k ? 1 : 0, b->mlp ? 1 : 0, b->g_search, b->g_brush, b->g_smooth,
                      b->g_post, b->g_learned, b->brush_threads, b->brush_vpl};
   long long key = 1469598103934665603ll;
@@ -1084,6 +1120,7 @@ int sg_batch_timer_stop(SgBatch *b, float *ms) {
 int sg_batch_set_persistent(SgBatch *b, int on) {
   if (batch_check(b)) return -1;
   b->persistent = on != 0;
+  b->persistent_auto = false;
   return b->pm_ok ? 1 : 0;
 }
 
@@ -1126,6 +1163,7 @@ int sg_batch_autotune(SgBatch *b, const SgDabParams *dabs, int steps, double *ou
   // the step graph's launch shape first (the persistent step has none), then the
   // persistent step against the tuned graph
   const bool pm_entry = b->persistent;
+  b->persistent_auto = false;
   b->persistent = false;
   double best = pm_entry ? time_once() : start;
   if (best < 0) return -1;

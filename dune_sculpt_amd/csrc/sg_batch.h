@@ -109,7 +109,9 @@ struct SgBatch {
   int *pm_aff_v = nullptr, *pm_g_off = nullptr, *pm_err = nullptr;
   float *pm_aff_f = nullptr;
   bool pm_ok = false;       // every mesh fits the persistent step (at most 1024 search cuts)
-  bool persistent = false;  // graph launches of tables without learned dabs use it (default: >= 128 meshes)
+  bool persistent = false;  // graph launches of tables without learned dabs use it
+  bool persistent_auto = true;  // ... decided per loaded table, until the caller or the autotuner sets it
+  std::vector<double> density;  // [M] vertices per unit of surface area (sampled at the build)
 };
 
 // A learned Smooth dab of mesh m is rejected (the plain brush redoes it in the same
