@@ -532,7 +532,7 @@ int sg_dab_apply(PBVH *p, const SgDabParams *dab) {
   SgDabK k = sg_make_dab(dab, g_stats ? 1 : 0);
   const int stamp = (++p->stamp) * 128;
   p->halt_live = k.learned && p->mlp;
-  int rc = sg_enqueue_clear_ctr(p, 1);
+  int rc = sg_enqueue_clear_ctr(p, sg_dab_launches(k));
   if (!rc) rc = sg_enqueue_dab(p, k, curve, nullptr, 0, stamp, 0);
   if (!rc) rc = sg_enqueue_finish(p, 0);
   if (!rc) rc = sg_enqueue_flush(p);
@@ -655,7 +655,9 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
       int ci = 0;
       for (int i = 0; i < a0; i++)
         ci += (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table) ? 1 : 0;
-      if (sg_enqueue_clear_ctr(p, n - a0)) return -1;
+      int nlaunch = 0;
+      for (int i = a0; i < n; i++) nlaunch += sg_dab_launches(sg_make_dab(&dabs[i], 0));
+      if (sg_enqueue_clear_ctr(p, nlaunch)) return -1;
       for (int i = a0; i < n; i++) {
         const float *curve = nullptr;
         if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
@@ -898,7 +900,9 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
     rc = erc ? erc : sg_check_hip(e, "end capture");
   } else if (!rc) {
     int ci = 0;
-    erc = sg_enqueue_clear_ctr(p, n);
+    int nlaunch = 0;
+    for (int i = 0; i < n; i++) nlaunch += sg_dab_launches(sg_make_dab(&dabs[i], 0));
+    erc = sg_enqueue_clear_ctr(p, nlaunch);
     for (int i = 0; i < n && !erc; i++) {
       const float *curve = nullptr;
       if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)

@@ -210,9 +210,10 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
   if (k.stats && lane == 0) atomicAdd((unsigned long long *)&d.ctr[SG_CTR_TESTS], (unsigned long long)ntests);
 }
 
-// At the start of a stroke of n dabs: zero the counter sets and the halt flag, and take
-// the stamps dstamp[0] + serial for its dabs, above every earlier one and leaving the
-// stamp before the first one unused (no staged value belongs to "the dab before" it).
+// At the start of a stroke of n launches and dabs at most: zero the counter sets and the
+// halt flag, and take the stamps dstamp[0] + number for them, past every earlier one (the
+// 32-bit stamps wrap) and leaving the stamp before the first one unused (no staged value
+// belongs to "the launch before" it).
 __global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp, long long *ch_ctr, int n) {
   if (threadIdx.x < 2 * SG_CTR_COUNT) ctr[threadIdx.x] = 0;
   if (threadIdx.x == 0) halt[0] = 0;
@@ -811,9 +812,15 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // normal in another.  Whoever reads a vertex in launch i takes the staged value when it
 // carries dab i - 1's stamp and the mesh array otherwise: C may be writing exactly those
 // vertices' mesh values.  What launch i reads and writes at the same time therefore
-// differs in its slot: staging, gather stamps and copied counts by the dab's parity,
-// leaf lists and counters by the dab modulo 3 (dab i + 1's list fills while C reads dab
-// i - 1's).
+// differs in its slot: staging by the launch's parity, gather stamps and copied counts by
+// the dab's, leaf lists and counters by the dab modulo 3 (dab i + 1's list fills while C
+// reads dab i - 1's).
+//
+// Smooth(k) with k above the halo's rings runs as ceil(k / rings) launches over the dab's
+// list, each with an even share of the steps: a launch that another one continues stages
+// its positions and Smooth factors only, and the continuing launch takes the staged
+// vertices as the affected ones.  Smooth(8) on 655 k vertices, 60 dabs: 2.65 ms with a
+// kernel per step, 1.35 as two launches per dab.
 // ---------------------------------------------------------------------------
 #define FUSED_THREADS 256
 #define FUSED_LEAD 256  // F blocks started before the S and C blocks: more leaves than most dabs gather
@@ -831,7 +838,11 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 #define FUSED_FACE_THREADS 192   // the first three waves compute the face normals, the last the leaf box
 
 struct SgChainArgs {
-  int serial;
+  int ls;                    // the dab's number: lists, counters and gather stamps
+  int ss;                    // the launch's number: staged results (a Smooth of more steps than
+                             // the halo has rings is several launches over one list)
+  int iters;                 // Jacobi steps of this launch
+  int cont_in, cont_out;     // the launch continues a Smooth / another launch continues it
   int f0;                    // F blocks ahead of the S and C blocks in launch order
   int nf, ns, nc;            // F, S, C blocks
   int cap, fcap;             // LDS: locals, faces
@@ -840,16 +851,16 @@ struct SgChainArgs {
   long long *log;            // per-dab counter rows, or null
 };
 
-// Affected vertices of dab `serial` from staging into the mesh arrays: a wave per leaf it
-// gathered (its uniq range, staged entries of that dab only).
-__device__ __forceinline__ void chain_copy_back(const SgDevView &d, int serial, int gw, int nw) {
-  const float4 *sp = d.st_pos + (size_t)(serial & 1) * d.V, *sn = d.st_nor + (size_t)(serial & 1) * d.V;
+// Affected vertices of dab `ls`, staged by launch `ss`, into the mesh arrays: a wave per
+// leaf it gathered (its uniq range, entries of that launch only).
+__device__ __forceinline__ void chain_copy_back(const SgDevView &d, int ls, int ss, int gw, int nw) {
+  const float4 *sp = d.st_pos + (size_t)(ss & 1) * d.V, *sn = d.st_nor + (size_t)(ss & 1) * d.V;
   // wave gw takes its share of segment gw % SG_CH_SEG
   const int seg = gw % SG_CH_SEG, i0 = gw / SG_CH_SEG;
-  const int4 *rec = d.ch_rec + 2 * ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  const int4 *rec = d.ch_rec + 2 * ((size_t)(ls % 3) * SG_CH_SEG + seg) * d.ch_cap;
   const int gc = min(i0, d.ch_cap - 1);
   const int4 ra0 = rec[2 * gc], rb0 = rec[2 * gc + 1];
-  const int ng = d.pend[(serial & 1) * SG_CH_SEG + seg], stamp = d.dstamp[0] + serial;
+  const int ng = d.pend[(ls & 1) * SG_CH_SEG + seg], stamp = d.dstamp[0] + ss;
   for (int g = i0; g < ng; g += nw / SG_CH_SEG) {
     const int4 ra = g == i0 ? ra0 : rec[2 * g], rb = g == i0 ? rb0 : rec[2 * g + 1];
     const int nu = rb.x & 0xffff;
@@ -905,23 +916,23 @@ __device__ __forceinline__ void area_flush(const AreaSum &s, long long *ctr) {
   }
 }
 
-// S: dab serial + 1's search over the leaves that dab `serial` does not touch, block b.
-__device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &kn, int serial, int b, int2 *s_q,
+// S: dab ls + 1's search over the leaves that dab ls (launch ss) does not touch, block b.
+__device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &kn, int ls, int ss, int b, int2 *s_q,
                                              int *s_nq) {
   const int lane = lane_id();
   if (threadIdx.x == 0) *s_nq = 0;
   const int l = b * blockDim.x + threadIdx.x, lc = min(l, d.L - 1);
   const BB6 bb = bb_load((kn.use_orig ? d.leaf_obb : d.leaf_bb) + 8 * (size_t)lc);
-  const int gs = d.ch_gstamp[(size_t)(serial & 1) * d.L + lc];
+  const int gs = d.ch_gstamp[(size_t)(ls & 1) * d.L + lc];
   const int fl = kn.hide_skip ? d.leaf_flags[lc] : 0;
-  const int stamp = d.dstamp[0] + serial;
-  const bool pass = l < d.L && gs != stamp && !(fl & kn.hide_skip) && sphere_box(bb, kn.cx, kn.cy, kn.cz, kn.r2);
+  const int gstamp = d.dstamp[0] + ls, stamp = d.dstamp[0] + ss;
+  const bool pass = l < d.L && gs != gstamp && !(fl & kn.hide_skip) && sphere_box(bb, kn.cx, kn.cy, kn.cz, kn.r2);
   const unsigned long long m = __ballot(pass);
   int4 r0 = make_int4(0, 0, 0, 0), r1 = make_int4(0, 0, 0, 0);
   if (m) {
     r0 = d.hl_rec[2 * (size_t)lc];
     r1 = d.hl_rec[2 * (size_t)lc + 1];
-    chain_append(d, serial + 1, l, pass, m, r0, r1, stamp + 1);
+    chain_append(d, ls + 1, l, pass, m, r0, r1, gstamp + 1);
   }
   if (kn.tool != SG_TOOL_DRAW) return;
   // the area normal's share of the new leaves that reach into its sphere (usually none:
@@ -938,7 +949,7 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
   if (pass && t2 <= kn.nr2) s_q[atomicAdd(s_nq, 1)] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
   __syncthreads();
   const int nq = *s_nq;
-  const float4 *sp = d.st_pos + (size_t)((serial + 1) & 1) * d.V, *sn = d.st_nor + (size_t)((serial + 1) & 1) * d.V;
+  const float4 *sp = d.st_pos + (size_t)((ss + 1) & 1) * d.V, *sn = d.st_nor + (size_t)((ss + 1) & 1) * d.V;
   const bool hide = d.vhide && d.respect_hide;
   const int *hp = hide ? d.vhide : (const int *)d.px;
   AreaSum sum = {0, 0, 0, 0};
@@ -956,7 +967,7 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
       }
     }
   }
-  area_flush(sum, d.ch_ctr + ((size_t)((serial + 1) % 3) * SG_CH_SEG + b % SG_CH_AREA) * SG_CH_CTR);
+  area_flush(sum, d.ch_ctr + ((size_t)((ls + 1) % 3) * SG_CH_SEG + b % SG_CH_AREA) * SG_CH_CTR);
 }
 
 // Counter i (SG_CTR_*) of a chained dab: its lines summed.
@@ -975,23 +986,24 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
   extern __shared__ __align__(16) unsigned char fused_smem[];
   __shared__ int s_cnt, s_next;
   __shared__ int2 s_q[FUSED_THREADS];
-  const int serial = ca.serial;
+  const int ls = ca.ls, ss = ca.ss;
   int g0 = (int)blockIdx.x;
   if (g0 >= ca.f0) {
     const int o = g0 - ca.f0;
     if (o < ca.ns) {
-      chain_search(d, kn, serial, o, s_q, &s_cnt);
+      chain_search(d, kn, ls, ss, o, s_q, &s_cnt);
       return;
     }
     if (o < ca.ns + ca.nc) {
-      chain_copy_back(d, serial - 1, ((o - ca.ns) * FUSED_THREADS + (int)threadIdx.x) / SG_WAVE,
+      chain_copy_back(d, ls - 1, ss - 1, ((o - ca.ns) * FUSED_THREADS + (int)threadIdx.x) / SG_WAVE,
                       ca.nc * (FUSED_THREADS / SG_WAVE));
       return;
     }
-    if (o == ca.ns + ca.nc) {  // log the previous dab's counters and clear its set (dab serial + 2's)
-      long long *ctr = d.ch_ctr + (size_t)((serial + 2) % 3) * SG_CH_SEG * SG_CH_CTR;
+    if (o == ca.ns + ca.nc) {  // log the previous dab's counters and clear its set (dab ls + 2's)
+      if (ca.cont_in) return;
+      long long *ctr = d.ch_ctr + (size_t)((ls + 2) % 3) * SG_CH_SEG * SG_CH_CTR;
       if (ca.log && ca.has_prev && threadIdx.x < SG_CTR_COUNT)
-        ca.log[(size_t)(serial - 1) * SG_CTR_COUNT + threadIdx.x] = chain_counter(ctr, threadIdx.x);
+        ca.log[(size_t)(ls - 1) * SG_CTR_COUNT + threadIdx.x] = chain_counter(ctr, threadIdx.x);
       __syncthreads();
       if (threadIdx.x < SG_CH_SEG * SG_CH_CTR) ctr[threadIdx.x] = 0;
       return;
@@ -1011,22 +1023,22 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
   // after them: a load under a branch makes the compiler wait for it at the join.
   const int seg = g0 % SG_CH_SEG;
   g0 /= SG_CH_SEG;  // the workgroup's first entry of its segment
-  const int *list = d.ch_leaf + ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
-  const int4 *recs = d.ch_rec + 2 * ((size_t)(serial % 3) * SG_CH_SEG + seg) * d.ch_cap;
-  long long *lines = d.ch_ctr + (size_t)(serial % 3) * SG_CH_SEG * SG_CH_CTR;
-  long long *lines1 = d.ch_ctr + (size_t)((serial + 1) % 3) * SG_CH_SEG * SG_CH_CTR;
+  const int *list = d.ch_leaf + ((size_t)(ls % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  const int4 *recs = d.ch_rec + 2 * ((size_t)(ls % 3) * SG_CH_SEG + seg) * d.ch_cap;
+  long long *lines = d.ch_ctr + (size_t)(ls % 3) * SG_CH_SEG * SG_CH_CTR;
+  long long *lines1 = d.ch_ctr + (size_t)((ls + 1) % 3) * SG_CH_SEG * SG_CH_CTR;
   const int gc = min(g0, d.ch_cap - 1);
   const int leaf0 = list[gc];
   const int4 ra0 = recs[2 * gc], rb0 = recs[2 * gc + 1];
   const int ng = (int)lines[seg * SG_CH_CTR];
-  const int stamp = d.dstamp[0] + serial;
-  const bool undo = undo_active(d);
-  if (g0 == 0 && tid == 0) d.pend[(serial & 1) * SG_CH_SEG + seg] = ng;  // what the copy-back takes
-  const float4 *stp = d.st_pos + (size_t)((serial + 1) & 1) * d.V, *stn = d.st_nor + (size_t)((serial + 1) & 1) * d.V;
-  float4 *wtp = d.st_pos + (size_t)(serial & 1) * d.V, *wtn = d.st_nor + (size_t)(serial & 1) * d.V;
+  const int gstamp = d.dstamp[0] + ls, stamp = d.dstamp[0] + ss;
+  const bool undo = undo_active(d) && !ca.cont_in;
+  if (g0 == 0 && tid == 0) d.pend[(ls & 1) * SG_CH_SEG + seg] = ng;  // what the copy-back takes
+  const float4 *stp = d.st_pos + (size_t)((ss + 1) & 1) * d.V, *stn = d.st_nor + (size_t)((ss + 1) & 1) * d.V;
+  float4 *wtp = d.st_pos + (size_t)(ss & 1) * d.V, *wtn = d.st_nor + (size_t)(ss & 1) * d.V;
   const bool next_draw = ca.has_next && kn.tool == SG_TOOL_DRAW;
   const bool smooth = k.tool == SG_TOOL_SMOOTH;
-  const int K = smooth ? k.iters : 0;
+  const int K = smooth ? ca.iters : 0;
   // Draw offset: (normalize(area) * r) * bstrength
   float ox = 0.0f, oy = 0.0f, oz = 0.0f;
   if (k.tool == SG_TOOL_DRAW) {
@@ -1106,14 +1118,15 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     // level 3
     // stand-ins keep the loads unconditional without new traffic: a tool that needs no
     // normals, or a mesh with no mask or hidden vertices, reads the position lines again
-    const bool need_n = k.tool == SG_TOOL_INFLATE || next_draw;
+    const bool need_n = k.tool == SG_TOOL_INFLATE || next_draw, need_s = need_n || ca.cont_in;
     const float *mp = d.mask ? d.mask : d.px;
     const int *hp = hide ? d.vhide : (const int *)d.px;
     const float *nxp = need_n ? d.nx : d.px, *nyp = need_n ? d.ny : d.py, *nzp = need_n ? d.nz : d.pz;
-    const float4 *snp = need_n ? stn : stp;
-    const int *gst = d.ch_gstamp + (size_t)(serial & 1) * L;
+    const float4 *snp = need_s ? stn : stp;
+    const int *gst = d.ch_gstamp + (size_t)(ls & 1) * L;
     float x[LPT], y[LPT], z[LPT], nxv[LPT], nyv[LPT], nzv[LPT], mk[LPT];
-    bool own[LPT], hid[LPT];
+    bool own[LPT], hid[LPT], staged[LPT];
+    float sfade[LPT];
     unsigned short nb[LPT][FUSED_ROW];
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
@@ -1135,9 +1148,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       nxv[j] = st ? b.x : nxv[j];
       nyv[j] = st ? b.y : nyv[j];
       nzv[j] = st ? b.z : nzv[j];
+      staged[j] = st;
+      sfade[j] = b.w;
       mk[j] = d.mask ? m : 0.0f;
       hid[j] = hide && hv != 0;
-      own[j] = owner[j] < 0 || gs == stamp;  // its leaf was gathered by this search
+      own[j] = owner[j] < 0 || gs == gstamp;  // its leaf was gathered by this search
 #pragma unroll
       for (int q = 0; q < FUSED_ROW; q++) nb[j][q] = d.hl_nbl[nbb[j] + q < nbe[j] ? nbb[j] + q : 0];
     }
@@ -1156,7 +1171,10 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       const float d2 = dx * dx + dy * dy + dz * dz;
       aff[j] = vid[j] >= 0 && own[j] && d2 <= k.r2 && !hid[j];
       fade[j] = 0.0f;
-      if (aff[j]) {
+      if (ca.cont_in) {  // affected by the launch before, which staged its Smooth factor
+        aff[j] = vid[j] >= 0 && staged[j];
+        fade[j] = sfade[j];
+      } else if (aff[j]) {
         const float f = sg_falloff(k, curve, sqrtf(d2)) * (1.0f - mk[j]);
         if (k.tool == SG_TOOL_DRAW) {
           x[j] = x[j] + ox * f;
@@ -1228,14 +1246,30 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     // the affected uniq vertices: normal (spec S10, incident tris in vertex->tri order),
     // position, list record
     const float4 *F = S + cur * cap;  // final positions of the locals
+    if (ca.cont_out) {  // the next launch goes on from here
+#pragma unroll
+      for (int j = 0; j < LPT; j++) {
+        const int i = tid + j * FUSED_THREADS;
+        if (i >= nu || !aff[j]) continue;
+        wtp[vr.x + i] = make_float4(x[j], y[j], z[j], __int_as_float(stamp));
+        wtn[vr.x + i] = make_float4(0.0f, 0.0f, 0.0f, fade[j]);
+      }
+      __syncthreads();  // LDS is reused by the next leaf
+      continue;
+    }
     bool pass = false;
     int slot = 0;
     if (tid < FUSED_FACE_THREADS) {
       // each face normal once (spec S10's face normal; faces in the tables' order)
       auto face_normal = [&](unsigned c0, unsigned c1, int j) {
-        const float4 a = F[c0 & 0xffff], b = F[c0 >> 16], e = F[c1];
+        const float4 a = F[c0 & 0xffff], b = F[c0 >> 16], e = F[c1 & 0xffff];
         float fx, fy, fz;
-        sg_tri_normal(a.x, a.y, a.z, b.x, b.y, b.z, e.x, e.y, e.z, fx, fy, fz);
+        if ((c1 >> 16) == SG_FACE_TRI) {
+          sg_tri_normal(a.x, a.y, a.z, b.x, b.y, b.z, e.x, e.y, e.z, fx, fy, fz);
+        } else {  // a quad polygon
+          const float4 f = F[c1 >> 16];
+          sg_quad_normal(a.x, a.y, a.z, b.x, b.y, b.z, e.x, e.y, e.z, f.x, f.y, f.z, fx, fy, fz);
+        }
         Sfn[j] = make_float4(fx, fy, fz, 0.0f);
       };
 #pragma unroll
@@ -1274,11 +1308,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     }
     __syncthreads();
     if (pass) {  // (the last lane; its slot arrived during the barrier)
-      const size_t q = ((size_t)((serial + 1) % 3) * SG_CH_SEG + seg) * d.ch_cap + slot;
+      const size_t q = ((size_t)((ls + 1) % 3) * SG_CH_SEG + seg) * d.ch_cap + slot;
       d.ch_leaf[q] = leaf;
       d.ch_rec[2 * q] = ra;
       d.ch_rec[2 * q + 1] = rb;
-      d.ch_gstamp[(size_t)((serial + 1) & 1) * L + leaf] = stamp + 1;
+      d.ch_gstamp[(size_t)((ls + 1) & 1) * L + leaf] = gstamp + 1;
     }
     AreaSum area = {0, 0, 0, 0};
     const bool area_leaf = next_draw && s_next != 0;
@@ -1331,9 +1365,9 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
 // After a chain: copy its last dab's results in, hand the dab's counters (with its
 // affected count) to the counter set of its serial, and leave the other set and the
 // chain's own sets clear for what follows.
-__global__ __launch_bounds__(256) void k_dab_finish(SgDevView d, int serial) {
+__global__ __launch_bounds__(256) void k_dab_finish(SgDevView d, int serial, int ss) {
   if (d.halt && d.halt[0]) return;
-  chain_copy_back(d, serial, (blockIdx.x * blockDim.x + threadIdx.x) / SG_WAVE, gridDim.x * blockDim.x / SG_WAVE);
+  chain_copy_back(d, serial, ss, (blockIdx.x * blockDim.x + threadIdx.x) / SG_WAVE, gridDim.x * blockDim.x / SG_WAVE);
   if (blockIdx.x == 0 && threadIdx.x < SG_WAVE) {
     const CountPrefetch cp = aff_count_prefetch(d, threadIdx.x);
     long long *lines = d.ch_ctr + (size_t)(serial % 3) * SG_CH_SEG * SG_CH_CTR;
@@ -1908,31 +1942,38 @@ int sg_profile_collect(PBVH *p) {
   return 0;
 }
 
-int sg_enqueue_clear_ctr(PBVH *p, int ndabs) {
+int sg_enqueue_clear_ctr(PBVH *p, int nlaunch) {
   p->fused_pending = p->chain_live = false;  // (a failed enqueue may have left them set)
+  p->ch_ss = 0;
   hipLaunchKernelGGL(k_clear_ctr, dim3(1), dim3(128), 0, p->stream, p->d.ctr, p->d.halt, p->d.dstamp, p->d.ch_ctr,
-                     ndabs);
+                     nlaunch);
   return sg_check_hip(hipGetLastError(), "clear launch");
 }
 
 // LDS and locals per thread of the chain kernel for dab k; lpt 0 when the mesh has no
 // halo tables or the dab is not one it covers.
 struct FusedShape {
-  int cap = 0, fcap = 1, lpt = 0;
+  int cap = 0, fcap = 1, lpt = 0, launches = 1;
   size_t lds = 0;
 };
 static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
   FusedShape f;
   const bool tool = k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_GRAB ||
-                    (k.tool == SG_TOOL_SMOOTH && k.iters >= 1 && k.iters <= SG_HALO_RINGS);
+                    (k.tool == SG_TOOL_SMOOTH && k.iters >= 1);
   if (!p->d.halo_ok || !p->fused_enabled || !tool || k.stats || k.orig_co || (k.learned && p->mlp)) return f;
-  f.cap = p->d.halo_maxlocr[k.tool == SG_TOOL_SMOOTH ? k.iters : 0];
+  if (k.tool == SG_TOOL_SMOOTH) f.launches = (k.iters + SG_HALO_RINGS - 1) / SG_HALO_RINGS;
+  const int steps = k.tool == SG_TOOL_SMOOTH ? (k.iters + f.launches - 1) / f.launches : 0;  // most in one launch
+  f.cap = p->d.halo_maxlocr[steps];
   f.fcap = std::max(1, p->d.halo_maxlt);
   f.lds = (size_t)f.cap * 2 * sizeof(float4) + (size_t)f.fcap * sizeof(float4) + (size_t)(p->d.leaf_maxsh + 2) * 2 + 16;
   const int lpt = (f.cap + FUSED_THREADS - 1) / FUSED_THREADS;
   // larger halos (very large leaves) take the separate kernels
   f.lpt = lpt >= 1 && lpt <= 4 && f.lds <= 65536 - 4096 ? lpt : 0;
   return f;
+}
+// Chain launches (and a stamp of its own for the start of a chain) of one dab at most.
+int sg_dab_launches(const SgDabK &k) {
+  return 1 + (k.tool == SG_TOOL_SMOOTH ? (std::max(k.iters, 1) + SG_HALO_RINGS - 1) / SG_HALO_RINGS : 1);
 }
 
 // One dab; `serial` is the dab's position in its stroke (selects the counter set and
@@ -1980,28 +2021,36 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
     SgDabK kn = next ? *next : k;
     if (p->d.nhidden_leaves == 0) kn.hide_skip = 0;
     SgChainArgs ca;
-    ca.serial = serial;
-    ca.has_next = next && fused_shape(p, *next).lpt > 0 ? 1 : 0;
-    ca.has_prev = chained ? 1 : 0;
-    ca.last = ca.has_next ? 0 : 1;
+    const bool has_next = next && fused_shape(p, *next).lpt > 0;
+    ca.ls = serial;
     ca.nf = p->grid_fused;
     ca.f0 = std::min(ca.nf, FUSED_LEAD);
-    ca.ns = ca.has_next ? leaf_blocks : 0;
-    ca.nc = ca.has_prev ? 128 : 0;
     ca.cap = fs.cap;
     ca.fcap = fs.fcap;
     ca.log = log;
-    ProfScope ps(p, SG_K_BRUSH);
-    const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(FUSED_THREADS);
-    if (fs.lpt == 1)
-      SG_LAUNCH(ps, k_dab_chain<1>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
-    else if (fs.lpt == 2)
-      SG_LAUNCH(ps, k_dab_chain<2>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
-    else if (fs.lpt == 3)
-      SG_LAUNCH(ps, k_dab_chain<3>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
-    else
-      SG_LAUNCH(ps, k_dab_chain<4>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
-    p->chain_live = ca.has_next != 0;
+    if (!chained) p->ch_ss++;  // no launch had the stamp before this chain's first
+    for (int q = 0; q < fs.launches; q++) {
+      ca.ss = ++p->ch_ss;
+      ca.iters = k.iters / fs.launches + (q < k.iters % fs.launches ? 1 : 0);
+      ca.cont_in = q > 0 ? 1 : 0;
+      ca.cont_out = q + 1 < fs.launches ? 1 : 0;
+      ca.has_next = has_next && !ca.cont_out ? 1 : 0;
+      ca.has_prev = chained && !ca.cont_in ? 1 : 0;
+      ca.last = !has_next && !ca.cont_out ? 1 : 0;
+      ca.ns = ca.has_next ? leaf_blocks : 0;
+      ca.nc = ca.has_prev ? 128 : 0;
+      ProfScope ps(p, SG_K_BRUSH);
+      const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(FUSED_THREADS);
+      if (fs.lpt == 1)
+        SG_LAUNCH(ps, k_dab_chain<1>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+      else if (fs.lpt == 2)
+        SG_LAUNCH(ps, k_dab_chain<2>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+      else if (fs.lpt == 3)
+        SG_LAUNCH(ps, k_dab_chain<3>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+      else
+        SG_LAUNCH(ps, k_dab_chain<4>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca);
+    }
+    p->chain_live = has_next;
     p->fused_pending = true;
     return sg_check_hip(hipGetLastError(), "dab launch");
   }
@@ -2147,7 +2196,7 @@ int sg_enqueue_finish(PBVH *p, int serial_last) {
   SgDevView v = sg_view(p);
   v.ctr = p->d.ctr + (size_t)(serial_last & 1) * SG_CTR_COUNT;  // the last dab's counter set
   v.ctr_next = p->d.ctr + (size_t)((serial_last + 1) & 1) * SG_CTR_COUNT;
-  hipLaunchKernelGGL(k_dab_finish, dim3(128), dim3(256), 0, p->stream, v, serial_last);
+  hipLaunchKernelGGL(k_dab_finish, dim3(128), dim3(256), 0, p->stream, v, serial_last, p->ch_ss);
   return sg_check_hip(hipGetLastError(), "finish launch");
 }
 

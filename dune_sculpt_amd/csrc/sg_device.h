@@ -54,6 +54,18 @@ __device__ __forceinline__ void sg_tri_normal(float ax, float ay, float az, floa
   sg_normalize(nx, ny, nz);
 }
 
+// normal_quad_v3 (math_geom.cc:48-68): the cross product of the diagonals
+__device__ __forceinline__ void sg_quad_normal(float ax, float ay, float az, float bx, float by, float bz, float cx,
+                                               float cy, float cz, float dx, float dy, float dz, float &nx, float &ny,
+                                               float &nz) {
+  const float n10 = ax - cx, n11 = ay - cy, n12 = az - cz;
+  const float n20 = bx - dx, n21 = by - dy, n22 = bz - dz;
+  nx = n11 * n22 - n12 * n21;
+  ny = n12 * n20 - n10 * n22;
+  nz = n10 * n21 - n11 * n20;
+  sg_normalize(nx, ny, nz);
+}
+
 // BKE_mesh_calc_poly_normal (mesh_evaluate.c:62-84) of polygon q, corners read from
 // the position arrays (x, y, z): more than 4 corners Newell's method from the last
 // corner (mesh_calc_ngon_normal :39-60, add_newell_cross_v3_v3v3
@@ -80,12 +92,8 @@ __device__ __forceinline__ void sg_poly_normal(const int *__restrict__ poly_off,
     if (n == 3) {
       sg_tri_normal(P[0][0], P[0][1], P[0][2], P[1][0], P[1][1], P[1][2], P[2][0], P[2][1], P[2][2], nx, ny, nz);
     } else {
-      const float n10 = P[0][0] - P[2][0], n11 = P[0][1] - P[2][1], n12 = P[0][2] - P[2][2];
-      const float n20 = P[1][0] - P[3][0], n21 = P[1][1] - P[3][1], n22 = P[1][2] - P[3][2];
-      nx = n11 * n22 - n12 * n21;
-      ny = n12 * n20 - n10 * n22;
-      nz = n10 * n21 - n11 * n20;
-      sg_normalize(nx, ny, nz);
+      sg_quad_normal(P[0][0], P[0][1], P[0][2], P[1][0], P[1][1], P[1][2], P[2][0], P[2][1], P[2][2], P[3][0],
+                     P[3][1], P[3][2], nx, ny, nz);
     }
   } else if (n > 4) {
     nx = ny = nz = 0.0f;

@@ -13,7 +13,8 @@
 #define SG_CH_CTR 8   // counters of a segment (a 64-byte line): SG_CTR_NGATHER .. SG_CTR_AREA_Z, then SG_CH_NAREA
 #define SG_CH_NAREA 5
 #define SG_CH_AREA 4   // segments whose lines take area-normal sums
-#define SG_HALO_RINGS 4  // Smooth(k) runs fused for k <= this
+#define SG_HALO_RINGS 4  // Jacobi steps of Smooth one launch of the fused dab covers
+#define SG_FACE_TRI 0xffffu  // fourth corner of a triangle in the halo's face table (local ids are below)
 
 // Cut of the tree used by the two-level sphere search: maximal subtrees holding at
 // most cut_leaf_cap leaves.  Leaves are numbered in DFS (left->right) order, so every
@@ -281,6 +282,7 @@ struct PBVH {
   bool fused_enabled = true;
   bool fused_pending = false;        // the last dab enqueued was fused and no finish followed yet
   bool chain_live = false;           // ... and its launch searches for the next one
+  int ch_ss = 0;                     // chain launches enqueued since the counters were cleared (and a gap per chain)
   // device snapshot (checkpoint) of the mutable mesh state
   // slot 0: the caller's (sg_pbvh_snapshot_save/restore); slot 1: internal (autotuner, judge)
   std::vector<void *> snap[2];

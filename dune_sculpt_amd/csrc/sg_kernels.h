@@ -117,7 +117,8 @@ SgDabK sg_make_dab(const SgDabParams *dab, int stats);
 int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index,
                    int stamp, int serial, const SgCollect *col = nullptr, const float *place = nullptr,
                    const SgDabK *next = nullptr);
-int sg_enqueue_clear_ctr(PBVH *p, int ndabs);
+int sg_dab_launches(const SgDabK &k);
+int sg_enqueue_clear_ctr(PBVH *p, int nlaunch);
 int sg_enqueue_flush(PBVH *p);
 int sg_enqueue_log_row(PBVH *p, long long *log, int row);
 int sg_enqueue_full_normals(PBVH *p);

@@ -80,6 +80,61 @@ def test_area_normal_of_jumping_radii(sg, factor):
     _check(sg, co, tris, _path(sg, 24, 7, radii, (1,), normal_radius_factor=factor), leaf=32)
 
 
+@pytest.mark.parametrize("k", [5, 6, 7, 8, 9, 13, 64])
+def test_smooth_over_several_launches(sg, k):
+    """More steps than one launch covers, beside other tools, with a mask."""
+    co, tris = sg.noisy_icosphere(5, seed=10, amplitude=0.02)
+    mask = np.clip(0.5 - co[:, 1], 0, 1).astype(np.float32)
+    _check(sg, co, tris, _path(sg, 9, 3, np.full(9, 0.25), (2, 1, 2, 2, 5), (k,)), mask=mask)
+    _check(sg, co, tris, _path(sg, 1, 3, [0.4], (2,), (k,)), graph=False)
+
+
+def _quad_torus(sg, nu, nv, mixed):
+    """Quads of a torus; with `mixed` every third one split into two triangles."""
+    co, _ = sg.noisy_torus(nu, nv, seed=3, amplitude=0.02)
+    i, j = np.meshgrid(np.arange(nu), np.arange(nv), indexing="ij")
+    q = np.stack([i * nv + j, (i + 1) % nu * nv + j, (i + 1) % nu * nv + (j + 1) % nv, i * nv + (j + 1) % nv], -1)
+    faces = []
+    for n, f in enumerate(q.reshape(-1, 4).tolist()):
+        faces += [f[:3], [f[0], f[2], f[3]]] if mixed and n % 3 == 0 else [f]
+    off = np.concatenate([[0], np.cumsum([len(f) for f in faces])]).astype(np.int32)
+    return co, (off, np.concatenate(faces).astype(np.int32), np.ones(len(faces), np.uint8),
+                np.zeros(len(faces), np.int16))
+
+
+@pytest.mark.parametrize("nu,nv,leaf,mixed", [(40, 13, 64, False), (40, 13, 64, True), (9, 9, 128, True),
+                                              (101, 31, 17, False)])
+def test_quads(sg, nu, nv, leaf, mixed):
+    co, polys = _quad_torus(sg, nu, nv, mixed)
+    rng = np.random.default_rng(4)
+    dabs = [sg.make_dab(tool=(1, 4, 2, 5)[i % 4], location=co[rng.integers(len(co))], radius=float(rng.uniform(0.1, 0.5)),
+                        strength=0.6, smooth_iterations=1 + i % 6, grab_delta=rng.normal(size=3) * 0.02)
+            for i in range(20)]
+    got = []
+    for fused in (True, False):
+        p = sg.PBVH(co, None, leaf_limit=leaf, polys=polys)
+        assert p.set_fused(fused), "triangles and quads have halo tables"
+        p.stroke(dabs, log=True)
+        got.append([*_state(p), p.last_affected(), p.last_gathered(), p.stroke_log(20)[:, :5]])
+        p.close()
+    for x, y in zip(*got):
+        assert x.tobytes() == y.tobytes()
+
+
+def test_ngons_keep_the_separate_kernels(sg):
+    """A pentagon's corners do not fit a face record: no halo tables, the dab still runs."""
+    t = np.linspace(0, 2 * np.pi, 6)[:5]
+    co = np.concatenate([np.stack([np.cos(t), np.sin(t), 0 * t], -1), [[0, 0, 1]]]).astype(np.float32)
+    faces = [[4, 3, 2, 1, 0]] + [[i, (i + 1) % 5, 5] for i in range(5)]
+    off = np.concatenate([[0], np.cumsum([len(f) for f in faces])]).astype(np.int32)
+    p = sg.PBVH(co, None, polys=(off, np.concatenate(faces).astype(np.int32), np.zeros(6, np.uint8),
+                                 np.zeros(6, np.int16)))
+    assert not p.set_fused(True)
+    p.stroke([sg.make_dab(tool=1, location=(0, 0, 1), radius=0.8)] * 2)
+    assert p.positions()[5, 2] > 1.0
+    p.close()
+
+
 def test_hidden_masked_refit_each(sg):
     co, tris = sg.noisy_icosphere(5, seed=8, amplitude=0.02)
     hidden = co[:, 2] > 0.55
