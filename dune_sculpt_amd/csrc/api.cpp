@@ -12,6 +12,7 @@
 #include "sg_grids.h"
 #include "sg_dyn.h"
 #include "sg_kernels.h"
+#include "sg_xfer.h"
 #include "sg_learned.h"
 
 namespace {
@@ -486,8 +487,9 @@ static int snap_save(PBVH *p, int slot) {
       if (sg_check_hip(hipMalloc(&sn[i], std::max<size_t>(items[i].bytes, 4)), "hipMalloc")) return -1;
   }
   if (p->nodes_dirty_deferred) sg_enqueue_flush(p);
-  for (size_t i = 0; i < items.size(); i++)
-    hipMemcpyAsync(sn[i], items[i].dev, items[i].bytes, hipMemcpyDeviceToDevice, p->stream);
+  std::vector<SgCopy> cp;
+  for (size_t i = 0; i < items.size(); i++) cp.push_back({sn[i], items[i].dev, items[i].bytes});
+  if (int rc = sg_enqueue_copies(p->stream, cp.data(), (int)cp.size())) return rc;
   p->snap_valid[slot] = true;
   return sg_check_hip(hipStreamSynchronize(p->stream), "snapshot");
 }
@@ -495,8 +497,9 @@ static int snap_save(PBVH *p, int slot) {
 static int snap_restore(PBVH *p, int slot) {
   if (!p || !p->snap_valid[slot]) return sg_set_error("no snapshot");
   auto items = snap_items(p);
-  for (size_t i = 0; i < items.size(); i++)
-    hipMemcpyAsync(items[i].dev, p->snap[slot][i], items[i].bytes, hipMemcpyDeviceToDevice, p->stream);
+  std::vector<SgCopy> cp;
+  for (size_t i = 0; i < items.size(); i++) cp.push_back({items[i].dev, p->snap[slot][i], items[i].bytes});
+  if (int rc = sg_enqueue_copies(p->stream, cp.data(), (int)cp.size())) return rc;
   invalidate_host_views(p);
   return sg_check_hip(hipStreamSynchronize(p->stream), "restore");
 }

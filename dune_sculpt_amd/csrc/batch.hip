@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "sg_batch.h"
+#include "sg_xfer.h"
 #include "sg_device.h"
 #include "sg_learned.h"
 
@@ -1067,8 +1068,9 @@ int sg_batch_snapshot_save(SgBatch *b) {
     for (size_t i = 0; i < items.size(); i++)
       if (sg_check_hip(hipMalloc(&b->snap[i], std::max<size_t>(items[i].bytes, 4)), "hipMalloc")) return -1;
   }
-  for (size_t i = 0; i < items.size(); i++)
-    hipMemcpyAsync(b->snap[i], items[i].dev, items[i].bytes, hipMemcpyDeviceToDevice, b->stream);
+  std::vector<SgCopy> cp;
+  for (size_t i = 0; i < items.size(); i++) cp.push_back({b->snap[i], items[i].dev, items[i].bytes});
+  if (int rc = sg_enqueue_copies(b->stream, cp.data(), (int)cp.size())) return rc;
   b->snap_valid = true;
   return sg_check_hip(hipStreamSynchronize(b->stream), "snapshot");
 }
@@ -1077,8 +1079,9 @@ int sg_batch_snapshot_restore(SgBatch *b) {
   if (batch_check(b)) return -1;
   if (!b->snap_valid) return sg_set_error("no batch snapshot");
   auto items = batch_snap_items(b);
-  for (size_t i = 0; i < items.size(); i++)
-    hipMemcpyAsync(items[i].dev, b->snap[i], items[i].bytes, hipMemcpyDeviceToDevice, b->stream);
+  std::vector<SgCopy> cp;
+  for (size_t i = 0; i < items.size(); i++) cp.push_back({items[i].dev, b->snap[i], items[i].bytes});
+  if (int rc = sg_enqueue_copies(b->stream, cp.data(), (int)cp.size())) return rc;
   return sg_check_hip(hipStreamSynchronize(b->stream), "restore");
 }
 

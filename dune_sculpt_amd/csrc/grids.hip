@@ -27,6 +27,7 @@
 
 #include "sg_device.h"
 #include "sg_grids.h"
+#include "sg_xfer.h"
 
 #define GR_THREADS 256
 #define GR_CHUNK 256  // elements per work item (1 per thread)
@@ -1206,30 +1207,24 @@ int sg_grids_snapshot(PBVH *p, int restore) {
                {d.mask, d.mask ? E * 4 : 0}, {d.leaf_bb, (size_t)d.L * 32}, {d.leaf_obb, (size_t)d.L * 32},
                {d.node_bb, (size_t)d.N * 32}, {d.node_obb, (size_t)d.N * 32}};
   const int np = sizeof(parts) / sizeof(parts[0]);
+  auto padded = [](size_t n) { return (n + 255) & ~(size_t)255; };  // every array's part starts aligned
   if (!restore && !d.snap) {
     size_t tot = 0;
-    for (const Part &q : parts) tot += q.bytes;
+    for (const Part &q : parts) tot += padded(q.bytes);
     if (sg_check_hip(hipMalloc(&d.snap, tot), "hipMalloc")) return -1;
   }
   if (!d.snap) return sg_set_error("no grids snapshot saved");
+  std::vector<SgCopy> cp;
   size_t off = 0;
   for (int i = 0; i < np; i++) {
-    if (!parts[i].bytes) continue;
     unsigned char *s = (unsigned char *)d.snap + off;
-    if (restore) {
-      if (sg_check_hip(hipMemcpyAsync(parts[i].dev, s, parts[i].bytes, hipMemcpyDeviceToDevice, p->stream), "copy"))
-        return -1;
-    } else {
-      if (sg_check_hip(hipMemcpyAsync(s, parts[i].dev, parts[i].bytes, hipMemcpyDeviceToDevice, p->stream), "copy"))
-        return -1;
-    }
-    off += parts[i].bytes;
+    cp.push_back(restore ? SgCopy{parts[i].dev, s, parts[i].bytes} : SgCopy{s, parts[i].dev, parts[i].bytes});
+    off += padded(parts[i].bytes);
   }
   if (restore) {  // the shadow copy equals the positions between dabs
-    const float *src[3] = {d.px, d.py, d.pz};
     float *dst[3] = {d.qx, d.qy, d.qz};
-    for (int i = 0; i < 3; i++)
-      if (sg_check_hip(hipMemcpyAsync(dst[i], src[i], E * 4, hipMemcpyDeviceToDevice, p->stream), "copy")) return -1;
+    for (int i = 0; i < 3; i++) cp.push_back({dst[i], cp[i].src, E * 4});
   }
+  if (int rc = sg_enqueue_copies(p->stream, cp.data(), (int)cp.size())) return rc;
   return sg_check_hip(hipStreamSynchronize(p->stream), "snapshot");
 }
