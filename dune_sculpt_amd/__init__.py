@@ -946,9 +946,10 @@ class PBVH:
         """Rays (n x 3 starts, n x 3 directions, optional initial depths) -> structured
         array of hits (sg_raycast)."""
         rays = make_rays(starts, normals, depths)
-        hits = (SgRayHit * len(rays))()
-        _check(lib().sg_raycast(self.h, rays, len(rays), 1 if original else 0, hits), "sg_raycast")
-        return hits_to_numpy(hits)
+        hits = np.empty(len(rays), RAY_HIT_DTYPE)
+        out = C.cast(hits.ctypes.data, C.POINTER(SgRayHit))
+        _check(lib().sg_raycast(self.h, rays, len(rays), 1 if original else 0, out), "sg_raycast")
+        return hits
 
     def raycast_stats(self, starts, normals, depths=None, original=False):
         """Work counters of a ray batch: boxes tested, leaves scanned, tris tested."""

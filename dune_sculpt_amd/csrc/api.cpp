@@ -114,8 +114,7 @@ int read_aos(PBVH *p, int which, float *out) {
   float *tmp = (float *)stage(p, n * sizeof(float));
   if (!tmp) return -1;
   int rc = sg_enqueue_gather(p, which, tmp);
-  if (!rc) rc = sg_check_hip(hipMemcpyAsync(out, tmp, n * sizeof(float), hipMemcpyDeviceToHost, p->stream), "copy");
-  if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "sync");
+  if (!rc) rc = sg_read_back(p->stream, p->pin, tmp, out, n * sizeof(float), "read");
   return rc;
 }
 
@@ -203,6 +202,11 @@ PBVH *BKE_pbvh_new(void) {
     delete p;
     return nullptr;
   }
+  if (sg_check_hip(hipHostMalloc((void **)&p->mail, SG_MAIL_BYTES, hipHostMallocDefault), "hipHostMalloc")) {
+    (void)hipStreamDestroy(p->stream);
+    delete p;
+    return nullptr;
+  }
   return p;
 }
 
@@ -229,6 +233,8 @@ void BKE_pbvh_free(PBVH *p) {
   free(p->looptri);
   for (int i = 0; i < 2; i++)
     if (p->timer[i]) hipEventDestroy(p->timer[i]);
+  sg_pinned_free(p->pin);
+  if (p->mail) (void)hipHostFree(p->mail);
   if (!p->no_device) hipStreamDestroy(p->stream);
   delete p;
 }
@@ -538,13 +544,12 @@ int sg_dab_apply(PBVH *p, const SgDabParams *dab) {
   int rc = sg_enqueue_clear_ctr(p, sg_dab_launches(k));
   if (!rc) rc = sg_enqueue_dab(p, k, curve, nullptr, 0, stamp, 0);
   if (!rc) rc = sg_enqueue_finish(p, 0);
-  if (!rc) rc = sg_enqueue_flush(p);
-  long long ctr[SG_CTR_COUNT];
-  int halt = 0;
-  if (!rc) rc = sg_check_hip(hipMemcpyAsync(ctr, p->d.ctr, sizeof(ctr), hipMemcpyDeviceToHost, p->stream), "copy");
-  if (!rc) rc = sg_check_hip(hipMemcpyAsync(&halt, p->d.halt, 4, hipMemcpyDeviceToHost, p->stream), "copy");
+  if (!rc) rc = sg_enqueue_flush(p, p->d.ctr);
   if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "dab");
   if (rc) return rc;
+  long long ctr[SG_CTR_COUNT];
+  memcpy(ctr, p->mail, sizeof(ctr));
+  const bool halt = p->mail[SG_CTR_COUNT] != 0;
   if (k.learned && p->mlp) {
     if (halt) {  // rejected: the plain brush does this dab
       p->learned_fallbacks++;
@@ -641,15 +646,17 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
   if (ncustom && ensure_curves(p, ncustom)) return -1;
   if (log && ensure_log(p, n)) return -1;
   if (g_stats && !ensure_stats_buffers(p)) return -1;
-  {
-    int ci = 0;
-    for (int i = 0; i < n; i++) {
-      if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table) {
-        hipMemcpyAsync(p->d.curve + (size_t)ci * (SG_CM_TABLE + 1), dabs[i].curve_table,
-                       (SG_CM_TABLE + 1) * sizeof(float), hipMemcpyHostToDevice, p->stream);
-        ci++;
-      }
-    }
+  if (ncustom) {  // every curve in one copy
+    std::vector<float> curves;
+    curves.reserve((size_t)ncustom * (SG_CM_TABLE + 1));
+    for (int i = 0; i < n; i++)
+      if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
+        curves.insert(curves.end(), dabs[i].curve_table, dabs[i].curve_table + SG_CM_TABLE + 1);
+    if (sg_check_hip(hipMemcpyAsync(p->d.curve, curves.data(), curves.size() * sizeof(float), hipMemcpyHostToDevice,
+                                    p->stream),
+                     "copy") ||
+        sg_check_hip(hipStreamSynchronize(p->stream), "copy"))
+      return -1;
   }
   // Dabs [a, n) as one segment (serials restart at 0); returns the position of a
   // rejected learned dab (halt) or -1.
@@ -681,7 +688,7 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
         if (flush_each && sg_enqueue_flush(p)) return -1;
       }
       if (sg_enqueue_finish(p, n - 1 - a0)) return -1;
-      if (!flush_each && sg_enqueue_flush(p)) return -1;
+      if (!flush_each && sg_enqueue_flush(p, p->d.ctr + (size_t)((n - 1 - a0) & 1) * SG_CTR_COUNT)) return -1;
       if (log && sg_enqueue_log_row(p, p->d.log, n - 1 - a0)) return -1;
       return 0;
     };
@@ -707,7 +714,10 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
       if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "stroke");
     }
     int h = 0;
-    if (!rc) rc = sg_check_hip(hipMemcpy(&h, p->d.halt, 4, hipMemcpyDeviceToHost), "copy");
+    if (!flush_each)  // the last refit mailed it
+      h = rc ? 0 : (int)p->mail[SG_CTR_COUNT];
+    else if (!rc)
+      rc = sg_check_hip(hipMemcpy(&h, p->d.halt, 4, hipMemcpyDeviceToHost), "copy");
     *halted = h ? a0 + h - 1 : -1;
     return rc;
   };
@@ -734,9 +744,11 @@ static int stroke_apply(PBVH *p, const SgDabParams *dabs, const SgRay *rays, int
   p->learned_fallbacks += nfallback;
   p->learned_accepted += nlearned - nfallback;
   if (a0 < n) {  // otherwise the last dab was a plain fallback and set last_ctr itself
-    long long ctr[SG_CTR_COUNT];
-    hipMemcpy(ctr, p->d.ctr + (size_t)((n - 1 - a0) & 1) * SG_CTR_COUNT, sizeof(ctr), hipMemcpyDeviceToHost);
-    memcpy(p->last_ctr, ctr, sizeof(ctr));
+    if (!flush_each)
+      memcpy(p->last_ctr, p->mail, SG_CTR_COUNT * sizeof(long long));
+    else
+      hipMemcpy(p->last_ctr, p->d.ctr + (size_t)((n - 1 - a0) & 1) * SG_CTR_COUNT, SG_CTR_COUNT * sizeof(long long),
+                hipMemcpyDeviceToHost);
     p->last_learned = p->mlp && dabs[n - 1].sculpt_tool == SG_TOOL_SMOOTH && (dabs[n - 1].flag & SG_SMOOTH_LEARNED);
     p->last_tool = dabs[n - 1].sculpt_tool;
   }
@@ -924,7 +936,7 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
       if (!erc && flush_each) erc = sg_enqueue_flush(p);
     }
     if (!erc) erc = sg_enqueue_finish(p, n - 1);
-    if (!erc && !flush_each) erc = sg_enqueue_flush(p);
+    if (!erc && !flush_each) erc = sg_enqueue_flush(p, p->d.ctr + (size_t)((n - 1) & 1) * SG_CTR_COUNT);
     if (!erc && log) erc = sg_enqueue_log_row(p, p->d.log, n - 1);
     const hipError_t e = hipStreamEndCapture(p->stream, &s->graph);
     rc = erc ? erc : sg_check_hip(e, "end capture");
@@ -965,8 +977,8 @@ int sg_stroke_launch(SgStroke *s, int sync) {
   int rc = sg_check_hip(hipGraphLaunch(s->exec, p->stream), "graph launch");
   if (!rc && (sync || s->learned)) rc = sg_check_hip(hipStreamSynchronize(p->stream), "stroke");
   if (!rc && s->learned) {
-    int h = 0;
-    rc = sg_check_hip(hipMemcpy(&h, p->d.halt, 4, hipMemcpyDeviceToHost), "copy");
+    int h = (int)p->mail[SG_CTR_COUNT];
+    if (s->flags & 2) rc = sg_check_hip(hipMemcpy(&h, p->d.halt, 4, hipMemcpyDeviceToHost), "copy");
     const int ran = h ? h - 1 : s->n;  // dabs the graph completed
     if (p->mlp)
       for (int i = 0; i < ran; i++)
@@ -994,9 +1006,12 @@ int sg_stroke_launch(SgStroke *s, int sync) {
   }
   if (!rc && (sync || s->learned)) {  // the stream is idle: record the last dab's counters
     const SgDabParams &last = s->dabs[s->n - 1];
-    rc = sg_check_hip(hipMemcpy(p->last_ctr, p->d.ctr + (size_t)((s->n - 1) & 1) * SG_CTR_COUNT,
-                                SG_CTR_COUNT * sizeof(long long), hipMemcpyDeviceToHost),
-                      "copy");
+    if (!(s->flags & 2))  // its last refit mailed them
+      memcpy(p->last_ctr, p->mail, SG_CTR_COUNT * sizeof(long long));
+    else
+      rc = sg_check_hip(hipMemcpy(p->last_ctr, p->d.ctr + (size_t)((s->n - 1) & 1) * SG_CTR_COUNT,
+                                  SG_CTR_COUNT * sizeof(long long), hipMemcpyDeviceToHost),
+                        "copy");
     p->last_tool = last.sculpt_tool;
     p->last_learned = s->learned && last.sculpt_tool == SG_TOOL_SMOOTH && (last.flag & SG_SMOOTH_LEARNED);
   }

@@ -872,6 +872,7 @@ void sg_batch_free(SgBatch *b) {
   for (int i = 0; i < 2; i++)
     if (b->timer[i]) hipEventDestroy(b->timer[i]);
   batch_free_device(b);
+  sg_pinned_free(b->pin);
   hipStreamDestroy(b->stream);
   delete b;
 }
@@ -1051,9 +1052,7 @@ static int batch_read(SgBatch *b, int mesh, int which, float *out) {
   const SgDev &d = b->d;
   const float *x = which ? d.nx : d.px, *y = which ? d.ny : d.py, *z = which ? d.nz : d.pz;
   int rc = sg_enqueue_gather_raw(b->stream, x + vb, y + vb, z + vb, d.vperm_old + vb, V, b->gather_buf);
-  if (!rc) rc = sg_check_hip(hipMemcpyAsync(out, b->gather_buf, (size_t)V * 12, hipMemcpyDeviceToHost, b->stream),
-                             "copy");
-  if (!rc) rc = sg_check_hip(hipStreamSynchronize(b->stream), "read");
+  if (!rc) rc = sg_read_back(b->stream, b->pin, b->gather_buf, out, (size_t)V * 12, "read");
   return rc;
 }
 

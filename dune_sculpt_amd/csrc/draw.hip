@@ -448,7 +448,7 @@ int sg_pbvh_draw_buffers_update(PBVH *p, int all) {
   hipLaunchKernelGGL(k_draw_fill, dim3(std::max(1, std::min((L + DRAW_WAVES - 1) / DRAW_WAVES, 8192))),
                      dim3(64 * DRAW_WAVES), 0, p->stream, sg_view(p), draw_view(p), L, all ? 1 : 0);
   rc = sg_check_hip(hipGetLastError(), "draw fill launch");
-  if (!rc) rc = sg_check_hip(hipMemsetAsync(p->d.draw_dirty, 0, (size_t)p->d.C * sizeof(int), p->stream), "memset");
+  if (!rc) rc = sg_enqueue_zero(p->stream, p->d.draw_dirty, p->d.C);
   if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "draw update");
   if (dl) (void)hipFree(dl);
   return rc;

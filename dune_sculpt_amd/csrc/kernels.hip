@@ -1455,7 +1455,8 @@ __global__ __launch_bounds__(FLUSH_THREADS) void k_flush_sub(SgDevView d, int ma
   }
 }
 
-__global__ __launch_bounds__(1024) void k_flush_top(SgDevView d, int top_n, int clear) {
+__global__ __launch_bounds__(1024) void k_flush_top(SgDevView d, int top_n, int clear, const long long *ctr,
+                                                    const int *halt, long long *mail) {
   extern __shared__ float s_bb[];  // [(C + top_n) * 6]
   __shared__ int s_hs[FLUSH_MAXH + 1];
   const int C = d.C;
@@ -1491,6 +1492,10 @@ __global__ __launch_bounds__(1024) void k_flush_top(SgDevView d, int top_n, int 
   }
   if (clear) {
     for (int i = threadIdx.x; i < C; i += blockDim.x) d.cut_dirty[i] = 0;
+  }
+  if (ctr) {  // the last dab's counters and the halt flag for the host (pinned memory: no copies after the wait)
+    if (threadIdx.x < SG_CTR_COUNT) mail[threadIdx.x] = ctr[threadIdx.x];
+    if (threadIdx.x == SG_CTR_COUNT) mail[SG_CTR_COUNT] = halt[0];
   }
 }
 
@@ -2080,7 +2085,8 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
     {
       ProfScope ps(p, SG_K_FLUSH_TOP);
       const size_t top_lds = (size_t)(p->d.C + p->d.top_n) * 6 * sizeof(float);
-      SG_LAUNCH(ps, k_flush_top, dim3(1), dim3(1024), top_lds, s, v, p->d.top_n, 1);
+      SG_LAUNCH(ps, k_flush_top, dim3(1), dim3(1024), top_lds, s, v, p->d.top_n, 1, (const long long *)nullptr,
+                (const int *)nullptr, (long long *)nullptr);
     }
     return sg_check_hip(hipGetLastError(), "dab launch");
   }
@@ -2131,7 +2137,7 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
   return sg_check_hip(hipGetLastError(), "dab launch");
 }
 
-int sg_enqueue_flush(PBVH *p) {
+int sg_enqueue_flush(PBVH *p, const long long *ctr) {
   const SgDevView v = sg_view(p);
   hipStream_t s = p->stream;
   const size_t sub_lds = (size_t)p->d.sub_maxn * 6 * sizeof(float);
@@ -2142,7 +2148,7 @@ int sg_enqueue_flush(PBVH *p) {
   const size_t top_lds = (size_t)(p->d.C + p->d.top_n) * 6 * sizeof(float);
   {
     ProfScope ps(p, SG_K_FLUSH_TOP);
-    SG_LAUNCH(ps, k_flush_top, dim3(1), dim3(1024), top_lds, s, v, p->d.top_n, 1);
+    SG_LAUNCH(ps, k_flush_top, dim3(1), dim3(1024), top_lds, s, v, p->d.top_n, 1, ctr, (const int *)p->d.halt, p->mail);
   }
   return sg_check_hip(hipGetLastError(), "flush launch");
 }

