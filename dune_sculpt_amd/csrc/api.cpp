@@ -785,6 +785,7 @@ int sg_dab_apply_stroke(PBVH *p, const SgDabParams *dabs, int n, int flags) {
     if (ncustom && sg_check_hip(hipMalloc(&curves, (size_t)ncustom * (SG_CM_TABLE + 1) * sizeof(float)), "hipMalloc"))
       return -1;
     int rc = 0, ci = 0;
+    p->gd->searched = false;  // (a stroke that failed midway may have left it)
     for (int i = 0; i < n && !rc; i++) {
       const float *curve = nullptr;
       if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table) {
@@ -794,7 +795,11 @@ int sg_dab_apply_stroke(PBVH *p, const SgDabParams *dabs, int n, int flags) {
                           "copy");
         curve = c;
       }
-      if (!rc) rc = sg_grids_enqueue_dab(p, sg_make_dab(&dabs[i], 0), curve, log ? p->d.log : nullptr, i);
+      if (!rc) {
+        const SgDabK kn = sg_make_dab(&dabs[i + 1 < n ? i + 1 : i], 0);
+        rc = sg_grids_enqueue_dab(p, sg_make_dab(&dabs[i], 0), curve, log ? p->d.log : nullptr, i,
+                                  i + 1 < n ? &kn : nullptr);
+      }
     }
     if (!rc) rc = sg_grids_enqueue_flush(p);
     if (!rc) rc = sg_grids_fetch_last(p);  // waits for the stream
@@ -904,11 +909,14 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
   int erc = 0;
   if (!rc && p->type == PBVH_GRIDS) {  // each grid dab is self-contained (counters, normals, refit)
     int ci = 0;
+    p->gd->searched = false;
     for (int i = 0; i < n && !erc; i++) {
       const float *curve = nullptr;
       if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
         curve = s->curves + (size_t)(ci++) * (SG_CM_TABLE + 1);
-      erc = sg_grids_enqueue_dab(p, sg_make_dab(&dabs[i], 0), curve, log ? p->d.log : nullptr, i);
+      const SgDabK kn = sg_make_dab(&dabs[i + 1 < n ? i + 1 : i], 0);
+      erc = sg_grids_enqueue_dab(p, sg_make_dab(&dabs[i], 0), curve, log ? p->d.log : nullptr, i,
+                                 i + 1 < n ? &kn : nullptr);
     }
     if (!erc) erc = sg_grids_enqueue_flush(p);
     const hipError_t e = hipStreamEndCapture(p->stream, &s->graph);

@@ -56,6 +56,11 @@ struct GView {  // kernel view of SgGridDev (by value)
   long long *ctr, *ctr_last;
   int *dser;  // [0] the running operation's serial, [1] the last dab's
   int *leaf_dirty, *node_dirty;  // refit since the last internal-node flush
+  int *leaf_gmark;               // serial of the last dab that gathered the leaf
+  const int4 *face_leaf;
+  const int2 *grid_pl;
+  long long *lines;
+  int maxn;
 };
 
 GView view_of(const SgGridDev &d) {
@@ -120,6 +125,11 @@ GView view_of(const SgGridDev &d) {
   v.dser = d.dser;
   v.leaf_dirty = d.leaf_dirty;
   v.node_dirty = d.node_dirty;
+  v.leaf_gmark = d.leaf_gmark;
+  v.face_leaf = d.face_leaf;
+  v.grid_pl = d.grid_pl;
+  v.lines = d.lines;
+  v.maxn = d.maxn;
   return v;
 }
 
@@ -154,6 +164,7 @@ __global__ __launch_bounds__(GR_THREADS) void kg_search(GView g, SgDabK k) {
   if (pass) {
     g.gathered[base + mask_prefix(m)] = l;
     g.leaf_mark[l] = serial;
+    g.leaf_gmark[l] = serial;
   }
 }
 
@@ -268,6 +279,45 @@ __global__ __launch_bounds__(GR_THREADS) void kg_brush(GView g, SgDabK k, const 
   if (lane_id() == 0 && naff) atomicAdd((unsigned long long *)&g.ctr[SGG_NAFF], (unsigned long long)naff);
 }
 
+// One Jacobi step of spec S8 for element v.
+__device__ __forceinline__ void smooth_element(const GView &g, int v, const float *sx, const float *sy, const float *sz,
+                                               float fade, float *dx, float *dy, float *dz) {
+  const int local = v % g.ga, y = local / g.gs, x = local - y * g.gs;
+  const float px = sx[v], py = sy[v], pz = sz[v];
+  float ax = 0.0f, ay = 0.0f, az = 0.0f;
+  int cnt;
+  if (x > 0 && y > 0 && x < g.gs - 1 && y < g.gs - 1) {
+    // inside the grid: previous row, next row, previous column, next column
+    // (neighbor_coords_inner_get, subdiv_ccg.c:1870-1880)
+    const int u[4] = {v - g.gs, v + g.gs, v - 1, v + 1};
+    for (int q = 0; q < 4; q++) {
+      ax = ax + sx[u[q]];
+      ay = ay + sy[u[q]];
+      az = az + sz[u[q]];
+    }
+    cnt = 4;
+  } else {
+    const long long nb = g.nb_off[v], ne = g.nb_off[v + 1];
+    for (long long q = nb; q < ne; q++) {
+      const int u = g.nb_idx[q];
+      ax = ax + sx[u];
+      ay = ay + sy[u];
+      az = az + sz[u];
+    }
+    cnt = (int)(ne - nb);
+  }
+  float rx = px, ry = py, rz = pz;
+  if (cnt > 0) {
+    const float inv = 1.0f / (float)cnt;
+    rx = px + (ax * inv - px) * fade;
+    ry = py + (ay * inv - py) * fade;
+    rz = pz + (az * inv - pz) * fade;
+  }
+  dx[v] = rx;
+  dy[v] = ry;
+  dz[v] = rz;
+}
+
 // One Jacobi step of spec S8: src -> dst for this dab's affected elements; the others
 // hold the same values in both copies.
 __global__ __launch_bounds__(GR_THREADS) void kg_smooth(GView g, const float *sx, const float *sy, const float *sz,
@@ -277,44 +327,8 @@ __global__ __launch_bounds__(GR_THREADS) void kg_smooth(GView g, const float *sx
   for (int it = blockIdx.x; it < ng * g.nchunk; it += gridDim.x) {
     int b, e;
     if (!chunk_range(g, it, ng, b, e)) continue;
-    for (int v = b + threadIdx.x; v < e; v += GR_THREADS) {
-      if (g.stamp[v] != serial) continue;
-      const int local = v % g.ga, y = local / g.gs, x = local - y * g.gs;
-      const float px = sx[v], py = sy[v], pz = sz[v];
-      float ax = 0.0f, ay = 0.0f, az = 0.0f;
-      int cnt;
-      if (x > 0 && y > 0 && x < g.gs - 1 && y < g.gs - 1) {
-        // inside the grid: previous row, next row, previous column, next column
-        // (neighbor_coords_inner_get, subdiv_ccg.c:1870-1880)
-        const int u[4] = {v - g.gs, v + g.gs, v - 1, v + 1};
-        for (int q = 0; q < 4; q++) {
-          ax = ax + sx[u[q]];
-          ay = ay + sy[u[q]];
-          az = az + sz[u[q]];
-        }
-        cnt = 4;
-      } else {
-        const long long nb = g.nb_off[v], ne = g.nb_off[v + 1];
-        for (long long q = nb; q < ne; q++) {
-          const int u = g.nb_idx[q];
-          ax = ax + sx[u];
-          ay = ay + sy[u];
-          az = az + sz[u];
-        }
-        cnt = (int)(ne - nb);
-      }
-      float rx = px, ry = py, rz = pz;
-      if (cnt > 0) {
-        const float fade = g.fade[v];
-        const float inv = 1.0f / (float)cnt;
-        rx = px + (ax * inv - px) * fade;
-        ry = py + (ay * inv - py) * fade;
-        rz = pz + (az * inv - pz) * fade;
-      }
-      dx[v] = rx;
-      dy[v] = ry;
-      dz[v] = rz;
-    }
+    for (int v = b + threadIdx.x; v < e; v += GR_THREADS)
+      if (g.stamp[v] == serial) smooth_element(g, v, sx, sy, sz, g.fade[v], dx, dy, dz);
   }
 }
 
@@ -601,6 +615,326 @@ __global__ __launch_bounds__(GR_THREADS) void kg_edges_verts(GView g) {
 }
 
 
+// ---------------------------------------------------------------------------
+// A dab on a mesh whose faces fit a workgroup's LDS: per face, not per leaf.
+//   kg_dab_faces    a workgroup per face with a grid in a gathered leaf: brush, element
+//                   normals, the seams between its grids and the shared centre, all on the
+//                   face's elements in LDS; every element is read and written once
+//   kg_dab_edges    a wave per edge or coarse vertex of such a face: the averages
+//   kg_dab_refit    leaf boxes; its last workgroup closes the dab and searches for the next
+// Smooth(k) has its k Jacobi steps before (the first with the brush); the face kernel then
+// takes their result.  Every kernel is a chain of dependent loads of 1 us each on a few
+// hundred workgroups, so what counts is the number of kernels and of such loads: search,
+// brush, face normals, edges, box parts and box combine took 2.2 + 4.9 + 8.3 + 6.8 + 5.0 +
+// 3.6 us and as many boundaries (381 k elements, r 0.03 to 0.12).
+// ---------------------------------------------------------------------------
+#define DF_THREADS 512  // a face's grids (4 x 81 elements) in one pass
+#define DF_MAX_EPT 16   // passes over a face at most (the affected flags are a bit per pass)
+#define GR_LINES 16     // counter lines: [0] affected elements and, from bit 40, faces; [1] edges and vertices
+#define GR_LINE 16      // long longs per line
+
+__device__ __forceinline__ bool face_gathered(const GView &g, const int4 &fl, int serial) {
+  const int a = g.leaf_gmark[fl.x], b = g.leaf_gmark[fl.y], c = g.leaf_gmark[fl.z];
+  return a == serial || b == serial || c == serial;
+}
+
+__global__ __launch_bounds__(DF_THREADS) void kg_dab_faces(GView g, SgDabK k, const float *curve, int respect_hide,
+                                                           const float *sx, const float *sy, const float *sz) {
+  extern __shared__ float s_face[];
+  __shared__ int4 s_list[DF_THREADS];  // face, first grid, grids
+  __shared__ int s_n, s_naff, s_nface;
+  const int tid = threadIdx.x;
+  const int gs = g.gs, g1 = gs - 1, ga = g.ga, q1 = g1 * g1;
+  float *const P = s_face, *const N = P + 3 * g.maxn * ga, *const Q = N + 3 * g.maxn * ga;
+  float *const M = Q + 3 * g.maxn * q1;
+  int2 *const s_gpl = (int2 *)(M + (g.mask ? g.maxn * ga : 0) + (g.maxn * (q1 + (g.mask ? ga : 0)) & 1));
+  const int serial = g.dser[0];
+  const bool smooth = k.tool == SG_TOOL_SMOOTH;
+  float ox = 0.0f, oy = 0.0f, oz = 0.0f;
+  if (k.tool == SG_TOOL_DRAW) {
+    float ax = (float)((double)g.ctr[SGG_AREA_X] * (1.0 / 4294967296.0));
+    float ay = (float)((double)g.ctr[SGG_AREA_Y] * (1.0 / 4294967296.0));
+    float az = (float)((double)g.ctr[SGG_AREA_Z] * (1.0 / 4294967296.0));
+    sg_normalize(ax, ay, az);
+    ox = (ax * k.r) * k.bstr;
+    oy = (ay * k.r) * k.bstr;
+    oz = (az * k.r) * k.bstr;
+  }
+  if (tid == 0) s_naff = s_nface = 0;
+  for (int base = 0; base < g.F; base += gridDim.x * DF_THREADS) {
+    if (tid == 0) s_n = 0;
+    __syncthreads();
+    // the workgroup's faces of this round (every gridDim-th), a thread each
+    const int f = base + (int)blockIdx.x + tid * (int)gridDim.x;
+    if (f < g.F) {
+      const int4 fl = g.face_leaf[f];
+      const int g0 = g.face_gbeg[f], n = g.face_gbeg[f + 1] - g0;
+      bool hit = face_gathered(g, fl, serial);
+      if (fl.w == -2 && !hit)  // grids in more leaves than the record holds
+        for (int c = 0; c < n && !hit; c++) hit = g.leaf_gmark[g.grid_pl[g0 + c].y] == serial;
+      if (hit) s_list[atomicAdd(&s_n, 1)] = make_int4(f, g0, n, 0);
+    }
+    __syncthreads();
+    const int nl = s_n;
+    for (int q = 0; q < nl; q++) {
+      const int g0 = s_list[q].y, n = s_list[q].z, ne = n * ga;
+      for (int c = tid; c < n; c += DF_THREADS) s_gpl[c] = g.grid_pl[g0 + c];
+      __syncthreads();
+      unsigned affm = 0, gatm = 0;
+      int naff = 0;
+      for (int t = tid, it = 0; t < ne; t += DF_THREADS, it++) {
+        const int c = t / ga;
+        const int2 pl = s_gpl[c];
+        const int v = pl.x * ga + (t - c * ga);
+        float x = sx[v], y = sy[v], z = sz[v];
+        const bool gat = g.leaf_gmark[pl.y] == serial;
+        const float mk = g.mask ? g.mask[v] : 0.0f;
+        bool aff;
+        if (smooth) {
+          aff = g.stamp[v] == serial;
+        } else {
+          const float dx = k.cx - x, dy = k.cy - y, dz = k.cz - z;
+          const float d2 = dx * dx + dy * dy + dz * dz;
+          aff = gat && d2 <= k.r2 && !(g.hide && respect_hide && g.hide[v]);
+          if (aff) {
+            g.stamp[v] = serial;
+            const float fo = sg_falloff(k, curve, sqrtf(d2)) * (1.0f - mk);
+            if (k.tool == SG_TOOL_DRAW) {
+              x = x + ox * fo;
+              y = y + oy * fo;
+              z = z + oz * fo;
+            } else if (k.tool == SG_TOOL_INFLATE) {
+              const float s = (k.bstr * fo) * k.r;
+              x = x + g.nx[v] * s;
+              y = y + g.ny[v] * s;
+              z = z + g.nz[v] * s;
+            } else {
+              const float fade = k.bstr * fo;
+              x = x + k.gx * fade;
+              y = y + k.gy * fade;
+              z = z + k.gz * fade;
+            }
+          }
+        }
+        affm |= aff ? 1u << it : 0u;
+        gatm |= gat ? 1u << it : 0u;
+        naff += aff ? 1 : 0;
+        P[3 * t] = x;
+        P[3 * t + 1] = y;
+        P[3 * t + 2] = z;
+        if (g.mask) M[t] = mk;
+      }
+      __syncthreads();
+      // each quad's normal once (subdiv_ccg.c:670-740)
+      for (int t = tid; t < n * q1; t += DF_THREADS) {
+        const int c = t / q1, l = t - c * q1, qy = l / g1, qx = l - qy * g1;
+        quad_normal(P + 3 * c * ga, gs, qx, qy, Q[3 * t], Q[3 * t + 1], Q[3 * t + 2]);
+      }
+      __syncthreads();
+      for (int t = tid; t < ne; t += DF_THREADS) {
+        const int c = t / ga, l = t - c * ga, y = l / gs, x = l - y * gs;
+        const float *q0 = Q + 3 * (c * q1 + y * g1 + x);
+        float ax = 0.0f, ay = 0.0f, az = 0.0f;
+        int counter = 0;
+        auto add = [&](const float *p) {
+          ax += p[0];
+          ay += p[1];
+          az += p[2];
+          counter++;
+        };
+        if (x < g1 && y < g1) add(q0);
+        if (x >= 1) {
+          if (y < g1) add(q0 - 3);
+          if (y >= 1) add(q0 - 3 * (g1 + 1));
+        }
+        if (y >= 1 && x < g1) add(q0 - 3 * g1);
+        const float inv = 1.0f / (float)counter;
+        N[3 * t] = ax * inv;
+        N[3 * t + 1] = ay * inv;
+        N[3 * t + 2] = az * inv;
+      }
+      __syncthreads();
+      // seams (subdiv_ccg.c:876-900, :951-984): disjoint pairs; the centre by the last thread
+      for (int t = tid; t < n * g1; t += DF_THREADS) {
+        const int c = t / g1, ii = 1 + (t - c * g1);
+        const int a = ((c + n - 1) % n) * ga + ii, b = c * ga + ii * gs;
+        for (int i = 0; i < 3; i++) {
+          P[3 * a + i] = P[3 * b + i] = (P[3 * a + i] + P[3 * b + i]) * 0.5f;
+          N[3 * a + i] = N[3 * b + i] = (N[3 * a + i] + N[3 * b + i]) * 0.5f;
+        }
+        if (g.mask) M[a] = M[b] = (M[a] + M[b]) * 0.5f;
+      }
+      if (tid == DF_THREADS - 1) {
+        float s[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        for (int c = 0; c < n; c++) {
+          for (int i = 0; i < 3; i++) {
+            s[i] += P[3 * c * ga + i];
+            s[3 + i] += N[3 * c * ga + i];
+          }
+          if (g.mask) s[6] += M[c * ga];
+        }
+        const float inv = 1.0f / n;
+        for (int i = 0; i < 7; i++) s[i] *= inv;
+        for (int c = 0; c < n; c++) {
+          for (int i = 0; i < 3; i++) {
+            P[3 * c * ga + i] = s[i];
+            N[3 * c * ga + i] = s[3 + i];
+          }
+          if (g.mask) M[c * ga] = s[6];
+        }
+      }
+      for (int c = tid; c < n; c += DF_THREADS) {
+        g.edge_stamp[g.face_edge[g0 + c]] = serial;  // (every face of the edge or vertex writes the same)
+        g.vert_stamp[g.face_vert[g0 + c]] = serial;
+      }
+      __syncthreads();
+      for (int t = tid, it = 0; t < ne; t += DF_THREADS, it++) {
+        const int c = t / ga, l = t - c * ga;
+        const int v = s_gpl[c].x * ga + l;
+        const bool seam = l < gs || l % gs == 0;
+        if (seam || (affm >> it & 1)) {
+          const float x = P[3 * t], y = P[3 * t + 1], z = P[3 * t + 2];
+          // leaves that were not gathered join the refit when an average moved their element
+          if (!(gatm >> it & 1) &&
+              (__float_as_uint(g.px[v]) != __float_as_uint(x) || __float_as_uint(g.py[v]) != __float_as_uint(y) ||
+               __float_as_uint(g.pz[v]) != __float_as_uint(z)))
+            mark_moved(g, v, serial);
+          g.px[v] = g.qx[v] = x;
+          g.py[v] = g.qy[v] = y;
+          g.pz[v] = g.qz[v] = z;
+          if (seam && g.mask) g.mask[v] = M[t];
+        }
+        g.nx[v] = N[3 * t];
+        g.ny[v] = N[3 * t + 1];
+        g.nz[v] = N[3 * t + 2];
+      }
+      naff = wave_sum_i(naff);
+      if (lane_id() == 0 && naff) atomicAdd(&s_naff, naff);
+      if (tid == 0) s_nface++;
+      __syncthreads();  // LDS is reused by the next face
+    }
+    __syncthreads();
+  }
+  if (tid == 0 && s_nface)  // 16 lines: one counter took 12 ns per workgroup
+    atomicAdd((unsigned long long *)&g.lines[(blockIdx.x % GR_LINES) * GR_LINE],
+              ((unsigned long long)s_nface << 40) + (unsigned long long)s_naff);
+}
+
+// Smooth: the factors of the affected elements and the first Jacobi step (p -> q).
+__global__ __launch_bounds__(GR_THREADS) void kg_smooth_first(GView g, SgDabK k, const float *curve, int respect_hide) {
+  const int serial = g.dser[0];
+  const int ng = (int)g.ctr[SGG_NGATHER];
+  for (int it = blockIdx.x; it < ng * g.nchunk; it += gridDim.x) {
+    int b, e;
+    if (!chunk_range(g, it, ng, b, e)) continue;
+    for (int v = b + threadIdx.x; v < e; v += GR_THREADS) {
+      if (g.hide && respect_hide && g.hide[v]) continue;
+      const float x = g.px[v], y = g.py[v], z = g.pz[v];
+      const float dx = k.cx - x, dy = k.cy - y, dz = k.cz - z;
+      const float d2 = dx * dx + dy * dy + dz * dz;
+      if (!(d2 <= k.r2)) continue;
+      g.stamp[v] = serial;
+      const float mk = g.mask ? g.mask[v] : 0.0f;
+      const float fade = k.bstr * (sg_falloff(k, curve, sqrtf(d2)) * (1.0f - mk));
+      g.fade[v] = fade;
+      smooth_element(g, v, g.px, g.py, g.pz, fade, g.qx, g.qy, g.qz);
+    }
+  }
+}
+
+// The mean of up to four listed elements: every load ahead of the sums (element order).
+__device__ __forceinline__ void avg_few(const GView &g, const int *els, int stride, int n, int serial) {
+  int id[4];
+  float v[4][7];
+#pragma unroll
+  for (int k = 0; k < 4; k++) id[k] = els[(size_t)min(k, n - 1) * stride];
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    v[k][0] = g.px[id[k]];
+    v[k][1] = g.py[id[k]];
+    v[k][2] = g.pz[id[k]];
+    v[k][3] = g.nx[id[k]];
+    v[k][4] = g.ny[id[k]];
+    v[k][5] = g.nz[id[k]];
+    v[k][6] = g.mask ? g.mask[id[k]] : 0.0f;
+  }
+  float s[7] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (k < n)
+      for (int i = 0; i < 7; i++) s[i] += v[k][i];
+  const float inv = 1.0f / n;
+  for (int i = 0; i < 7; i++) s[i] *= inv;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    if (k >= n) continue;
+    const int e = id[k];
+    if (__float_as_uint(v[k][0]) != __float_as_uint(s[0]) || __float_as_uint(v[k][1]) != __float_as_uint(s[1]) ||
+        __float_as_uint(v[k][2]) != __float_as_uint(s[2]))
+      mark_moved(g, e, serial);
+    g.px[e] = g.qx[e] = s[0];
+    g.py[e] = g.qy[e] = s[1];
+    g.pz[e] = g.qz[e] = s[2];
+    g.nx[e] = s[3];
+    g.ny[e] = s[4];
+    g.nz[e] = s[5];
+    if (g.mask) g.mask[e] = s[6];
+  }
+}
+
+// The averages of kg_edges_verts for the edges and vertices the face kernel stamped: a lane
+// checks an item (every wave-count-th, so that neighbours go to different waves), the wave
+// then takes the stamped ones.
+__global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
+  __shared__ int s_n;
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  const int serial = g.dser[0];
+  const int lane = lane_id();
+  const int w = (blockIdx.x * blockDim.x + threadIdx.x) / SG_WAVE;
+  const int nw = gridDim.x * blockDim.x / SG_WAVE;
+  const int n2 = 2 * g.gs, total = g.Ed + g.Vc;
+  int cnt = 0;
+  for (int base = 0; base < total; base += nw * SG_WAVE) {
+    const int item = base + w + lane * nw;
+    bool hit = false;
+    int fb = 0, nf = 0;
+    if (item < total) {
+      const bool edge = item < g.Ed;
+      const int j = edge ? item : item - g.Ed;
+      const int *off = edge ? g.edge_foff : g.vert_foff;
+      hit = (edge ? g.edge_stamp[j] : g.vert_stamp[j]) == serial;
+      fb = off[j];
+      nf = off[j + 1] - fb;
+    }
+    unsigned long long m = __ballot(hit);
+    cnt += __popcll(m);
+    while (m) {
+      const int src = __ffsll((unsigned long long)m) - 1;
+      m &= m - 1;
+      const int it = __shfl(item, src), b = __shfl(fb, src), n = __shfl(nf, src);
+      if (n <= 1) continue;
+      if (it < g.Ed) {
+        for (int p = 1 + lane; p < n2 - 1; p += SG_WAVE) {
+          if (n <= 4)
+            avg_few(g, g.edge_el + (size_t)b * n2 + p, n2, n, serial);
+          else
+            avg_list(g, g.edge_el + (size_t)b * n2 + p, n2, n, serial);
+        }
+      } else if (lane == 0) {
+        if (n <= 4)
+          avg_few(g, g.vert_el + b, 1, n, serial);
+        else
+          avg_list(g, g.vert_el + b, 1, n, serial);
+      }
+    }
+  }
+  if (lane == 0 && cnt) atomicAdd(&s_n, cnt);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_n)
+    atomicAdd((unsigned long long *)&g.lines[(blockIdx.x % GR_LINES) * GR_LINE + 1], (unsigned long long)s_n);
+}
+
 // Leaf refit (update_node_vb, pbvh.c:108-128): vb = min/max over the leaf's elements
 // in iteration order.  min_ff / max_ff keep the later of equal values, so any fold that
 // combines contiguous pieces left to right gives the sequential result.  The listed
@@ -610,65 +944,171 @@ __global__ __launch_bounds__(GR_THREADS) void kg_edges_verts(GView g) {
 // coordinate, an ordered DPP scan over the lanes), 4 rounds in flight; the waves
 // combine in order into the part's box.
 #define GR_SPLIT 8
-__global__ __launch_bounds__(GR_THREADS) void kg_refit_parts(GView g, const int *list, int list_n, float *parts) {
+#define GR_ROUNDS 8  // rounds of a wave in flight
+// A fold without the order is the same box unless a value is not a number or a side is zero
+// (equal values of two signs), so each lane first folds its own elements and one scan joins
+// the lanes; only those cases fold round by round in order (a scan per round: 6 values times
+// 6 steps each).
+__device__ __forceinline__ void part_box(const GView &g, int l, int part, float (*s_bb)[6], BB6 &r) {
   constexpr int NW = GR_THREADS / SG_WAVE;
-  __shared__ float s_bb[NW][6];
   const int lane = lane_id(), w = threadIdx.x / SG_WAVE;
+  const int b = g.leaf_gbeg[l] * g.ga, e = g.leaf_gbeg[l + 1] * g.ga;
+  const int seg = (e - b + GR_SPLIT - 1) / GR_SPLIT;
+  const int pb = min(e, b + part * seg), pe = min(e, pb + seg);
+  const int q = (pe - pb + NW - 1) / NW;
+  const int wb = min(pe, pb + w * q), we = min(pe, wb + q);
+  BB6 acc;
+  bb_reset(acc);
+  bool odd = false;
+  for (int base = wb; base < we; base += SG_WAVE * GR_ROUNDS) {
+    float x[GR_ROUNDS], y[GR_ROUNDS], z[GR_ROUNDS];
+#pragma unroll
+    for (int i = 0; i < GR_ROUNDS; i++) {  // every load issued (clamped index) before any is folded
+      const int v = min(base + i * SG_WAVE + lane, we - 1);
+      x[i] = g.px[v];
+      y[i] = g.py[v];
+      z[i] = g.pz[v];
+    }
+#pragma unroll
+    for (int i = 0; i < GR_ROUNDS; i++) {
+      odd = odd || x[i] != x[i] || y[i] != y[i] || z[i] != z[i];
+      bb_add_point(acc, x[i], y[i], z[i]);  // (a clamped lane folds the last element again)
+    }
+  }
+  acc = bb_wave_scan(acc);
+  for (int i = 0; i < 3; i++) {
+    acc.mn[i] = __shfl(acc.mn[i], SG_WAVE - 1);
+    acc.mx[i] = __shfl(acc.mx[i], SG_WAVE - 1);
+    odd = odd || acc.mn[i] == 0.0f || acc.mx[i] == 0.0f;
+  }
+  if (__any(odd)) {
+    bb_reset(acc);
+    for (int base = wb; base < we; base += SG_WAVE) {
+      const int v = base + lane;
+      BB6 t;
+      bb_reset(t);
+      if (v < we) bb_add_point(t, g.px[v], g.py[v], g.pz[v]);
+      t = bb_wave_scan(t);
+      BB6 tot;
+      for (int i = 0; i < 3; i++) {
+        tot.mn[i] = __shfl(t.mn[i], SG_WAVE - 1);
+        tot.mx[i] = __shfl(t.mx[i], SG_WAVE - 1);
+      }
+      bb_add_bb(acc, tot);
+    }
+  }
+  if (lane == 0)
+    for (int i = 0; i < 3; i++) {
+      s_bb[w][i] = acc.mn[i];
+      s_bb[w][3 + i] = acc.mx[i];
+    }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    bb_reset(r);
+    for (int k = 0; k < NW; k++) {
+      BB6 xk;
+      for (int i = 0; i < 3; i++) {
+        xk.mn[i] = s_bb[k][i];
+        xk.mx[i] = s_bb[k][3 + i];
+      }
+      bb_add_bb(r, xk);
+    }
+  }
+}
+
+__global__ __launch_bounds__(GR_THREADS) void kg_refit_parts(GView g, const int *list, int list_n, float *parts) {
+  __shared__ float s_bb[GR_THREADS / SG_WAVE][6];
   const int nl = list ? list_n : (int)(g.ctr[SGG_NGATHER] + g.ctr[SGG_NMOVED]);
   for (int item = blockIdx.x; item < nl * GR_SPLIT; item += gridDim.x) {
-    const int li = item / GR_SPLIT, part = item - li * GR_SPLIT;
-    const int l = list ? list[li] : g.gathered[li];
-    const int b = g.leaf_gbeg[l] * g.ga, e = g.leaf_gbeg[l + 1] * g.ga;
-    const int seg = (e - b + GR_SPLIT - 1) / GR_SPLIT;
-    const int pb = min(e, b + part * seg), pe = min(e, pb + seg);
-    const int q = (pe - pb + NW - 1) / NW;
-    const int wb = min(pe, pb + w * q), we = min(pe, wb + q);
-    BB6 acc;
-    bb_reset(acc);
-    for (int base = wb; base < we; base += SG_WAVE * 4) {
-      float x[4], y[4], z[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {  // every load issued (clamped index) before any is folded
-        const int v = min(base + r * SG_WAVE + lane, we - 1);
-        x[r] = g.px[v];
-        y[r] = g.py[v];
-        z[r] = g.pz[v];
-      }
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        BB6 t;
-        bb_reset(t);
-        if (base + r * SG_WAVE + lane < we) bb_add_point(t, x[r], y[r], z[r]);
-        t = bb_wave_scan(t);
-        BB6 tot;
-        for (int i = 0; i < 3; i++) {
-          tot.mn[i] = __shfl(t.mn[i], SG_WAVE - 1);
-          tot.mx[i] = __shfl(t.mx[i], SG_WAVE - 1);
-        }
-        bb_add_bb(acc, tot);
-      }
-    }
-    if (lane == 0)
-      for (int i = 0; i < 3; i++) {
-        s_bb[w][i] = acc.mn[i];
-        s_bb[w][3 + i] = acc.mx[i];
-      }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      BB6 r;
-      bb_reset(r);
-      for (int k = 0; k < NW; k++) {
-        BB6 xk;
-        for (int i = 0; i < 3; i++) {
-          xk.mn[i] = s_bb[k][i];
-          xk.mx[i] = s_bb[k][3 + i];
-        }
-        bb_add_bb(r, xk);
-      }
-      bb_store(parts + 8 * (size_t)item, r);
-    }
+    const int li = item / GR_SPLIT;
+    BB6 r;
+    part_box(g, list ? list[li] : g.gathered[li], item - li * GR_SPLIT, s_bb, r);
+    if (threadIdx.x == 0) bb_store(parts + 8 * (size_t)item, r);
     __syncthreads();
   }
+}
+
+// The dab's leaf boxes, then in the workgroup that finishes last what kg_refit_combine does
+// with `finish`, and, when a dab follows (has_next), its search: as launches of their own
+// these were 3.6 and 2.2 us and two boundaries.  Workgroups with no part leave at once; the
+// others count themselves in with release and acquire at agent scope, so the last one sees
+// every part.
+__global__ __launch_bounds__(GR_THREADS) void kg_dab_refit(GView g, float *parts, long long *log, SgDabK kn,
+                                                           int has_next) {
+  __shared__ float s_bb[GR_THREADS / SG_WAVE][6];
+  __shared__ long long s_c[SGG_CTR_COUNT];
+  __shared__ int s_last, s_ng;
+  const int t = threadIdx.x;
+  const int nl = (int)(g.ctr[SGG_NGATHER] + g.ctr[SGG_NMOVED]);
+  const int nb = max(1, min((int)gridDim.x, nl * GR_SPLIT));  // workgroups that take part
+  if ((int)blockIdx.x >= nb) return;
+  for (int item = blockIdx.x; item < nl * GR_SPLIT; item += gridDim.x) {
+    const int li = item / GR_SPLIT;
+    BB6 r;
+    part_box(g, g.gathered[li], item - li * GR_SPLIT, s_bb, r);
+    if (t == 0) bb_store(parts + 8 * (size_t)item, r);
+    __syncthreads();
+  }
+  if (t == 0) {
+    s_last = __hip_atomic_fetch_add(&g.dser[2], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == nb - 1;
+    s_ng = 0;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const int serial = g.dser[0];
+  for (int li = t; li < nl; li += GR_THREADS) {
+    const int l = g.gathered[li];
+    BB6 p[GR_SPLIT], r;
+#pragma unroll
+    for (int i = 0; i < GR_SPLIT; i++) p[i] = gbb_load(parts + 8 * ((size_t)li * GR_SPLIT + i));
+    bb_reset(r);
+#pragma unroll
+    for (int i = 0; i < GR_SPLIT; i++) bb_add_bb(r, p[i]);
+    bb_store(g.leaf_bb + 8 * (size_t)l, r);
+    bb_store(g.leaf_obb + 8 * (size_t)l, r);
+    g.leaf_dirty[l] = 1;
+  }
+  if (t < SGG_CTR_COUNT) s_c[t] = g.ctr[t];
+  if (t < SG_WAVE) {  // the counter lines
+    const bool in = t < GR_LINES;
+    const long long a = in ? g.lines[t * GR_LINE] : 0, b = in ? g.lines[t * GR_LINE + 1] : 0;
+    const long long sa = wave_sum_ll(a), sb = wave_sum_ll(b);
+    if (in) g.lines[t * GR_LINE] = g.lines[t * GR_LINE + 1] = 0;
+    if (t == 0) {
+      s_c[SGG_NAFF] = sa & ((1ll << 40) - 1);
+      s_c[SGG_NFACES] = sa >> 40;
+      s_c[SGG_NITEMS] = sb;
+    }
+  }
+  __syncthreads();
+  if (t < SGG_CTR_COUNT) {
+    g.ctr_last[t] = t == SGG_NLEAVES ? nl : s_c[t];
+    g.ctr[t] = 0;
+  }
+  if (log && t < SG_CTR_COUNT) {
+    const int src = t == SG_CTR_NGATHER ? SGG_NGATHER : t == SG_CTR_NAFF ? SGG_NAFF : t == SG_CTR_AREA_X ? SGG_AREA_X
+                  : t == SG_CTR_AREA_Y ? SGG_AREA_Y : t == SG_CTR_AREA_Z ? SGG_AREA_Z : t == SG_CTR_NAREA ? SGG_NAREA
+                  : -1;
+    log[t] = src >= 0 ? s_c[src] : 0;
+  }
+  if (t == 0) {
+    g.dser[1] = serial;
+    g.dser[0] = serial + 1;
+    g.dser[2] = 0;
+  }
+  if (!has_next) return;
+  for (int l = t; l < g.L; l += GR_THREADS) {
+    const BB6 b = gbb_load((kn.use_orig ? g.leaf_obb : g.leaf_bb) + 8 * (size_t)l);
+    const bool pass = !((g.leaf_flags[l] & 1) && kn.hide_skip) && sphere_box(b, kn.cx, kn.cy, kn.cz, kn.r2);
+    if (pass) {
+      g.gathered[atomicAdd(&s_ng, 1)] = l;
+      g.leaf_mark[l] = serial + 1;
+      g.leaf_gmark[l] = serial + 1;
+    }
+  }
+  __syncthreads();
+  if (t == 0) g.ctr[SGG_NGATHER] = s_ng;
 }
 
 // The listed leaves' boxes from their parts, in order; orig_vb = vb when set_orig; the
@@ -747,8 +1187,10 @@ __global__ __launch_bounds__(1024) void kg_flush_nodes(GView g, int set_orig) {
 // and take the next serial on the device (a dab ends the same way in kg_refit_combine).
 __global__ void kg_clear_ctr(GView g) {
   if (threadIdx.x < SGG_CTR_COUNT) g.ctr[threadIdx.x] = 0;
+  if (threadIdx.x < GR_LINES) g.lines[threadIdx.x * GR_LINE] = g.lines[threadIdx.x * GR_LINE + 1] = 0;
   if (threadIdx.x == 0) {
     g.dser[0] = g.dser[0] + 1;
+    g.dser[2] = 0;
   }
 }
 
@@ -788,6 +1230,10 @@ void free_topology(SgGridDev &d) {
   gfree(d.face_stamp);
   gfree(d.edge_stamp);
   gfree(d.vert_stamp);
+  gfree(d.face_leaf);
+  gfree(d.grid_pl);
+  d.maxn = 0;
+  d.face_lds = 0;
   gfree(d.dfaces);
   gfree(d.ditems);
   d.F = d.Ed = d.Vc = 0;
@@ -808,13 +1254,14 @@ void sg_grids_free_device(PBVH *p) {
                   &d.leaf_bb, &d.leaf_obb, &d.node_bb, &d.node_obb, &d.curve};
   for (float **q : fl) gfree(*q);
   int **il[] = {&d.stamp, &d.grid_pos, &d.grid_old, &d.grid_leaf, &d.leaf_gbeg, &d.leaf_flags, &d.leaf_mark,
-                &d.node_child, &d.node_leaf, &d.node_mark, &d.lvl_off, &d.lvl_node, &d.gathered};
+                &d.leaf_gmark, &d.node_child, &d.node_leaf, &d.node_mark, &d.lvl_off, &d.lvl_node, &d.gathered};
   for (int **q : il) gfree(*q);
   gfree(d.hide);
   gfree(d.ctr);
   gfree(d.ctr_last);
   gfree(d.hlist);
   gfree(d.dser);
+  gfree(d.lines);
   gfree(d.parts);
   gfree(d.leaf_dirty);
   gfree(d.node_dirty);
@@ -928,6 +1375,8 @@ int sg_grids_build_device(PBVH *p) {
   rc |= gupload(&d.leaf_gbeg, leaf_gbeg.data(), leaf_gbeg.size());
   rc |= gupload(&d.leaf_flags, leaf_flags.data(), leaf_flags.size());
   rc |= gzeros(&d.leaf_mark, (size_t)d.L);
+  rc |= gzeros(&d.leaf_gmark, (size_t)d.L);
+  rc |= gzeros(&d.lines, (size_t)GR_LINES * GR_LINE);
   rc |= gupload(&d.leaf_bb, lbb.data(), lbb.size());
   rc |= gupload(&d.leaf_obb, lobb.data(), lobb.size());
   rc |= gupload(&d.node_child, child.data(), child.size());
@@ -994,6 +1443,32 @@ int sg_grids_attach_topology(PBVH *p, const SubdivCCG *s) {
   std::vector<int> edge_el(s->edge_coords.size()), vert_el(s->vert_coords.size());
   for (size_t i = 0; i < edge_el.size(); i++) edge_el[i] = el(s->edge_coords[i]);
   for (size_t i = 0; i < vert_el.size(); i++) vert_el[i] = el(s->vert_coords[i]);
+  // by grid id: position and leaf; by face: up to three leaves (the first one repeated; .w =
+  // -2: there are more)
+  std::vector<int> grid_leaf(d.G);
+  if (sg_check_hip(hipMemcpy(grid_leaf.data(), d.grid_leaf, d.G * sizeof(int), hipMemcpyDeviceToHost), "copy"))
+    return -1;
+  std::vector<int2> grid_pl(d.G);
+  for (int g = 0; g < d.G; g++) grid_pl[g] = make_int2(grid_pos[g], grid_leaf[grid_pos[g]]);
+  std::vector<int4> face_leaf(s->num_faces);
+  int maxn = 1;
+  for (int f = 0; f < s->num_faces; f++) {
+    int lv[4], nl = 0;
+    for (int g = face_gbeg[f]; g < face_gbeg[f + 1]; g++) {
+      const int l = grid_pl[g].y;
+      if (std::find(lv, lv + std::min(nl, 3), l) != lv + std::min(nl, 3)) continue;
+      if (nl < 3) lv[nl] = l;
+      nl++;
+    }
+    for (int i = std::max(nl, 1); i < 3; i++) lv[i] = nl > 0 ? lv[0] : 0;
+    face_leaf[f] = make_int4(nl > 0 ? lv[0] : 0, lv[1], lv[2], nl > 3 ? -2 : -1);
+    maxn = std::max(maxn, face_gbeg[f + 1] - face_gbeg[f]);
+  }
+  d.maxn = maxn;
+  const size_t words = (size_t)maxn * (6 * (size_t)ga + 3 * (size_t)(gs - 1) * (gs - 1) + (d.mask ? ga : 0) + 2) + 2;
+  // the face kernel's LDS; faces past its limits (grids of level 6, polygons of many corners)
+  // take the kernels per leaf
+  d.face_lds = words * 4 <= 52 * 1024 && (size_t)maxn * ga <= (size_t)DF_THREADS * DF_MAX_EPT ? (int)(words * 4) : 0;
   d.F = s->num_faces;
   d.Ed = s->num_edges;
   d.Vc = s->num_coarse_verts;
@@ -1013,6 +1488,8 @@ int sg_grids_attach_topology(PBVH *p, const SubdivCCG *s) {
   rc |= gzeros(&d.face_stamp, (size_t)d.F);
   rc |= gzeros(&d.edge_stamp, (size_t)d.Ed);
   rc |= gzeros(&d.vert_stamp, (size_t)d.Vc);
+  rc |= gupload(&d.grid_pl, grid_pl.data(), grid_pl.size());
+  rc |= gupload(&d.face_leaf, face_leaf.data(), face_leaf.size());
   rc |= gzeros(&d.dfaces, (size_t)d.F);
   rc |= gzeros(&d.ditems, (size_t)d.Ed + d.Vc);
   if (rc) return -1;
@@ -1039,9 +1516,12 @@ static int enqueue_normals(PBVH *p, const GView &g, const int *leaves, int n) {
   return launch_check("grid normals");
 }
 
-int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index) {
+int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index,
+                         const SgDabK *next) {
   if (!p->gd) return sg_set_error("grids: no device layout");
   SgGridDev &d = *p->gd;
+  const bool searched = d.searched;  // by the dab before
+  d.searched = false;
   if (!d.topo_of) return sg_set_error("grids: no SubdivCCG attached (DUNE_pbvh_subdiv_cgg_set)");
   if (k.tool != SG_TOOL_DRAW && k.tool != SG_TOOL_INFLATE && k.tool != SG_TOOL_SMOOTH && k.tool != SG_TOOL_GRAB)
     return sg_set_error("grids: tool %d is not supported on PBVH_GRIDS (Draw, Inflate, Smooth, Grab)", k.tool);
@@ -1050,10 +1530,39 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   const int rh = p->respect_hide ? 1 : 0;
   const int eb = elem_blocks(d);
   const bool normals = p->gridkey.has_normals != 0;
-  if (d.ctr_unclean) kg_clear_ctr<<<1, 64, 0, p->stream>>>(g);  // a failed launch left the counters
+  // a failed launch, or a search for a dab that did not follow, left the counters
+  if (d.ctr_unclean && !searched) kg_clear_ctr<<<1, 64, 0, p->stream>>>(g);
   d.ctr_unclean = true;
-  kg_search<<<(d.L + GR_THREADS - 1) / GR_THREADS, GR_THREADS, 0, p->stream>>>(g, k);
+  if (!searched) kg_search<<<(d.L + GR_THREADS - 1) / GR_THREADS, GR_THREADS, 0, p->stream>>>(g, k);
   if (k.tool == SG_TOOL_DRAW) kg_area<<<eb, GR_THREADS, 0, p->stream>>>(g, k, rh);
+  if (normals && d.face_lds > 0) {
+    const float *s[3] = {d.px, d.py, d.pz};
+    if (k.tool == SG_TOOL_SMOOTH) {
+      if (k.iters < 1) {
+        kg_brush<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh, 0);
+      } else {
+        kg_smooth_first<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh);
+        for (int it = 1; it < k.iters; it++) {
+          if (it & 1)
+            kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.qx, d.qy, d.qz, d.px, d.py, d.pz);
+          else
+            kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.px, d.py, d.pz, d.qx, d.qy, d.qz);
+        }
+        if (k.iters & 1) s[0] = d.qx, s[1] = d.qy, s[2] = d.qz;
+      }
+    }
+    kg_dab_faces<<<std::max(1, std::min(d.F, 2048)), DF_THREADS, d.face_lds, p->stream>>>(g, k, curve_dev, rh, s[0], s[1],
+                                                                                        s[2]);
+    kg_dab_edges<<<std::max(1, std::min((d.Ed + d.Vc + 3) / 4, 1024)), GR_THREADS, 0, p->stream>>>(g);
+    // one workgroup searches 256 leaves at a time: past a few rounds a launch of its own is shorter
+    const bool search = next && d.L <= 4 * GR_THREADS;
+    const SgDabK kn = search ? *next : k;
+    kg_dab_refit<<<std::max(1, std::min(d.L * GR_SPLIT, 512)), GR_THREADS, 0, p->stream>>>(
+        g, d.parts, log ? log + (size_t)log_index * SG_CTR_COUNT : nullptr, kn, search ? 1 : 0);
+    if (int rc = launch_check("grid dab")) return rc;
+    d.searched = d.ctr_unclean = search;
+    return 0;
+  }
   kg_brush<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh, normals ? 1 : 0);
   if (k.tool == SG_TOOL_SMOOTH) {
     for (int it = 0; it < k.iters; it++) {

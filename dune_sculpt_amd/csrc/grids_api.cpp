@@ -208,6 +208,7 @@ int sg_grids_dab_apply(PBVH *p, const SgDabParams *dab) {
     if (int rc = sg_grids_attach_topology(p, p->subdiv_ccg)) return rc;
   }
   const SgDabK k = sg_make_dab(dab, 0);
+  p->gd->searched = false;
   const float *curve = nullptr;
   if (dab->curve_preset == SG_CURVE_CUSTOM && dab->curve_table) {
     if (sg_check_hip(hipMemcpyAsync(p->gd->curve, dab->curve_table, (SG_CM_TABLE + 1) * sizeof(float),

@@ -1,0 +1,72 @@
+"""Strokes on grids, where each dab searches for the next and the faces fit a workgroup,
+against the oracle and against the same dabs one by one, bit for bit: small and large
+grids (level 6: the kernels per leaf), more leaves than one workgroup searches, faces whose
+grids lie in several leaves, coordinates that are zero (boxes with a side of either sign)."""
+import numpy as np
+import pytest
+
+from dune_sculpt_amd import grids as gr
+from test_gpu_grids import noisy_sphere_grids, oracle_of, stroke
+
+pytestmark = pytest.mark.gpu
+
+
+def _all(p):
+    co, no, mk = p.state()
+    vb, ob = p.boxes()
+    return [co, no, vb, ob, p.last_affected(), p.last_gathered(), p.last_stats()[:2]] + ([mk] if mk is not None else [])
+
+
+@pytest.mark.parametrize("n,level,leaf_limit,amp,mask", [
+    (1, 2, 10, 0.02, False), (3, 3, 100, 0.0, False), (4, 5, 1500, 0.02, True), (2, 6, 4000, 0.02, False),
+    (20, 2, 40, 0.02, False), (9, 4, 100, 0.0, True)])
+def test_stroke(sg, po, n, level, leaf_limit, amp, mask):
+    dabs = stroke(sg, 3, 21, 0.1, 0.5)
+    got = []
+    for how in ("graph", "stream", "dabs"):
+        g, mesh = noisy_sphere_grids(sg, n, level, seed=5, amp=amp, mask=mask)
+        if mask:
+            g.set_mask(np.clip(g.co()[:, 0], 0, 1).astype(np.float32))
+        if how == "graph":
+            o = oracle_of(po, g, mesh, leaf_limit)
+            for d in dabs + dabs:
+                o.dab(po.to_orc(d))
+            want = [*o.state()[:2], *o.boxes()]
+            o.close()
+        p = gr.GridPBVH(g, leaf_limit=leaf_limit)
+        if how == "dabs":
+            for d in dabs + dabs:
+                p.dab(d)
+        elif how == "stream":
+            p.stroke(dabs, graph=False)
+            p.stroke(dabs, graph=False)
+        else:
+            s = p.prepare(dabs)
+            s.launch(sync=False)
+            s.launch()
+        got.append(_all(p))
+        p.close()
+    for a in got:
+        for x, y in zip(a[:4], want):
+            assert np.array_equal(np.ascontiguousarray(x).view(np.uint32), np.ascontiguousarray(y).view(np.uint32))
+        for x, y in zip(a, got[0]):
+            assert np.asarray(x).tobytes() == np.asarray(y).tobytes()
+
+
+def test_single_dab_after_strokes_and_edits(sg, po):
+    """The counters and marks a stroke leaves: a dab, a host edit's updates, a replay."""
+    dabs = stroke(sg, 3, 5, 0.2, 0.4)
+    got = []
+    for chained in (True, False):
+        g, _ = noisy_sphere_grids(sg, 5, 4, seed=5)
+        p = gr.GridPBVH(g, leaf_limit=1000)
+        run = (lambda: p.stroke(dabs, graph=False)) if chained else (lambda: [p.dab(d) for d in dabs])
+        run()
+        p.dab(dabs[2])
+        p.snapshot()
+        run()
+        p.restore()
+        run()
+        got.append(_all(p))
+        p.close()
+    assert all(np.asarray(x).tobytes() == np.asarray(y).tobytes() for x, y in zip(*got))
