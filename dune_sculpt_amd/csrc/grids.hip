@@ -1194,6 +1194,19 @@ __global__ void kg_clear_ctr(GView g) {
   }
 }
 
+// The elements as the SubdivCCG stores them: grid by grid (id order), `words` 32-bit words
+// each, position first, normal and mask at their word offsets (-1: none).
+__global__ __launch_bounds__(GR_THREADS) void kg_pack(GView g, int words, int no, int mk, unsigned *out) {
+  const size_t n = (size_t)g.G * g.ga * words;
+  for (size_t i = (size_t)blockIdx.x * GR_THREADS + threadIdx.x; i < n; i += (size_t)gridDim.x * GR_THREADS) {
+    const int e = (int)(i / words), w = (int)(i - (size_t)e * words), id = e / g.ga;
+    const size_t v = (size_t)g.grid_pos[id] * g.ga + (e - id * g.ga);
+    const float *src = w == 0 ? g.px : w == 1 ? g.py : w == 2 ? g.pz : w == mk ? g.mask
+                     : w == no ? g.nx : w == no + 1 ? g.ny : g.nz;
+    out[i] = __float_as_uint(src[v]);
+  }
+}
+
 template <class T>
 int gupload(T **dst, const T *src, size_t n) {
   if (sg_check_hip(hipMalloc(dst, std::max<size_t>(n, 1) * sizeof(T)), "hipMalloc")) return -1;
@@ -1261,6 +1274,7 @@ void sg_grids_free_device(PBVH *p) {
   gfree(d.ctr_last);
   gfree(d.hlist);
   gfree(d.dser);
+  gfree(d.pack);
   gfree(d.lines);
   gfree(d.parts);
   gfree(d.leaf_dirty);
@@ -1614,6 +1628,27 @@ int sg_grids_enqueue_refit(PBVH *p, const int *leaves_dev, int n, int set_orig) 
   kg_flush_nodes<<<1, 1024, 0, p->stream>>>(g, set_orig);
   kg_clear_ctr<<<1, 64, 0, p->stream>>>(g);
   return launch_check("grid refit");
+}
+
+// Every element into contiguous storage of the caller's layout; 1 when the layout is not one
+// that the elements fill word for word (the caller then copies field by field).
+// Field by field this was six copies, a host pass from three arrays to one and another into
+// the storage: 1.25 ms for 381 k elements, where packing on the GPU and one copy take
+// 0.57.
+int sg_grids_download_packed(PBVH *p, void *out) {
+  SgGridDev &d = *p->gd;
+  const CCGKey &key = p->gridkey;
+  const int words = key.elem_size / 4, no = key.has_normals ? key.normal_offset / 4 : -1,
+            mk = key.has_mask && d.mask ? key.mask_offset / 4 : -1;
+  if (key.elem_size % 4 || (key.has_normals && key.normal_offset % 4) || (key.has_mask && key.mask_offset % 4) ||
+      words != 3 + (no >= 0 ? 3 : 0) + (mk >= 0 ? 1 : 0) || (key.has_mask && mk < 0))
+    return 1;
+  const size_t bytes = (size_t)d.E * key.elem_size;
+  if (!d.pack && sg_check_hip(hipMalloc(&d.pack, std::max<size_t>(bytes, 4)), "hipMalloc")) return -1;
+  kg_pack<<<(int)std::max<size_t>(1, std::min<size_t>((bytes / 4 + GR_THREADS - 1) / GR_THREADS, 8192)), GR_THREADS, 0,
+            p->stream>>>(view_of(d), words, no, mk, d.pack);
+  if (int rc = launch_check("grid pack")) return rc;
+  return sg_read_back(p->stream, p->pin, d.pack, out, bytes, "grid read");
 }
 
 int sg_grids_download(PBVH *p, float *co, float *no, float *mask) {

@@ -163,6 +163,13 @@ int sg_pbvh_grids_sync_host(PBVH *p) {
   if (!p || p->type != PBVH_GRIDS || !p->gd) return sg_set_error("not a PBVH over grids on the device");
   const CCGKey &key = p->gridkey;
   const size_t E = (size_t)p->gd->E;
+  bool whole = p->totgrid > 0;  // the grids one after the other in memory
+  for (int g = 1; g < p->totgrid && whole; g++)
+    whole = (unsigned char *)p->grids[g] == (unsigned char *)p->grids[0] + (size_t)g * key.grid_area * key.elem_size;
+  if (whole) {
+    const int rc = sg_grids_download_packed(p, p->grids[0]);
+    if (rc <= 0) return rc;
+  }
   std::vector<float> co(3 * E), no(key.has_normals ? 3 * E : 0), mk(key.has_mask ? E : 0);
   if (sg_grids_download(p, co.data(), key.has_normals ? no.data() : nullptr, key.has_mask ? mk.data() : nullptr))
     return -1;

@@ -98,6 +98,7 @@ struct SgGridDev {
   int *leaf_gmark = nullptr;  // [L] serial of the last dab that gathered the leaf
   int4 *face_leaf = nullptr;  // [F] the leaves of the face's grids
   int2 *grid_pl = nullptr;    // [G] by grid id: position, leaf
+  unsigned *pack = nullptr;   // the elements in the caller's layout (first read)
   long long *lines = nullptr; // counter lines of the per-face kernels
   int maxn = 0;               // most grids of a face
   int face_lds = 0;           // LDS bytes of the per-face dab kernel; 0: the faces do not fit
@@ -124,6 +125,7 @@ int sg_grids_enqueue_update_normals(PBVH *p, const int *leaves_dev, int n);
 int sg_grids_enqueue_refit(PBVH *p, const int *leaves_dev, int n, int set_orig);
 int sg_grids_enqueue_flush(PBVH *p);  // internal nodes above the leaves refit since the last flush
 int sg_grids_download(PBVH *p, float *co, float *no, float *mask);  // element order of the grids (by grid id)
+int sg_grids_download_packed(PBVH *p, void *out);
 int sg_grids_upload(PBVH *p, const float *co, const float *no, const float *mask);
 int sg_grids_read_boxes(PBVH *p, float *leaf_bb, float *node_bb);
 int sg_grids_read_stamps(PBVH *p, int *stamp);
