@@ -206,6 +206,7 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
       }
       d.ctr_next[lane] = 0;
     }
+    if (lane < 2 * SG_LRN_LINES) d.lrn_next[(lane / 2) * SG_LRN_LINE + lane % 2] = 0;
     if (lane == 0 && d.seq) d.seq[0] += 1;  // this dab's stamp for the later kernels
     if (lane == 0 && undo_active(d)) atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], SG_NGATHER_UNDO);
     return;
@@ -259,8 +260,9 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
 // halt flag, and take the stamps dstamp[0] + number for them, past every earlier one (the
 // 32-bit stamps wrap) and leaving the stamp before the first one unused (no staged value
 // belongs to "the launch before" it).
-__global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp, long long *ch_ctr, int n) {
+__global__ void k_clear_ctr(long long *ctr, int *halt, int *dstamp, long long *ch_ctr, long long *lrn, int n) {
   if (threadIdx.x < 2 * SG_CTR_COUNT) ctr[threadIdx.x] = 0;
+  if (threadIdx.x < 4 * SG_LRN_LINES) lrn[(threadIdx.x / 2) * SG_LRN_LINE + threadIdx.x % 2] = 0;
   if (threadIdx.x == 0) halt[0] = 0;
   if (dstamp) {
     for (int i = threadIdx.x; i < 3 * SG_CH_SEG * SG_CH_CTR; i += blockDim.x) ch_ctr[i] = 0;
@@ -1834,6 +1836,7 @@ SgDevView sg_view_of(SgDev &d, bool respect_hide, bool halt_live) {
   v.aff_cnt = d.aff_cnt;
   v.aff_shift = d.aff_shift;
   v.prev_cuts = d.prev_cuts;
+  v.lrn = v.lrn_next = d.lrn;
   v.ctr = d.ctr;
   v.ctr_next = d.ctr + SG_CTR_COUNT;
   v.cut_touch = d.cut_touch;
@@ -1966,7 +1969,7 @@ int sg_enqueue_clear_ctr(PBVH *p, int nlaunch) {
   p->fused_pending = p->chain_live = false;  // (a failed enqueue may have left them set)
   p->ch_ss = 0;
   hipLaunchKernelGGL(k_clear_ctr, dim3(1), dim3(128), 0, p->stream, p->d.ctr, p->d.halt, p->d.dstamp, p->d.ch_ctr,
-                     nlaunch);
+                     p->d.lrn, nlaunch);
   return sg_check_hip(hipGetLastError(), "clear launch");
 }
 
@@ -2005,6 +2008,8 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
   SgDevView v = sg_view(p);
   v.ctr = p->d.ctr + (size_t)(serial & 1) * SG_CTR_COUNT;
   v.ctr_next = p->d.ctr + (size_t)((serial + 1) & 1) * SG_CTR_COUNT;
+  v.lrn = p->d.lrn + (size_t)(serial & 1) * SG_LRN_LINES * SG_LRN_LINE;
+  v.lrn_next = p->d.lrn + (size_t)((serial + 1) & 1) * SG_LRN_LINES * SG_LRN_LINE;
   hipStream_t s = p->stream;
   const int G = p->grid_wg;
   const int GB = p->grid_brush > 0 ? p->grid_brush : G;

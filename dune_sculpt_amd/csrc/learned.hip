@@ -395,72 +395,200 @@ __device__ __forceinline__ BrushIn learned_tile_load(const SgDevView &d, const S
   return in;
 }
 
+// A workgroup per 16-vertex tile (LRN_DSLOTS per gathered leaf).  Bound by its chain of
+// dependent loads and arithmetic on a few hundred tiles, so the tile is spread over lanes:
+// the first wave computes the features with four lanes a vertex (two neighbours each), then
+// each wave holds a quarter of the hidden columns, its weight fragments in registers.  Same
+// products and sums in the same order as learned_eval.  A wave per tile, a lane per vertex,
+// spent 5.8 us on the features and 3.0 on the network and the kernel took 14.7 us (1050
+// affected vertices, 37 leaves); now 8.7.
 __global__ __launch_bounds__(LRN_THREADS) void k_brush_learned(SgDevView d, SgDabK k, const float *curve,
                                                                SgMlpView m, const float *place) {
-  __shared__ MlpLds s;
-  __shared__ __align__(16) uint16_t bufA[LRN_WAVES][LRN_ROWS * MLP_ST];
-  __shared__ __align__(16) uint16_t bufB[LRN_WAVES][LRN_ROWS * MLP_ST];
-  __shared__ __align__(16) float sOut[LRN_WAVES][LRN_ROWS * 4];
-  __shared__ unsigned long long s_acc[3];
+  __shared__ __align__(16) uint16_t bufA[LRN_ROWS * MLP_ST];
+  __shared__ __align__(16) uint16_t bufB[LRN_ROWS * MLP_ST];
+  __shared__ __align__(16) float sOut[LRN_ROWS * 4];
   if (d.halt && d.halt[0]) return;
   sg_place(k, place);
-  const int w = threadIdx.x / 64, lane = __lane_id();
-  const int gw = blockIdx.x * LRN_WAVES + w;
-  const int nw = gridDim.x * LRN_WAVES;
-  // the wave's first leaf range, loaded beside the counter (speculatively: any index
-  // below L is inside the gathered-leaf list; the loop uses it only when it is live)
-  const int2 vr0 = gw / LRN_DSLOTS < d.L ? d.gl_v[gw / LRN_DSLOTS] : make_int2(0, 0);
+  const int w = threadIdx.x / SG_WAVE, lane = lane_id();
+  const int r = lane & 15, p = lane >> 4, kq = p * 4;
+  // the first leaf range beside the counter (any index below L is inside the list)
+  const int2 vr0 = d.gl_v[min((int)blockIdx.x / LRN_DSLOTS, d.L - 1)];
   const long long ng_ctr = d.ctr[SG_CTR_NGATHER];
   const int nitems = LRN_DSLOTS * (int)ng_ctr;
-  if (blockIdx.x * LRN_WAVES >= nitems) return;  // whole block idle: skip the weight fill
-  // the first tile's loads go out before the weight fill, so both share one round trip
-  const int base0 = vr0.x + (gw % LRN_DSLOTS) * LRN_ROWS;
-  float nx0 = 0.0f, ny0 = 0.0f, nz0 = 0.0f;
+  if ((int)blockIdx.x >= nitems) return;
+  // every wave loads the tile's vertices (lanes r, r + 16, ... the same one), so that the
+  // skip of tiles with no affected vertex is the workgroup's
+  auto tile = [&](int2 vr, int base, BrushIn &in, float &nx, float &ny, float &nz) {
+    const int v = base + r, vend = min(vr.y, base + LRN_ROWS), vc = min(v, vend - 1);
+    in = brush_load(d, k, v, vend, true);
+    nx = d.nx[vc];
+    ny = d.ny[vc];
+    nz = d.nz[vc];
+  };
+  const int base0 = vr0.x + ((int)blockIdx.x % LRN_DSLOTS) * LRN_ROWS;
   BrushIn in0{};
-  if (gw < nitems && base0 < vr0.y) in0 = learned_tile_load(d, k, base0, vr0.y, lane, nx0, ny0, nz0);
-  mlp_lds_load<LRN_THREADS>(s, m);
-  if (threadIdx.x < 3) s_acc[threadIdx.x] = 0ull;
-  __syncthreads();
+  float nx0 = 0.0f, ny0 = 0.0f, nz0 = 0.0f;
+  if (base0 < vr0.y) tile(vr0, base0, in0, nx0, ny0, nz0);
+  // weight fragments and biases of the wave's columns, normalisation of the lane's features
+  const uint16_t *w1t = m.wb, *w2t = w1t + 64 * 32, *w3t = w2t + 64 * 64;
+  const int col = w * 16 + r;
+  sg_short4 f1[2], f2[4], f3[4];
+#pragma unroll
+  for (int kt = 0; kt < 2; kt++) f1[kt] = *(const sg_short4 *)&w1t[col * 32 + kt * 16 + kq];
+#pragma unroll
+  for (int kt = 0; kt < 4; kt++) {
+    f2[kt] = *(const sg_short4 *)&w2t[col * 64 + kt * 16 + kq];
+    f3[kt] = *(const sg_short4 *)&w3t[r * 64 + kt * 16 + kq];
+  }
+  const float b1 = m.bias[col], b2 = m.bias[64 + col], b3 = m.bias[128 + r];
+  float mu[7], iv[7];
+#pragma unroll
+  for (int i = 0; i < 7; i++) {
+    const int q = i < 6 ? 6 * p + i : 24 + p;
+    mu[i] = m.norm[q];
+    iv[i] = m.norm[28 + q];
+  }
+  const float sc0 = m.norm[56], sc1 = m.norm[57], sc2 = m.norm[58];
   const int stamp = d.seq[0];
   long long esum = 0;
   int nood = 0, naff = 0;
-  if (ng_ctr & SG_NGATHER_UNDO) {
+  if ((ng_ctr & SG_NGATHER_UNDO) && w == 0) {
     // an undo step is open: the learned brush writes the shadow copy and leaves the
     // positions alone (k_post_learned copies or redoes them), so each leaf is saved
-    // from the positions by the wave of its first slot, whatever the other slots write
-    for (int it = gw; it < nitems; it += nw)
+    // from the positions by the workgroup of its first slot, whatever the others write
+    for (int it = blockIdx.x; it < nitems; it += gridDim.x)
       if (it % LRN_DSLOTS == 0)
         undo_save_leaf(d, d.gathered[it / LRN_DSLOTS], d.gl_v[it / LRN_DSLOTS], d.px, d.py, d.pz);
   }
-  for (int it = gw; it < nitems; it += nw) {
-    int2 vr = vr0;
-    if (it != gw) vr = d.gl_v[it / LRN_DSLOTS];
+  for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+    const int2 vr = it == (int)blockIdx.x ? vr0 : d.gl_v[it / LRN_DSLOTS];
     for (int base = vr.x + (it % LRN_DSLOTS) * LRN_ROWS; base < vr.y; base += LRN_DSLOTS * LRN_ROWS) {
-      float nx = nx0, ny = ny0, nz = nz0;
       BrushIn in = in0;
-      if (base != base0 || it != gw) in = learned_tile_load(d, k, base, vr.y, lane, nx, ny, nz);
-      if (__ballot(in.aff) == 0ull) continue;
-      const int v = base + lane;
-      learned_eval(d, k, curve, m, s, bufA[w], bufB[w], sOut[w], v, in, nx, ny, nz, esum, nood);
-      if (in.aff) {
+      float nx = nx0, ny = ny0, nz = nz0;
+      if (base != base0 || it != (int)blockIdx.x) tile(vr, base, in, nx, ny, nz);
+      if (__ballot(in.aff) == 0ull) continue;  // the same in every wave
+      float R[9], h = 0.0f;
+      bool ok = true;
+      if (w == 0) {
+        // features (learned_features): this lane's neighbours 2p and 2p + 1
+        const int deg = in.aff ? in.vv.y - in.vv.x : 0, j0 = 2 * p;
+        const int u0 = j0 < deg ? d.vv_idx[in.vv.x + j0] : -1, u1 = j0 + 1 < deg ? d.vv_idx[in.vv.x + j0 + 1] : -1;
+        const int c0 = max(u0, 0), c1 = max(u1, 0);
+        const float ax = d.px[c0], ay = d.py[c0], az = d.pz[c0], bx = d.px[c1], by = d.py[c1], bz = d.pz[c1];
+        float e[6] = {ax - in.x, ay - in.y, az - in.z, bx - in.x, by - in.y, bz - in.z};
+        if (u0 < 0) e[0] = e[1] = e[2] = 0.0f;
+        if (u1 < 0) e[3] = e[4] = e[5] = 0.0f;
+        const float l0 = sqrtf(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]);
+        const float l1 = sqrtf(e[3] * e[3] + e[4] * e[4] + e[5] * e[5]);
+        float fade = 0.0f;
+        if (in.aff) fade = k.bstr * (sg_falloff(k, curve, sqrtf(in.d2)) * (1.0f - in.mk));
+        const int mm = deg < 8 ? deg : 8;
+        float len[8];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          len[2 * q] = __shfl(l0, r + 16 * q);
+          len[2 * q + 1] = __shfl(l1, r + 16 * q);
+        }
+        float hs = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          if (j < mm) hs += len[j];
+        h = mm > 0 ? hs / (float)mm : 0.0f;
+        const float ex = __shfl(e[0], r), ey = __shfl(e[1], r), ez = __shfl(e[2], r);
+        const float en = ex * nx + ey * ny + ez * nz;
+        float t1x = ex - en * nx, t1y = ey - en * ny, t1z = ez - en * nz;
+        const float t1l = sqrtf(t1x * t1x + t1y * t1y + t1z * t1z);
+        ok = deg >= 3 && deg <= 8 && h > 0.0f && t1l > 1e-6f * h;
+        const float itl = ok ? 1.0f / t1l : 0.0f;
+        t1x *= itl;
+        t1y *= itl;
+        t1z *= itl;
+        const float t2x = ny * t1z - nz * t1y, t2y = nz * t1x - nx * t1z, t2z = nx * t1y - ny * t1x;
+        R[0] = t1x;
+        R[1] = t1y;
+        R[2] = t1z;
+        R[3] = t2x;
+        R[4] = t2y;
+        R[5] = t2z;
+        R[6] = nx;
+        R[7] = ny;
+        R[8] = nz;
+        const float ih = ok ? 1.0f / h : 0.0f;
+        float ft[7];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+          ft[3 * j + 0] = (t1x * e[3 * j] + t1y * e[3 * j + 1] + t1z * e[3 * j + 2]) * ih;
+          ft[3 * j + 1] = (t2x * e[3 * j] + t2y * e[3 * j + 1] + t2z * e[3 * j + 2]) * ih;
+          ft[3 * j + 2] = (nx * e[3 * j] + ny * e[3 * j + 1] + nz * e[3 * j + 2]) * ih;
+        }
+        const float omf = 1.0f - fade;
+        ft[6] = p == 0 ? (float)deg * 0.125f : p == 1 ? fade : p == 2 ? fade * fade : 1.0f - (omf * omf) * (omf * omf);
+        uint32_t b[7];
+#pragma unroll
+        for (int i = 0; i < 7; i++) b[i] = sg_f2bf(in.aff ? (ft[i] - mu[i]) * iv[i] : 0.0f);
+        uint32_t *row = (uint32_t *)&bufA[r * MLP_ST];
+#pragma unroll
+        for (int i = 0; i < 3; i++) row[3 * p + i] = b[2 * i] | (b[2 * i + 1] << 16);
+        bufA[r * MLP_ST + 24 + p] = (uint16_t)b[6];
+        bufA[r * MLP_ST + 28 + p] = 0;
+      }
+      __syncthreads();
+      sg_float4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const sg_short4 *)&bufA[r * MLP_ST + kt * 16 + kq], f1[kt], acc,
+                                                        0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) bufB[(kq + i) * MLP_ST + col] = sg_f2bf(sg_silu(acc[i] + b1));
+      __syncthreads();
+      acc = sg_float4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const sg_short4 *)&bufB[r * MLP_ST + kt * 16 + kq], f2[kt], acc,
+                                                        0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) bufA[(kq + i) * MLP_ST + col] = sg_f2bf(sg_silu(acc[i] + b2));
+      __syncthreads();
+      if (w != 0) continue;  // (the others wait at the next tile's first barrier)
+      sg_float4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int kt = 0; kt < 4; kt++)
+        o = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*(const sg_short4 *)&bufA[r * MLP_ST + kt * 16 + kq], f3[kt], o, 0,
+                                                      0, 0);
+      if (r < 4) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) sOut[(kq + i) * 4 + r] = o[i] + b3;
+      }
+      wave_lds_sync();
+      if (p == 0 && in.aff) {
+        const int v = base + r;
+        const float o0 = sOut[r * 4] * sc0 * h, o1 = sOut[r * 4 + 1] * sc1 * h, o2 = sOut[r * 4 + 2] * sc2 * h;
+        const float dx = R[0] * o0 + R[3] * o1 + R[6] * o2;
+        const float dy = R[1] * o0 + R[4] * o1 + R[7] * o2;
+        const float dz = R[2] * o0 + R[5] * o1 + R[8] * o2;
+        d.qx[v] = in.x + dx;
+        d.qy[v] = in.y + dy;
+        d.qz[v] = in.z + dz;
+        const float rel2 = (dx * dx + dy * dy + dz * dz) / k.r2;
+        if (!ok || !(rel2 < 1.0f))  // out of range, NaN or a displacement beyond r
+          nood++;
+        else
+          esum += __double2ll_rn((double)rel2 * 4294967296.0);  // 2^32: rel2 < 1, no overflow below 2^31 vertices
         d.vstamp[v] = stamp;
         naff++;
       }
+      wave_lds_sync();
     }
   }
+  if (w != 0) return;
   esum = wave_sum_ll(esum);
   nood = wave_sum_i(nood);
   naff = wave_sum_i(naff);
   if (lane == 0 && naff) {
-    atomicAdd(&s_acc[0], (unsigned long long)esum);
-    atomicAdd(&s_acc[1], (unsigned long long)nood);
-    atomicAdd(&s_acc[2], (unsigned long long)naff);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0 && s_acc[2]) {
-    atomicAdd((unsigned long long *)&d.ctr[SG_CTR_LERR], s_acc[0]);
-    atomicAdd((unsigned long long *)&d.ctr[SG_CTR_LOOD], s_acc[1]);
-    atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NAFF], s_acc[2]);
+    // 16 counter lines (one line takes an atomic every 12 ns); k_post_learned adds them up
+    unsigned long long *c = (unsigned long long *)d.lrn + (blockIdx.x % SG_LRN_LINES) * SG_LRN_LINE;
+    atomicAdd(c, (unsigned long long)esum);
+    atomicAdd(c + 1, ((unsigned long long)nood << 32) + (unsigned long long)naff);
   }
 }
 
@@ -579,15 +707,16 @@ __global__ __launch_bounds__(256) void k_post_learned(SgDevView d, SgDevView dq,
   const int g0 = gw / 3, part0 = gw % 3;
   const int2 vr0 = g0 < d.L ? d.gl_v[g0] : make_int2(0, 0);
   const int stamp = d.seq[0];
-  const int na = (int)d.ctr[SG_CTR_NAFF];
+  const long long la = lane < SG_LRN_LINES ? d.lrn[lane * SG_LRN_LINE] : 0;
+  const long long lb = lane < SG_LRN_LINES ? d.lrn[lane * SG_LRN_LINE + 1] : 0;
   const int ng = (int)d.ctr[SG_CTR_NGATHER];
-  const long long es = d.ctr[SG_CTR_LERR];
-  const long long nood = d.ctr[SG_CTR_LOOD];
   const int v0 = vr0.x + part0 * SG_WAVE + lane;
   const bool pre = part0 < 2 && v0 < vr0.y;
   const int st0 = pre ? d.vstamp[v0] : 0;
   int2 vt0 = make_int2(0, 0);
   if (pre) vt0 = make_int2(d.vt_off[v0], d.vt_off[v0 + 1]);
+  const long long es = wave_sum_ll(la), cnt = wave_sum_ll(lb), nood = cnt >> 32;
+  const int na = (int)(cnt & 0xffffffffll);
   // error estimate: alpha * RMS(|d| / r), alpha = held-out RMS error / RMS displacement
   const double rms = na > 0 ? sqrt((double)es / 4294967296.0 / (double)na) : 0.0;
   const bool accept = nood == 0 && (double)alpha * rms <= (double)tol;
@@ -620,6 +749,9 @@ __global__ __launch_bounds__(256) void k_post_learned(SgDevView d, SgDevView dq,
     }
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
+    d.ctr[SG_CTR_NAFF] = na;
+    d.ctr[SG_CTR_LERR] = es;
+    d.ctr[SG_CTR_LOOD] = nood;
     if (accept)
       d.ctr[SG_CTR_LACC] = 1;
     else if (d.halt)
@@ -1155,9 +1287,9 @@ int sg_mfma_probe(const uint16_t *A, const uint16_t *B, float *D) {
 // ---- launch helpers used by the dab path (api.cpp / kernels.hip) ----
 int sg_enqueue_learned_brush(PBVH *p, const SgDevView &v, const SgDabK &k, const float *curve, SgMlp *m,
                              const float *place) {
-  // at least 512 workgroups (2048 waves): a wave per (leaf, slot) for up to 256 gathered
-  // leaves, so no wave runs two tiles' load chains back to back
-  const int G = std::max(512, p->grid_brush > 0 ? p->grid_brush : p->grid_wg);
+  // at least 1024 workgroups: one per (leaf, slot) for up to 128 gathered leaves, so that
+  // none runs two tiles' chains back to back
+  const int G = std::max(1024, p->grid_brush > 0 ? p->grid_brush : p->grid_wg);
   hipLaunchKernelGGL(k_brush_learned, dim3(G), dim3(LRN_THREADS), 0, p->stream, v, k, curve, sg_mlp_view(m),
                      place);
   return sg_check_hip(hipGetLastError(), "learned brush launch");

@@ -1047,6 +1047,7 @@ void sg_build_device(PBVH *p, const float *co) {
   alloc_fill(&d.aff_fade, na, 0, s);
   alloc_fill(&d.aff_cnt, std::max(L, 1), 0, s);
   alloc_fill(&d.ctr, 2 * SG_CTR_COUNT, 0, s);
+  alloc_fill(&d.lrn, 2 * SG_LRN_LINES * SG_LRN_LINE, 0, s);
   alloc_fill(&d.halt, 4, 0, s);
   alloc_fill(&d.seq, 1, 0, s);
   alloc_fill(&d.vstamp, V, 0xFF, s);  // -1: never a dab's stamp (stamps start at 1)
@@ -1078,7 +1079,7 @@ void sg_free_device(PBVH *p) {
                   d.cut_bb, d.cut_obb, d.cut_flags, d.cut_node, d.cut_lbeg, d.cut_lend,
                   d.sub_off, d.sub_tab, d.top_tab_n, d.top_tab, d.cut_dirty, d.vhide, d.vmark,
                   d.gathered, d.gl_v, d.gl_s, d.aff_v, d.aff_vt, d.aff_vv, d.aff_fade, d.aff_cnt,
-                  d.prev_cuts, d.cut_touch, d.halt, d.seq, d.vstamp, d.ctr, d.err, d.vperm_old, d.stamp_v, d.stamp_v2, d.stamp_t,
+                  d.prev_cuts, d.cut_touch, d.halt, d.seq, d.vstamp, d.ctr, d.lrn, d.err, d.vperm_old, d.stamp_v, d.stamp_v2, d.stamp_t,
                   d.stamp_a, d.curve, d.log, d.ltri, d.leaf_toff, d.tri_poly, d.node_parent, d.leaf_node,
                   d.ray_in, d.ray_out, d.place, d.place_rays, d.rl_list, d.rl_args,
                   d.draw_dirty, d.draw_tri, d.draw_off, d.draw_leaf, d.draw_fset, d.draw_poly_off,

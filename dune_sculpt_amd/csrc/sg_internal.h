@@ -122,6 +122,7 @@ struct SgDev {
   int aff_shift = 6;
   int *prev_cuts = nullptr;     // [C] cuts refit by the previous dab (+ count in ctr)
   long long *ctr = nullptr;     // two counter sets (even / odd dabs), see SG_CTR_*
+  long long *lrn = nullptr;  // learned Smooth counter lines, two sets
   int *err = nullptr;           // device error word
   int *vperm_old = nullptr;     // [V] new -> old id (device copy)
   int *stamp_v = nullptr, *stamp_v2 = nullptr, *stamp_t = nullptr, *stamp_a = nullptr; // stats mode

@@ -15,6 +15,9 @@ enum {
   SG_CTR_LACC = 17,   // learned Smooth: 1 when the dab was accepted
 };
 
+#define SG_LRN_LINES 16  // lines of the learned brush's counters: [0] sum as SG_CTR_LERR, [1] affected, bit 32 on: out of range
+#define SG_LRN_LINE 16   // long longs per line
+
 // High half of the gathered-leaf counter: an undo step is open.  k_search sets it for
 // the brush kernels, which load that counter anyway (a load of its own would add a
 // dependent memory round trip to their start); the count is the low half.
@@ -75,6 +78,7 @@ struct SgDevView {
   int *halt;
   int *seq, *vstamp;
   long long *ctr, *ctr_next;
+  long long *lrn, *lrn_next;  // learned Smooth: counter lines of this dab and the next
   const int *vperm_old;
   int *stamp_v, *stamp_v2, *stamp_t, *stamp_a;
   // fused dabs: per-leaf halos, and the chain's lists, stamps, counters and staged results
