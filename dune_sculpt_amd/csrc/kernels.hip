@@ -894,7 +894,6 @@ struct SgChainArgs {
   int nf, ns, nc;            // F, S, C blocks
   int cap, fcap;             // LDS: locals, faces
   int has_next, has_prev;
-  int direct;                // write the positions to the mesh's (qx, qy, qz) of this view as well (see there)
   int last;                  // the chain ends here: keep the affected list and the gathered leaves for the host
   long long *log;            // per-dab counter rows, or null
 };
@@ -990,11 +989,15 @@ __device__ __forceinline__ long long chain_counter(const long long *lines, int i
   return t;
 }
 
-template <int LPT>
+// PLACED: the dab's centre comes from `place`, and its positions go to the mesh's (qx, qy, qz)
+// of this view as well (see sg_enqueue_dab).  An instance of its own: the same tests at run
+// time cost the strokes that are not placed 3 percent (k in vector registers).
+// SMOOTH: a Smooth dab; the others have no Jacobi steps and load no neighbour rows.
+template <int LPT, bool SMOOTH, bool PLACED>
 __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK k, SgDabK kn, const float *curve,
                                                             SgChainArgs ca, const float *place) {
   if (d.halt && d.halt[0]) return;
-  sg_place(k, place);
+  if (PLACED) sg_place(k, place);
   extern __shared__ __align__(16) unsigned char fused_smem[];
   __shared__ int s_cnt, s_next;
   __shared__ int2 s_q[FUSED_THREADS];
@@ -1044,16 +1047,16 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
   const int4 ra0 = recs[2 * gc], rb0 = recs[2 * gc + 1];
   const int ng = (int)lines[seg * SG_CH_CTR];
   const int gstamp = d.dstamp[0] + ls, stamp = d.dstamp[0] + ss;
-  const bool undo = undo_active(d) && !ca.cont_in;
+  const bool cont_in = SMOOTH && ca.cont_in, cont_out = SMOOTH && ca.cont_out;
+  const bool undo = undo_active(d) && !cont_in;
   if (g0 == 0 && tid == 0) d.pend[(ls & 1) * SG_CH_SEG + seg] = ng;  // what the copy-back takes
   const float4 *stp = d.st_pos + (size_t)((ss + 1) & 1) * d.V, *stn = d.st_nor + (size_t)((ss + 1) & 1) * d.V;
   float4 *wtp = d.st_pos + (size_t)(ss & 1) * d.V, *wtn = d.st_nor + (size_t)(ss & 1) * d.V;
   const bool next_draw = ca.has_next && kn.tool == SG_TOOL_DRAW;
-  const bool smooth = k.tool == SG_TOOL_SMOOTH;
-  const int K = smooth ? ca.iters : 0;
+  const int K = SMOOTH ? ca.iters : 0;
   // Draw offset: (normalize(area) * r) * bstrength
   float ox = 0.0f, oy = 0.0f, oz = 0.0f;
-  if (k.tool == SG_TOOL_DRAW) {
+  if (!SMOOTH && k.tool == SG_TOOL_DRAW) {
     long long sx = 0, sy = 0, sz = 0;
 #pragma unroll
     for (int q = 0; q < SG_CH_AREA; q++) {
@@ -1101,7 +1104,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       const bool ext = i >= nu && i < nloc, inner = i < ninner;
       // (id, owner) as one 64-bit load, so both halves stay where they are issued
       const long long e = *(const long long *)(d.hl_v + (ext ? ext_off + i - nu : 0));
-      const int b = d.hl_nboff[inner ? nb_blk + i : 0], en = d.hl_nboff[inner ? nb_blk + i + 1 : 0];
+      int b = 0, en = 0;
+      if (SMOOTH) {
+        b = d.hl_nboff[inner ? nb_blk + i : 0];
+        en = d.hl_nboff[inner ? nb_blk + i + 1 : 0];
+      }
       int id = (int)e, ow = (int)(e >> 32);
       if (!ext) {
         id = -1;
@@ -1130,7 +1137,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     // level 3
     // stand-ins keep the loads unconditional without new traffic: a tool that needs no
     // normals, or a mesh with no mask or hidden vertices, reads the position lines again
-    const bool need_n = k.tool == SG_TOOL_INFLATE || next_draw, need_s = need_n || ca.cont_in;
+    const bool need_n = k.tool == SG_TOOL_INFLATE || next_draw, need_s = need_n || cont_in;
     const float *mp = d.mask ? d.mask : d.px;
     const int *hp = hide ? d.vhide : (const int *)d.px;
     const float *nxp = need_n ? d.nx : d.px, *nyp = need_n ? d.ny : d.py, *nzp = need_n ? d.nz : d.pz;
@@ -1165,8 +1172,10 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       mk[j] = d.mask ? m : 0.0f;
       hid[j] = hide && hv != 0;
       own[j] = owner[j] < 0 || gs == gstamp;  // its leaf was gathered by this search
+      if (SMOOTH) {
 #pragma unroll
-      for (int q = 0; q < FUSED_ROW; q++) nb[j][q] = d.hl_nbl[nbb[j] + q < nbe[j] ? nbb[j] + q : 0];
+        for (int q = 0; q < FUSED_ROW; q++) nb[j][q] = d.hl_nbl[nbb[j] + q < nbe[j] ? nbb[j] + q : 0];
+      }
     }
     unsigned short ti0[FUSED_ROW];  // the first incidences' local faces
 #pragma unroll
@@ -1183,12 +1192,14 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       const float d2 = dx * dx + dy * dy + dz * dz;
       aff[j] = vid[j] >= 0 && own[j] && d2 <= k.r2 && !hid[j];
       fade[j] = 0.0f;
-      if (ca.cont_in) {  // affected by the launch before, which staged its Smooth factor
+      if (cont_in) {  // affected by the launch before, which staged its Smooth factor
         aff[j] = vid[j] >= 0 && staged[j];
         fade[j] = sfade[j];
       } else if (aff[j]) {
         const float f = sg_falloff(k, curve, sqrtf(d2)) * (1.0f - mk[j]);
-        if (k.tool == SG_TOOL_DRAW) {
+        if (SMOOTH) {
+          fade[j] = k.bstr * f;
+        } else if (k.tool == SG_TOOL_DRAW) {
           x[j] = x[j] + ox * f;
           y[j] = y[j] + oy * f;
           z[j] = z[j] + oz * f;
@@ -1197,13 +1208,11 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
           x[j] = x[j] + nxv[j] * sc;
           y[j] = y[j] + nyv[j] * sc;
           z[j] = z[j] + nzv[j] * sc;
-        } else if (k.tool == SG_TOOL_GRAB) {
+        } else {  // Grab
           fade[j] = k.bstr * f;
           x[j] = x[j] + k.gx * fade[j];
           y[j] = y[j] + k.gy * fade[j];
           z[j] = z[j] + k.gz * fade[j];
-        } else {
-          fade[j] = k.bstr * f;
         }
       }
       if (i < nloc) S[i] = make_float4(x[j], y[j], z[j], 0.0f);
@@ -1226,21 +1235,23 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
         if (i < nact) {
           if (aff[j]) {
             const int cnt = nbe[j] - nbb[j];
+            // the row's reads ahead of its sum (a read under a branch each waits for it; the
+            // vertex itself stands in past the row's end): 0.6 us a step before, 0.45 now
+            float4 pu[FUSED_ROW];
+#pragma unroll
+            for (int q = 0; q < FUSED_ROW; q++) pu[q] = X[q < cnt ? nb[j][q] : i];
             float sx = 0.0f, sy = 0.0f, sz = 0.0f;
 #pragma unroll
             for (int q = 0; q < FUSED_ROW; q++) {
-              if (q < cnt) {
-                const float4 pu = X[nb[j][q]];
-                sx = sx + pu.x;
-                sy = sy + pu.y;
-                sz = sz + pu.z;
-              }
+              sx = q < cnt ? sx + pu[q].x : sx;
+              sy = q < cnt ? sy + pu[q].y : sy;
+              sz = q < cnt ? sz + pu[q].z : sz;
             }
             for (int q = FUSED_ROW; q < cnt; q++) {
-              const float4 pu = X[d.hl_nbl[nbb[j] + q]];
-              sx = sx + pu.x;
-              sy = sy + pu.y;
-              sz = sz + pu.z;
+              const float4 pv = X[d.hl_nbl[nbb[j] + q]];
+              sx = sx + pv.x;
+              sy = sy + pv.y;
+              sz = sz + pv.z;
             }
             if (cnt > 0) {
               const float avx = sx * inv[j], avy = sy * inv[j], avz = sz * inv[j];
@@ -1258,7 +1269,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     // the affected uniq vertices: normal (spec S10, incident tris in vertex->tri order),
     // position, list record
     const float4 *F = S + cur * cap;  // final positions of the locals
-    if (ca.cont_out) {  // the next launch goes on from here
+    if (cont_out) {  // the next launch goes on from here
 #pragma unroll
       for (int j = 0; j < LPT; j++) {
         const int i = tid + j * FUSED_THREADS;
@@ -1348,9 +1359,15 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       };
       if (j == 0) {
         const int cnt = qe0 - qb0;
+        float4 fn[FUSED_ROW];  // (face 0 stands in past the end)
 #pragma unroll
-        for (int q = 0; q < FUSED_ROW; q++)
-          if (q < cnt) add_face(ti0[q]);
+        for (int q = 0; q < FUSED_ROW; q++) fn[q] = Sfn[q < cnt ? ti0[q] : 0];
+#pragma unroll
+        for (int q = 0; q < FUSED_ROW; q++) {
+          ax = q < cnt ? ax + fn[q].x : ax;
+          ay = q < cnt ? ay + fn[q].y : ay;
+          az = q < cnt ? az + fn[q].z : az;
+        }
         for (int q = qb0 + FUSED_ROW; q < qe0; q++) add_face(d.hl_ti[q]);
       } else {  // leaves of more than FUSED_THREADS uniq vertices
         const int qb = d.vt_off[v], qe = d.vt_off[v + 1];
@@ -1359,7 +1376,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       sg_normalize(ax, ay, az);
       wtp[v] = make_float4(x[j], y[j], z[j], __int_as_float(stamp));
       wtn[v] = make_float4(ax, ay, az, 0.0f);
-      if (ca.direct) {
+      if (PLACED) {
         d.qx[v] = x[j];
         d.qy[v] = y[j];
         d.qz[v] = z[j];
@@ -2074,20 +2091,18 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
       ca.cont_out = q + 1 < fs.launches ? 1 : 0;
       ca.has_next = has_next && !ca.cont_out ? 1 : 0;
       ca.has_prev = prev && !ca.cont_in ? 1 : 0;
-      ca.direct = place ? 1 : 0;
       ca.last = !has_next && !ca.cont_out ? 1 : 0;
       ca.ns = ca.has_next ? leaf_blocks : 0;
       ca.nc = chained && !ca.cont_in ? 128 : 0;
       ProfScope ps(p, SG_K_BRUSH);
       const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(FUSED_THREADS);
-      if (fs.lpt == 1)
-        SG_LAUNCH(ps, k_dab_chain<1>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
-      else if (fs.lpt == 2)
-        SG_LAUNCH(ps, k_dab_chain<2>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
-      else if (fs.lpt == 3)
-        SG_LAUNCH(ps, k_dab_chain<3>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
-      else
-        SG_LAUNCH(ps, k_dab_chain<4>, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
+      using ChainKernel = void (*)(SgDevView, SgDabK, SgDabK, const float *, SgChainArgs, const float *);
+#define SG_CHAIN_LPT(S, P) {k_dab_chain<1, S, P>, k_dab_chain<2, S, P>, k_dab_chain<3, S, P>, k_dab_chain<4, S, P>}
+      static const ChainKernel kernels[2][2][4] = {{SG_CHAIN_LPT(false, false), SG_CHAIN_LPT(false, true)},
+                                                   {SG_CHAIN_LPT(true, false), SG_CHAIN_LPT(true, true)}};
+#undef SG_CHAIN_LPT
+      const ChainKernel kern = kernels[k.tool == SG_TOOL_SMOOTH ? 1 : 0][place ? 1 : 0][fs.lpt - 1];
+      SG_LAUNCH(ps, kern, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
     }
     p->chain_live = has_next;
     p->fused_pending = true;
