@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -869,7 +870,7 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // vertices as the affected ones.  Smooth(8) on 655 k vertices, 60 dabs: 2.65 ms with a
 // kernel per step, 1.35 as two launches per dab.
 // ---------------------------------------------------------------------------
-#define FUSED_THREADS 256
+#define FUSED_THREADS 256  // twice that for Smooth dabs whose halos have more locals
 #define FUSED_LEAD 256  // F blocks started before the S and C blocks: more leaves than most dabs gather
 #define FUSED_ROW 8  // neighbour / incidence entries per local held in registers
 
@@ -882,7 +883,6 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // after which the brush, the Jacobi steps, the normals and the box run from LDS and
 // registers.  Rows longer than 8 entries read the rest from memory where they are used.
 #define FUSED_FPT 2              // faces per face thread whose corners load up front
-#define FUSED_FACE_THREADS 192   // the first three waves compute the face normals, the last the leaf box
 
 struct SgChainArgs {
   int ls;                    // the dab's number: lists, counters and gather stamps
@@ -993,14 +993,14 @@ __device__ __forceinline__ long long chain_counter(const long long *lines, int i
 // of this view as well (see sg_enqueue_dab).  An instance of its own: the same tests at run
 // time cost the strokes that are not placed 3 percent (k in vector registers).
 // SMOOTH: a Smooth dab; the others have no Jacobi steps and load no neighbour rows.
-template <int LPT, bool SMOOTH, bool PLACED>
-__global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK k, SgDabK kn, const float *curve,
+template <int NT, int LPT, bool SMOOTH, bool PLACED>
+__global__ __launch_bounds__(NT) void k_dab_chain(SgDevView d, SgDabK k, SgDabK kn, const float *curve,
                                                             SgChainArgs ca, const float *place) {
   if (d.halt && d.halt[0]) return;
   if (PLACED) sg_place(k, place);
   extern __shared__ __align__(16) unsigned char fused_smem[];
   __shared__ int s_cnt, s_next;
-  __shared__ int2 s_q[FUSED_THREADS];
+  __shared__ int2 s_q[NT];
   const int ls = ca.ls, ss = ca.ss;
   int g0 = (int)blockIdx.x;
   if (g0 >= ca.f0) {
@@ -1010,8 +1010,8 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       return;
     }
     if (o < ca.ns + ca.nc) {
-      chain_copy_back(d, ls - 1, ss - 1, ((o - ca.ns) * FUSED_THREADS + (int)threadIdx.x) / SG_WAVE,
-                      ca.nc * (FUSED_THREADS / SG_WAVE));
+      chain_copy_back(d, ls - 1, ss - 1, ((o - ca.ns) * NT + (int)threadIdx.x) / SG_WAVE,
+                      ca.nc * (NT / SG_WAVE));
       return;
     }
     if (o == ca.ns + ca.nc) {  // log the previous dab's counters and clear its set (dab ls + 2's)
@@ -1100,7 +1100,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     int vid[LPT], owner[LPT], nbb[LPT], nbe[LPT];
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
-      const int i = tid + j * FUSED_THREADS;
+      const int i = tid + j * NT;
       const bool ext = i >= nu && i < nloc, inner = i < ninner;
       // (id, owner) as one 64-bit load, so both halves stay where they are issued
       const long long e = *(const long long *)(d.hl_v + (ext ? ext_off + i - nu : 0));
@@ -1130,7 +1130,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     unsigned int fc0[FUSED_FPT], fc1[FUSED_FPT];
 #pragma unroll
     for (int f = 0; f < FUSED_FPT; f++) {
-      const int j = tid < FUSED_FACE_THREADS ? tid + f * FUSED_FACE_THREADS : nlt;
+      const int j = tid < (NT - SG_WAVE) ? tid + f * (NT - SG_WAVE) : nlt;
       fc0[f] = (unsigned)d.hl_nboff[j < nlt ? lt_base + 2 * j : 0];
       fc1[f] = (unsigned)d.hl_nboff[j < nlt ? lt_base + 2 * j + 1 : 0];
     }
@@ -1185,7 +1185,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     bool aff[LPT];
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
-      const int i = tid + j * FUSED_THREADS;
+      const int i = tid + j * NT;
       const float dx = k.cx - x[j];
       const float dy = k.cy - y[j];
       const float dz = k.cz - z[j];
@@ -1218,7 +1218,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       if (i < nloc) S[i] = make_float4(x[j], y[j], z[j], 0.0f);
     }
     if (tid < ns) Sshl[tid] = (unsigned short)shv0;
-    for (int i = tid + FUSED_THREADS; i < ns; i += FUSED_THREADS) Sshl[i] = d.hl_sh[sr.x + i];
+    for (int i = tid + NT; i < ns; i += NT) Sshl[i] = d.hl_sh[sr.x + i];
     __syncthreads();
     // Smooth: Jacobi step t updates the locals of rings <= K - t from step t - 1
     float inv[LPT];  // 1 / neighbour count, the same value each step
@@ -1231,7 +1231,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       float4 *W = S + (cur ^ 1) * cap;
 #pragma unroll
       for (int j = 0; j < LPT; j++) {
-        const int i = tid + j * FUSED_THREADS;
+        const int i = tid + j * NT;
         if (i < nact) {
           if (aff[j]) {
             const int cnt = nbe[j] - nbb[j];
@@ -1272,7 +1272,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     if (cont_out) {  // the next launch goes on from here
 #pragma unroll
       for (int j = 0; j < LPT; j++) {
-        const int i = tid + j * FUSED_THREADS;
+        const int i = tid + j * NT;
         if (i >= nu || !aff[j]) continue;
         wtp[vr.x + i] = make_float4(x[j], y[j], z[j], __int_as_float(stamp));
         wtn[vr.x + i] = make_float4(0.0f, 0.0f, 0.0f, fade[j]);
@@ -1282,7 +1282,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     }
     bool pass = false;
     int slot = 0;
-    if (tid < FUSED_FACE_THREADS) {
+    if (tid < (NT - SG_WAVE)) {
       // each face normal once (spec S10's face normal; faces in the tables' order)
       auto face_normal = [&](unsigned c0, unsigned c1, int j) {
         const float4 a = F[c0 & 0xffff], b = F[c0 >> 16], e = F[c1 & 0xffff];
@@ -1297,15 +1297,15 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
       };
 #pragma unroll
       for (int f = 0; f < FUSED_FPT; f++) {
-        const int j = tid + f * FUSED_FACE_THREADS;
+        const int j = tid + f * (NT - SG_WAVE);
         if (j < nlt) face_normal(fc0[f], fc1[f], j);
       }
-      for (int j = tid + FUSED_FPT * FUSED_FACE_THREADS; j < nlt; j += FUSED_FACE_THREADS)
+      for (int j = tid + FUSED_FPT * (NT - SG_WAVE); j < nlt; j += (NT - SG_WAVE))
         face_normal((unsigned)d.hl_nboff[lt_base + 2 * j], (unsigned)d.hl_nboff[lt_base + 2 * j + 1], j);
     } else {
       // meanwhile the last wave folds the leaf's box over its uniq then shared vertices
       // (contiguous runs per lane, lanes in order, as leaf_box does)
-      const int lane = tid - FUSED_FACE_THREADS;
+      const int lane = tid - (NT - SG_WAVE);
       const int tot = nu + ns, per = (tot + SG_WAVE - 1) / SG_WAVE;
       BB6 acc;
       bb_reset(acc);
@@ -1343,7 +1343,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
     // vertex->tri order), position, list record
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
-      const int i = tid + j * FUSED_THREADS;
+      const int i = tid + j * NT;
       if (i >= nu) continue;
       if (!aff[j]) {
         if (area_leaf) area_add(area, kn, x[j], y[j], z[j], nxv[j], nyv[j], nzv[j], !hid[j]);
@@ -1369,7 +1369,7 @@ __global__ __launch_bounds__(FUSED_THREADS) void k_dab_chain(SgDevView d, SgDabK
           az = q < cnt ? az + fn[q].z : az;
         }
         for (int q = qb0 + FUSED_ROW; q < qe0; q++) add_face(d.hl_ti[q]);
-      } else {  // leaves of more than FUSED_THREADS uniq vertices
+      } else {  // leaves of more than NT uniq vertices
         const int qb = d.vt_off[v], qe = d.vt_off[v + 1];
         for (int q = qb; q < qe; q++) add_face(d.hl_ti[q]);
       }
@@ -1993,7 +1993,7 @@ int sg_enqueue_clear_ctr(PBVH *p, int nlaunch) {
 // LDS and locals per thread of the chain kernel for dab k; lpt 0 when the mesh has no
 // halo tables or the dab is not one it covers.
 struct FusedShape {
-  int cap = 0, fcap = 1, lpt = 0, launches = 1;
+  int cap = 0, fcap = 1, lpt = 0, launches = 1, threads = FUSED_THREADS;
   size_t lds = 0;
 };
 static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
@@ -2006,9 +2006,16 @@ static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
   f.cap = p->d.halo_maxlocr[steps];
   f.fcap = std::max(1, p->d.halo_maxlt);
   f.lds = (size_t)f.cap * 2 * sizeof(float4) + (size_t)f.fcap * sizeof(float4) + (size_t)(p->d.leaf_maxsh + 2) * 2 + 16;
-  const int lpt = (f.cap + FUSED_THREADS - 1) / FUSED_THREADS;
+  // A Smooth dab's halo is two to three times its leaf, so 512 threads with a local each run
+  // shorter than 256 with two, while every gathered leaf has a workgroup in flight: two of 512
+  // threads fit a CU, three of 256.  60 Smooth(8) dabs over some 60 leaves: 1.26 ms with 256,
+  // 1.18 with 512; 24 mixed ones over 700 to 4000: 0.76 and 0.78.
+  const double reach = (double)k.r + 0.5 / std::sqrt(std::max(p->leaf_density, 1e-30));
+  const bool few = 3.14159 * reach * reach * p->leaf_density <= 512.0;  // leaves the dab gathers on a surface
+  f.threads = k.tool == SG_TOOL_SMOOTH && f.cap > FUSED_THREADS && few ? 2 * FUSED_THREADS : FUSED_THREADS;
+  const int lpt = (f.cap + f.threads - 1) / f.threads, most = 4 * FUSED_THREADS / f.threads;
   // larger halos (very large leaves) take the separate kernels
-  f.lpt = lpt >= 1 && lpt <= 4 && f.lds <= 65536 - 4096 ? lpt : 0;
+  f.lpt = lpt >= 1 && lpt <= most && f.lds <= 65536 - 4096 ? lpt : 0;
   return f;
 }
 // Chain launches (and a stamp of its own for the start of a chain) of one dab at most.
@@ -2092,16 +2099,19 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
       ca.has_next = has_next && !ca.cont_out ? 1 : 0;
       ca.has_prev = prev && !ca.cont_in ? 1 : 0;
       ca.last = !has_next && !ca.cont_out ? 1 : 0;
-      ca.ns = ca.has_next ? leaf_blocks : 0;
-      ca.nc = chained && !ca.cont_in ? 128 : 0;
+      ca.ns = ca.has_next ? std::max(1, (p->d.L + fs.threads - 1) / fs.threads) : 0;
+      ca.nc = chained && !ca.cont_in ? 128 * FUSED_THREADS / fs.threads : 0;
       ProfScope ps(p, SG_K_BRUSH);
-      const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(FUSED_THREADS);
+      const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(fs.threads);
       using ChainKernel = void (*)(SgDevView, SgDabK, SgDabK, const float *, SgChainArgs, const float *);
-#define SG_CHAIN_LPT(S, P) {k_dab_chain<1, S, P>, k_dab_chain<2, S, P>, k_dab_chain<3, S, P>, k_dab_chain<4, S, P>}
-      static const ChainKernel kernels[2][2][4] = {{SG_CHAIN_LPT(false, false), SG_CHAIN_LPT(false, true)},
-                                                   {SG_CHAIN_LPT(true, false), SG_CHAIN_LPT(true, true)}};
-#undef SG_CHAIN_LPT
-      const ChainKernel kern = kernels[k.tool == SG_TOOL_SMOOTH ? 1 : 0][place ? 1 : 0][fs.lpt - 1];
+#define SG_CHAIN(P)                                                                                                \
+  {k_dab_chain<256, 1, false, P>, k_dab_chain<256, 2, false, P>, k_dab_chain<256, 3, false, P>, k_dab_chain<256, 4, false, P>, \
+   k_dab_chain<256, 1, true, P>, k_dab_chain<256, 2, true, P>, k_dab_chain<256, 3, true, P>, k_dab_chain<256, 4, true, P>,    \
+   k_dab_chain<512, 1, true, P>, k_dab_chain<512, 2, true, P>}
+      static const ChainKernel kernels[2][10] = {SG_CHAIN(false), SG_CHAIN(true)};
+#undef SG_CHAIN
+      const int variant = fs.lpt - 1 + (k.tool != SG_TOOL_SMOOTH ? 0 : fs.threads == FUSED_THREADS ? 4 : 8);
+      const ChainKernel kern = kernels[place ? 1 : 0][variant];
       SG_LAUNCH(ps, kern, gf, bf, fs.lds, s, v, kk, kn, curve_dev, ca, place);
     }
     p->chain_live = has_next;

@@ -16,6 +16,7 @@
 //    with height-ordered tables for the deferred refit of internal nodes.
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <atomic>
@@ -874,6 +875,21 @@ void sg_build_device(PBVH *p, const float *co) {
   d.T = h.T;
   d.L = L;
   d.N = N;
+  {  // leaves per unit of surface area, from up to 4096 triangles spread over the mesh
+    const int step = std::max(1, T / 4096);
+    double area = 0.0;
+    int n = 0;
+    for (int t = 0; t < T; t += step, n++) {
+      const float *a = co + 3 * (size_t)p->tris[3 * (size_t)t], *b = co + 3 * (size_t)p->tris[3 * (size_t)t + 1],
+                  *c = co + 3 * (size_t)p->tris[3 * (size_t)t + 2];
+      double u[3], v[3];
+      for (int i = 0; i < 3; i++) u[i] = (double)b[i] - a[i], v[i] = (double)c[i] - a[i];
+      const double x = u[1] * v[2] - u[2] * v[1], y = u[2] * v[0] - u[0] * v[2], z = u[0] * v[1] - u[1] * v[0];
+      area += 0.5 * std::sqrt(x * x + y * y + z * z);
+    }
+    if (n > 0) area *= (double)T / n;
+    p->leaf_density = area > 0.0 && area < 1e30 ? L / area : 0.0;
+  }
   upload(&d.px, h.x.data(), V, s);
   upload(&d.py, h.y.data(), V, s);
   upload(&d.pz, h.z.data(), V, s);

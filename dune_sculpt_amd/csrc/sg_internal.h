@@ -283,6 +283,7 @@ struct PBVH {
   int dab_count = 0;
   int grid_wg = 256;                 // workgroups of the per-dab kernels (tunable)
   int grid_brush = 0, grid_post = 0, grid_smooth = 0;  // per-kernel overrides (autotuner)
+  double leaf_density = 0.0;         // leaves per unit of surface area (sampled at the build)
   int grid_fused = 1024;             // workgroups of the fused dab kernel (a leaf each)
   bool fused_enabled = true;
   bool fused_pending = false;        // the last dab enqueued was fused and no finish followed yet
