@@ -843,8 +843,8 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // so a dab waits for one kernel boundary instead of two (three for Draw) and for no
 // search.  Bound by the chain of dependent loads, not by bytes.  As search, area normal
 // and brush kernels 240 mixed dabs on a 2.6 M-vertex mesh took 3.47 ms with the draw
-// refill after them, now 2.54; 200 Draw dabs on 41 k vertices 2.67 and 1.78; 24 dabs over
-// about 1250 leaves each 0.94 and 0.78.  The first dab of a chain has its own search (and
+// refill after them, now 2.24; 200 Draw dabs on 41 k vertices 2.67 and 1.58; 24 dabs over
+// about 1250 leaves each 0.94 and 0.76.  The first dab of a chain has its own search (and
 // k_area).
 //
 // F works on the leaf's halo (its uniq vertices, ring 0 = its shared vertices and their
@@ -868,7 +868,7 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // list, each with an even share of the steps: a launch that another one continues stages
 // its positions and Smooth factors only, and the continuing launch takes the staged
 // vertices as the affected ones.  Smooth(8) on 655 k vertices, 60 dabs: 2.65 ms with a
-// kernel per step, 1.35 as two launches per dab.
+// kernel per step, 1.18 as two launches per dab.
 // ---------------------------------------------------------------------------
 #define FUSED_THREADS 256  // twice that for Smooth dabs whose halos have more locals
 #define FUSED_LEAD 256  // F blocks started before the S and C blocks: more leaves than most dabs gather
@@ -2073,7 +2073,7 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
     // (the positions before it) and writes the mesh; normals stay staged, and the next dab's
     // search launch copies them and the shadow copy in.  80 placed dabs of r 0.03 to 0.1 on
     // 317 k vertices with an undo step: 2.44 ms as search, brush, Smooth and post kernels,
-    // 2.29 now.
+    // 2.20 now.
     if (place) {
       std::swap(v.px, v.qx);
       std::swap(v.py, v.qy);
