@@ -53,7 +53,7 @@ struct GView {  // kernel view of SgGridDev (by value)
   const int *face_gbeg, *grid_face, *face_edge, *face_vert, *edge_foff, *edge_el, *vert_foff, *vert_el;
   int *face_stamp, *edge_stamp, *vert_stamp;
   int *gathered, *dfaces, *ditems;
-  long long *ctr, *ctr_last;
+  long long *ctr, *ctr_next, *ctr_last;  // the operation's counters, the set of the dab after it, the last dab's
   int *dser;  // [0] the running operation's serial, [1] the last dab's
   int *leaf_dirty, *node_dirty;  // refit since the last internal-node flush
   int *leaf_gmark;               // serial of the last dab that gathered the leaf
@@ -120,7 +120,8 @@ GView view_of(const SgGridDev &d) {
   v.gathered = d.gathered;
   v.dfaces = d.dfaces;
   v.ditems = d.ditems;
-  v.ctr = d.ctr;
+  v.ctr = d.ctr + d.cset * SGG_CTR_SET;
+  v.ctr_next = d.ctr + (d.cset ^ 1) * SGG_CTR_SET;
   v.ctr_last = d.ctr_last;
   v.dser = d.dser;
   v.leaf_dirty = d.leaf_dirty;
@@ -1032,7 +1033,10 @@ __global__ __launch_bounds__(GR_THREADS) void kg_refit_parts(GView g, const int 
 // with `finish`, and, when a dab follows (has_next), its search: as launches of their own
 // these were 3.6 and 2.2 us and two boundaries.  Workgroups with no part leave at once; the
 // others count themselves in with release and acquire at agent scope, so the last one sees
-// every part.
+// every part.  A workgroup may start after the last one has closed the dab, so nothing that
+// it decides by may then say that it takes part: this dab's counters only fall to zero here
+// (nb is then 1, and workgroup 0 has been counted), and the next dab's leaves are counted in
+// the other set.
 __global__ __launch_bounds__(GR_THREADS) void kg_dab_refit(GView g, float *parts, long long *log, SgDabK kn,
                                                            int has_next) {
   __shared__ float s_bb[GR_THREADS / SG_WAVE][6];
@@ -1108,7 +1112,7 @@ __global__ __launch_bounds__(GR_THREADS) void kg_dab_refit(GView g, float *parts
     }
   }
   __syncthreads();
-  if (t == 0) g.ctr[SGG_NGATHER] = s_ng;
+  if (t == 0) g.ctr_next[SGG_NGATHER] = s_ng;
 }
 
 // The listed leaves' boxes from their parts, in order; orig_vb = vb when set_orig; the
@@ -1186,7 +1190,7 @@ __global__ __launch_bounds__(1024) void kg_flush_nodes(GView g, int set_orig) {
 // Around a drop-in update (and before a dab after a failed launch): zero the counters
 // and take the next serial on the device (a dab ends the same way in kg_refit_combine).
 __global__ void kg_clear_ctr(GView g) {
-  if (threadIdx.x < SGG_CTR_COUNT) g.ctr[threadIdx.x] = 0;
+  if (threadIdx.x < SGG_CTR_COUNT) g.ctr[threadIdx.x] = g.ctr_next[threadIdx.x] = 0;
   if (threadIdx.x < GR_LINES) g.lines[threadIdx.x * GR_LINE] = g.lines[threadIdx.x * GR_LINE + 1] = 0;
   if (threadIdx.x == 0) {
     g.dser[0] = g.dser[0] + 1;
@@ -1401,7 +1405,7 @@ int sg_grids_build_device(PBVH *p) {
   rc |= gupload(&d.lvl_off, lvl_off.data(), lvl_off.size());
   rc |= gupload(&d.lvl_node, lvl_node.data(), lvl_node.size());
   rc |= gzeros(&d.gathered, (size_t)d.L);
-  rc |= gzeros(&d.ctr, (size_t)SGG_CTR_COUNT);
+  rc |= gzeros(&d.ctr, (size_t)2 * SGG_CTR_SET);
   rc |= gzeros(&d.ctr_last, (size_t)SGG_CTR_COUNT);
   rc |= gzeros(&d.curve, (size_t)(SG_CM_TABLE + 1));
   rc |= gzeros(&d.hlist, (size_t)d.L);
@@ -1540,6 +1544,7 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   if (k.tool != SG_TOOL_DRAW && k.tool != SG_TOOL_INFLATE && k.tool != SG_TOOL_SMOOTH && k.tool != SG_TOOL_GRAB)
     return sg_set_error("grids: tool %d is not supported on PBVH_GRIDS (Draw, Inflate, Smooth, Grab)", k.tool);
   if (k.learned || k.orig_co) return sg_set_error("grids: learned Smooth and original-coordinate Grab are faces only");
+  d.cset = searched ? d.cset ^ 1 : 0;  // the set that the dab before counted this one's leaves in
   const GView g = view_of(d);
   const int rh = p->respect_hide ? 1 : 0;
   const int eb = elem_blocks(d);

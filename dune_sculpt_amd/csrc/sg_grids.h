@@ -85,7 +85,8 @@ struct SgGridDev {
   int *face_stamp = nullptr, *edge_stamp = nullptr, *vert_stamp = nullptr;
   int *gathered = nullptr;    // [L] the dab's gathered leaves, then the leaves its averages moved
   int *dfaces = nullptr, *ditems = nullptr;  // dirty faces [F], dirty edges then vertices [Ed + Vc]
-  long long *ctr = nullptr;   // live counters
+  long long *ctr = nullptr;   // live counters, two sets (a dab that searches for the next one counts in the other)
+  int cset = 0;               // the set of the last operation enqueued
   long long *ctr_last = nullptr;  // the last dab's counters
   float *curve = nullptr;     // CUSTOM falloff table
   int *hlist = nullptr;       // [L] leaf lists from the host (drop-in updates)
@@ -109,7 +110,8 @@ struct SgGridDev {
 // counters (ctr / ctr_last)
 enum {
   SGG_NGATHER = 0, SGG_NAFF = 1, SGG_AREA_X = 2, SGG_AREA_Y = 3, SGG_AREA_Z = 4, SGG_NAREA = 5,
-  SGG_NFACES = 6, SGG_NITEMS = 7, SGG_NMOVED = 8, SGG_NLEAVES = 9, SGG_CTR_COUNT = 12
+  SGG_NFACES = 6, SGG_NITEMS = 7, SGG_NMOVED = 8, SGG_NLEAVES = 9, SGG_CTR_COUNT = 12,
+  SGG_CTR_SET = 16  // from one set to the next
 };
 
 struct PBVH;

@@ -70,3 +70,35 @@ def test_single_dab_after_strokes_and_edits(sg, po):
         got.append(_all(p))
         p.close()
     assert all(np.asarray(x).tobytes() == np.asarray(y).tobytes() for x, y in zip(*got))
+
+
+def test_dabs_of_few_leaves_before_wide_ones_beside_other_work(sg):
+    """The refit's last workgroup searches for the next dab while others of its launch may not
+    have started: dabs that gather nothing or a leaf or two (few workgroups take part) before
+    dabs over most leaves, with another stream keeping the chip busy."""
+    wide, narrow = stroke(sg, 3, 30, 0.5, 1.2), stroke(sg, 4, 30, 0.01, 0.02)
+    away = sg.make_dab(tool=1, location=(9, 9, 9), radius=0.1, strength=0.5)
+    dabs = [d for i in range(30) for d in (narrow[i], away, wide[i])]
+    co, tris = sg.noisy_icosphere(7, seed=3, amplitude=0.02)
+    other = sg.PBVH(co, tris, leaf_limit=64)
+    cover = other.prepare([sg.make_dab(tool=2, location=co[0], radius=3.0, strength=0.5, smooth_iterations=8)] * 40)
+    got = []
+    for busy in (True, False, None):
+        g, _ = noisy_sphere_grids(sg, 16, 3, seed=5)
+        p = gr.GridPBVH(g, leaf_limit=200)
+        assert p.nodes > 200
+        for _ in range(2):
+            if busy:
+                for _ in range(4):
+                    cover.launch(sync=False)
+            if busy is None:  # each dab with a search of its own
+                for d in dabs:
+                    p.dab(d)
+            else:
+                p.stroke(dabs)
+        got.append(_all(p))
+        p.close()
+    cover.launch()
+    other.close()
+    for x in got[:2]:
+        assert all(np.asarray(u).tobytes() == np.asarray(w).tobytes() for u, w in zip(x, got[2]))
