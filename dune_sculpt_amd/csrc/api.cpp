@@ -900,7 +900,8 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
     }
   }
   p->halt_live = s->learned;
-  if (p->type == PBVH_GRIDS && !p->gd->topo_of && p->subdiv_ccg && sg_grids_attach_topology(p, p->subdiv_ccg)) {
+  if (p->type == PBVH_GRIDS &&
+      ((!p->gd->topo_of && p->subdiv_ccg && sg_grids_attach_topology(p, p->subdiv_ccg)) || sg_grids_settle(p))) {
     stroke_release(s);
     return nullptr;
   }
@@ -909,7 +910,6 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
   int erc = 0;
   if (!rc && p->type == PBVH_GRIDS) {  // each grid dab is self-contained (counters, normals, refit)
     int ci = 0;
-    p->gd->searched = false;
     for (int i = 0; i < n && !erc; i++) {
       const float *curve = nullptr;
       if (dabs[i].curve_preset == SG_CURVE_CUSTOM && dabs[i].curve_table)
@@ -921,6 +921,7 @@ static SgStroke *stroke_prepare(PBVH *p, const SgDabParams *dabs, const SgRay *r
     if (!erc) erc = sg_grids_enqueue_flush(p);
     const hipError_t e = hipStreamEndCapture(p->stream, &s->graph);
     rc = erc ? erc : sg_check_hip(e, "end capture");
+    if (erc) p->gd->ctr_unclean = p->gd->searched = false;  // nothing ran: the counters are as before the capture
   } else if (!rc) {
     int ci = 0;
     int nlaunch = 0;

@@ -1534,6 +1534,22 @@ static int enqueue_normals(PBVH *p, const GView &g, const int *leaves, int n) {
   return launch_check("grid normals");
 }
 
+// Clears now what a failed launch left in the counters: before a capture, which would only
+// record the clear and leave them to whatever runs before the graph does.
+int sg_grids_settle(PBVH *p) {
+  SgGridDev &d = *p->gd;
+  d.searched = false;
+  if (!d.ctr_unclean) return 0;
+  kg_clear_ctr<<<1, 64, 0, p->stream>>>(view_of(d));
+  if (int rc = launch_check("grid counters")) return rc;
+  d.ctr_unclean = false;
+  return 0;
+}
+
+static bool grid_tool(const SgDabK &k) {
+  return k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_SMOOTH || k.tool == SG_TOOL_GRAB;
+}
+
 int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log, int log_index,
                          const SgDabK *next) {
   if (!p->gd) return sg_set_error("grids: no device layout");
@@ -1541,7 +1557,7 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   const bool searched = d.searched;  // by the dab before
   d.searched = false;
   if (!d.topo_of) return sg_set_error("grids: no SubdivCCG attached (DUNE_pbvh_subdiv_cgg_set)");
-  if (k.tool != SG_TOOL_DRAW && k.tool != SG_TOOL_INFLATE && k.tool != SG_TOOL_SMOOTH && k.tool != SG_TOOL_GRAB)
+  if (!grid_tool(k))
     return sg_set_error("grids: tool %d is not supported on PBVH_GRIDS (Draw, Inflate, Smooth, Grab)", k.tool);
   if (k.learned || k.orig_co) return sg_set_error("grids: learned Smooth and original-coordinate Grab are faces only");
   d.cset = searched ? d.cset ^ 1 : 0;  // the set that the dab before counted this one's leaves in
@@ -1549,7 +1565,7 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   const int rh = p->respect_hide ? 1 : 0;
   const int eb = elem_blocks(d);
   const bool normals = p->gridkey.has_normals != 0;
-  // a failed launch, or a search for a dab that did not follow, left the counters
+  // a failed launch left the counters
   if (d.ctr_unclean && !searched) kg_clear_ctr<<<1, 64, 0, p->stream>>>(g);
   d.ctr_unclean = true;
   if (!searched) kg_search<<<(d.L + GR_THREADS - 1) / GR_THREADS, GR_THREADS, 0, p->stream>>>(g, k);
@@ -1573,8 +1589,9 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
     kg_dab_faces<<<std::max(1, std::min(d.F, 2048)), DF_THREADS, d.face_lds, p->stream>>>(g, k, curve_dev, rh, s[0], s[1],
                                                                                         s[2]);
     kg_dab_edges<<<std::max(1, std::min((d.Ed + d.Vc + 3) / 4, 1024)), GR_THREADS, 0, p->stream>>>(g);
-    // one workgroup searches 256 leaves at a time: past a few rounds a launch of its own is shorter
-    const bool search = next && d.L <= 4 * GR_THREADS;
+    // one workgroup searches 256 leaves at a time: past a few rounds a launch of its own is
+    // shorter; a dab that will be refused leaves no search behind
+    const bool search = next && d.L <= 4 * GR_THREADS && grid_tool(*next) && !next->learned && !next->orig_co;
     const SgDabK kn = search ? *next : k;
     kg_dab_refit<<<std::max(1, std::min(d.L * GR_SPLIT, 512)), GR_THREADS, 0, p->stream>>>(
         g, d.parts, log ? log + (size_t)log_index * SG_CTR_COUNT : nullptr, kn, search ? 1 : 0);

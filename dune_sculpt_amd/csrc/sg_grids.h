@@ -94,7 +94,7 @@ struct SgGridDev {
   int *dser = nullptr;        // [4] device serials: the running operation's, the last dab's; blocks done
   int *leaf_dirty = nullptr, *node_dirty = nullptr;  // refit since the last internal-node flush
   float *parts = nullptr;     // [L * 8 * 8] boxes of the parts of the leaves being refit
-  bool ctr_unclean = false;   // a dab's launches failed midway, or it searched for a next one: clear the counters first
+  bool ctr_unclean = false;   // a dab's launches failed midway, or the last one searched for a next one
   bool searched = false;      // the last dab enqueued searched for the one after it
   int *leaf_gmark = nullptr;  // [L] serial of the last dab that gathered the leaf
   int4 *face_leaf = nullptr;  // [F] the leaves of the face's grids
@@ -122,6 +122,7 @@ void sg_grids_free_device(PBVH *p);
 // next: the dab enqueued after this one with no other work between, or null
 int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *log = nullptr,
                          int log_index = 0, const SgDabK *next = nullptr);
+int sg_grids_settle(PBVH *p);
 int sg_grids_snapshot(PBVH *p, int restore);
 int sg_grids_enqueue_update_normals(PBVH *p, const int *leaves_dev, int n);
 int sg_grids_enqueue_refit(PBVH *p, const int *leaves_dev, int n, int set_orig);

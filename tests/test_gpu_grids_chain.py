@@ -102,3 +102,29 @@ def test_dabs_of_few_leaves_before_wide_ones_beside_other_work(sg):
     other.close()
     for x in got[:2]:
         assert all(np.asarray(u).tobytes() == np.asarray(w).tobytes() for u, w in zip(x, got[2]))
+
+
+@pytest.mark.parametrize("bad", [{"tool": 21}, {"tool": 2, "flag": "SMOOTH_LEARNED"}])
+def test_stroke_with_a_refused_dab(sg, bad):
+    """A stroke stops at a dab that grids do not cover; what ran before it stays, and the next
+    calls (a captured stroke that is not launched yet, a dab, the stroke) see clean counters."""
+    dabs = stroke(sg, 3, 6, 0.3, 0.6)
+    kw = {k: getattr(sg, v) if isinstance(v, str) else v for k, v in bad.items()}
+    no = sg.make_dab(location=(0, 0, 1), radius=0.3, strength=0.5, **kw)
+    got = []
+    for refused in (True, False):
+        g, _ = noisy_sphere_grids(sg, 12, 3, seed=5)
+        p = gr.GridPBVH(g, leaf_limit=200)
+        if refused:
+            with pytest.raises(RuntimeError):
+                p.stroke([dabs[0], no, dabs[1]], graph=False)
+            with pytest.raises(RuntimeError):
+                p.prepare([dabs[0], no])
+        else:
+            p.dab(dabs[0])
+        st = p.prepare(dabs[2:])
+        p.dab(dabs[1])
+        st.launch()
+        got.append(_all(p))
+        p.close()
+    assert all(np.asarray(x).tobytes() == np.asarray(y).tobytes() for x, y in zip(*got))
