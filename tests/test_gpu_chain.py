@@ -175,3 +175,68 @@ def test_replay_undo_and_readers(sg):
         p.close()
     for x, y in zip(*got):
         assert x.tobytes() == y.tobytes()
+
+
+def test_area_normal_of_leaves_whose_boxes_lag(sg, po):
+    """Host edits whose normals were updated and bounds not: a leaf that the dab before did
+    not touch is gathered by its old box, and every vertex of it counts for the area normal,
+    wherever it lies now."""
+    co, tris = sg.noisy_icosphere(5, seed=9, amplitude=0.02)
+    c, r = co[123], 0.6
+    dabs = [sg.make_dab(tool=1, location=-c, radius=0.1, strength=0.5),
+            sg.make_dab(tool=1, location=c, radius=r, strength=0.7, normal_radius_factor=0.5)]
+    o = po.Oracle(co, tris, leaf_limit=64)
+    near = {n: np.linalg.norm(co[o.node_verts(n)] - c, axis=1).min() for n in o.leaves_dfs()}
+    far = [n for n in near if 0.36 < near[n] < 0.55]
+    assert len(far) > 3
+    moved = np.unique(np.concatenate([o.node_verts(n) for n in far]))
+    got = []
+    for fused in (True, False):
+        p = sg.PBVH(co, tris, leaf_limit=64)
+        assert p.set_fused(fused)
+        if fused:
+            o.set_normals(p.normals())
+        mv = p.mverts()
+        for v in moved:
+            mv[v] = (c + 0.2 * (co[v] - c)).astype(np.float32)
+            if fused:
+                o.set_vert(v, mv[v])
+        for n in far:
+            p.node_mark_update(n)
+        p.update_normals()  # uploads the edit; no vertex is marked, and no bounds update follows
+        p.stroke(dabs, log=True)
+        got.append([p.stroke_log(2)[:, :6], p.positions(), p.normals()])
+        p.close()
+    assert all(x.tobytes() == y.tobytes() for x, y in zip(*got))
+    for d in dabs:
+        o.dab(d)
+    assert np.abs(got[0][1] - o.positions()).max() <= 1e-5
+    o.close()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_vertices_that_are_no_numbers(sg, value):
+    """A vertex of some leaves is NaN or infinite: its leaf's box folds over it, its neighbours'
+    normals and Smooth steps take it up, and the chain decides as the separate kernels do."""
+    co, tris = sg.noisy_icosphere(5, seed=9, amplitude=0.02)
+    dabs = _path(sg, 16, 5, np.resize([0.5, 0.1, 0.6], 16), (1, 4, 1, 2, 5), (3, 6))
+    at = np.stack([d.location for d in dabs[:4]]).astype(np.float32)
+    bad = [int(np.argsort(np.linalg.norm(co - c, axis=1))[j]) for c in at for j in (60, 140)]
+    got = []
+    for fused in (True, False):
+        p = sg.PBVH(co, tris, leaf_limit=64)
+        p.set_fused(fused)
+        mv = p.mverts()
+        for v in bad:
+            mv[v] = (co[v][0], value, co[v][2])
+            p.vert_mark_update(v)
+        for i in range(p.tree_info()["nodes"]):
+            if p.node_flag(i) & sg.PBVH_Leaf:
+                p.node_mark_update(i)
+        p.update_bounds(sg.PBVH_UpdateBB | sg.PBVH_UpdateOriginalBB)
+        p.stroke(dabs, log=True)
+        got.append([p.stroke_log(16)[:, :6], *_state(p), p.last_affected()])
+        p.close()
+    for x, y in zip(*got):
+        assert np.array_equal(x, y, equal_nan=x.dtype == np.float32)
+    assert np.isnan(got[0][1]).any() or np.isinf(got[0][1]).any()
