@@ -2029,8 +2029,9 @@ static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
   const bool few = 3.14159 * reach * reach * p->leaf_density <= 512.0;  // leaves the dab gathers on a surface
   f.threads = k.tool == SG_TOOL_SMOOTH && f.cap > FUSED_THREADS && few ? 2 * FUSED_THREADS : FUSED_THREADS;
   const int lpt = (f.cap + f.threads - 1) / f.threads, most = 4 * FUSED_THREADS / f.threads;
-  // larger halos (very large leaves) take the separate kernels
-  f.lpt = lpt >= 1 && lpt <= most && f.lds <= 65536 - 4096 ? lpt : 0;
+  // larger halos (very large leaves) take the separate kernels; the kernel's own arrays come on
+  // top of these 64 KiB (a workgroup may have 160)
+  f.lpt = lpt >= 1 && lpt <= most && f.lds <= 65536 ? lpt : 0;
   return f;
 }
 // Chain launches (and a stamp of its own for the start of a chain) of one dab at most.

@@ -240,3 +240,18 @@ def test_vertices_that_are_no_numbers(sg, value):
     for x, y in zip(*got):
         assert np.array_equal(x, y, equal_nan=x.dtype == np.float32)
     assert np.isnan(got[0][1]).any() or np.isinf(got[0][1]).any()
+
+
+@pytest.mark.parametrize("nu,nv,leaf", [(64, 28, 1900), (60, 30, 1800), (62, 30, 1900)])
+def test_largest_fused_leaves(sg, nu, nv, leaf):
+    """Two leaves whose vertices, ring and faces take 60.5 to 62.8 KiB of LDS for a Draw dab
+    are still one launch a dab (no normals kernel of its own)."""
+    co, tris = sg.noisy_torus(nu, nv, seed=2, amplitude=0.01)
+    dabs = [sg.make_dab(tool=(1, 4, 5)[i % 3], location=co[37 * i], radius=0.3, strength=0.5, grab_delta=(0.01, 0, 0))
+            for i in range(7)]
+    _check(sg, co, tris, dabs, leaf=leaf)
+    p = sg.PBVH(co, tris, leaf_limit=leaf)
+    p.set_profile(True)
+    p.stroke(dabs, graph=False)
+    assert [v[1] for k, v in p.profile_read().items() if "post" in k] == [0]
+    p.close()
