@@ -960,11 +960,10 @@ int sg_batch_load(SgBatch *b, const SgDabParams *dabs, int steps) {
   b->learned = learned;
   b->odd_k = odd_k;
   if (b->persistent_auto) b->persistent = persistent_pays(b, dabs, steps);
-  const int cfg[] = {maxk, learned ? 1 : 0, odd_k ? 1 : 0, b->mlp ? 1 : 0, b->g_search, b->g_brush, b->g_smooth,
-                     b->g_post, b->g_learned, b->brush_threads, b->brush_vpl};
-  long long key = 1469598103934665603ll;
-  for (int c : cfg) key = (key ^ (long long)c) * 1099511628211ll;
-  if (b->exec && b->exec_key == key) return 0;
+  // what the step graph depends on besides the table's contents
+  const std::vector<int> cfg = {maxk, learned ? 1 : 0, odd_k ? 1 : 0, b->mlp ? 1 : 0, b->g_search, b->g_brush,
+                                b->g_smooth, b->g_post, b->g_learned, b->brush_threads, b->brush_vpl};
+  if (b->exec && b->exec_cfg == cfg) return 0;
   if (b->exec) hipGraphExecDestroy(b->exec);
   b->exec = nullptr;
   hipGraph_t graph = nullptr;
@@ -976,7 +975,7 @@ int sg_batch_load(SgBatch *b, const SgDabParams *dabs, int steps) {
   }
   if (!rc) rc = sg_check_hip(hipGraphInstantiate(&b->exec, graph, nullptr, nullptr, 0), "instantiate");
   if (graph) hipGraphDestroy(graph);
-  if (!rc) b->exec_key = key;
+  if (!rc) b->exec_cfg = cfg;
   return rc;
 }
 

@@ -95,7 +95,7 @@ struct SgBatch {
   int brush_threads = 256, brush_vpl = 1;
   // captured step graph and the configuration it was captured for
   hipGraphExec_t exec = nullptr;
-  long long exec_key = -1;
+  std::vector<int> exec_cfg;
   // checkpoint
   std::vector<void *> snap;
   bool snap_valid = false;

@@ -36,3 +36,25 @@ def test_default_choice_keeps_the_bits(sg, levels, tables):
     assert a.totals() == b.totals()
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("persistent", [False, True])
+def test_tables_of_other_step_counts_in_one_batch(sg, persistent):
+    """Tables that need other kernels in the step graph than the one before them (Smooth steps,
+    odd and even) against the same dabs on each mesh alone."""
+    meshes = [sg.noisy_icosphere(lv, seed=60 + lv, amplitude=0.02) for lv in (4, 5)]
+    b = sg.Batch(meshes, leaf_limit=64)
+    b.set_persistent(persistent)
+    alone = [sg.PBVH(co, tris, leaf_limit=64) for co, tris in meshes]
+    rng = np.random.default_rng(5)
+    for tool, k in ((1, 1), (2, 4), (2, 16), (2, 3), (2, 1), (4, 1), (2, 64)):
+        table = [[sg.make_dab(tool=tool, location=co[rng.integers(len(co))], radius=0.3, strength=0.5,
+                              smooth_iterations=k) for co, _ in meshes] for _ in range(3)]
+        b.run(table)
+        for m, p in enumerate(alone):
+            p.stroke([row[m] for row in table])
+            assert np.array_equal(b.positions(m).view(np.uint32), p.positions().view(np.uint32)), (tool, k, m)
+            assert np.array_equal(b.normals(m).view(np.uint32), p.normals().view(np.uint32)), (tool, k, m)
+    b.close()
+    for p in alone:
+        p.close()
