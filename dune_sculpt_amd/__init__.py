@@ -1183,10 +1183,10 @@ class Batch:
             pass
 
     def info(self):
-        out = (C.c_longlong * (6 + self.M))()
-        _check(lib().sg_batch_info(self.h, out, 6 + self.M), "batch info")
+        out = (C.c_longlong * (7 + self.M))()
+        _check(lib().sg_batch_info(self.h, out, 7 + self.M), "batch info")
         return {"meshes": out[0], "verts": out[1], "tris": out[2], "leaves": out[3], "cuts": out[4],
-                "vbase": [out[5 + i] for i in range(self.M + 1)]}
+                "vbase": [out[5 + i] for i in range(self.M + 1)], "persistent": bool(out[6 + self.M])}
 
     def _table(self, table):
         steps = len(table)

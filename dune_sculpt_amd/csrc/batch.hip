@@ -877,38 +877,44 @@ void sg_batch_free(SgBatch *b) {
   delete b;
 }
 
-// out: meshes, vertices, tris, leaves, cuts, then the vertex and leaf offset of mesh i
-// for i < n_meshes when out has room (out_n entries).
+// out: meshes, vertices, tris, leaves, cuts, then the first vertex of each mesh (M + 1 entries)
+// and whether launches of the loaded table take the persistent step, while out has room.
 int sg_batch_info(SgBatch *b, long long *out, int out_n) {
   if (batch_check(b)) return -1;
   const long long head[5] = {b->M, b->vbase.back(), b->tbase.back(), b->lbase.back(), b->cbase.back()};
   for (int i = 0; i < 5 && i < out_n; i++) out[i] = head[i];
   for (int m = 0; m <= b->M && 5 + m < out_n; m++) out[5 + m] = b->vbase[m];
+  if (6 + b->M < out_n) out[6 + b->M] = b->persistent && b->pm_ok && !b->learned ? 1 : 0;
   return 0;
 }
 
 // Whether a table runs faster as one launch with a workgroup per mesh than as a graph per
-// step.  The persistent step lasts as long as its slowest mesh: 14 us per dab and 30 ns per
-// affected vertex on that mesh's one CU.  A step graph lasts 45 us (its 7 to 10 kernels and
-// their boundaries) and 0.45 ns per affected vertex of all meshes on the whole chip.
-// Measured per step, persistent / graph: 32 meshes of 5k-60k vertices 19.5 / 51.9 us; 2
-// meshes 15.3 / 43.9; 8 of 200k-500k 37.2 / 51.3; 96 of 5k-500k 34.6 / 59.5; 64 of 1M-4M
-// (r to 0.08) 92 / 92.
-static bool persistent_pays(const SgBatch *b, const SgDabParams *dabs, int steps) {
+// step.  The persistent launch lasts as long as its slowest mesh, whose dabs take 14.5 us each,
+// 0.7 a Smooth step after the first, and on that mesh's one CU 24 ns an affected vertex and 3.8
+// for each further step of it.  A step graph lasts 36 us (its kernels and their boundaries),
+// 3 us for each Smooth step after the first that any dab of the table has, and 0.4 ns an
+// affected vertex of all meshes and 0.03 for each further step of it, on the whole chip.
+// Measured per step, persistent / graph: 2 meshes of 41 k vertices, r 0.1, Draw 18 / 37 us,
+// Smooth(64) 74 / 241; r 0.6 92 / 45 and 1080 / 315; 130 of them, r 0.6, Draw 112 / 139,
+// Smooth(16) 385 / 390; one of 164 k, r 0.1, Smooth(4) 32 / 47, r 0.25 112 / 52; of 252 tables
+// (1 to 160 meshes of 2.6 k to 655 k vertices, r 0.04 to 0.6, k 1 to 64) one takes the other
+// side, by 4 percent.
+static bool persistent_pays(const SgBatch *b, const SgDabK *dabs, int steps, int maxk) {
   double slowest = 0.0, all = 0.0;
   for (int m = 0; m < b->M; m++) {
     const double nv = (double)(b->vbase[m + 1] - b->vbase[m]);
     double t = 0.0;
     for (int s = 0; s < steps; s++) {
-      const SgDabParams &p = dabs[(size_t)s * b->M + m];
-      if (p.sculpt_tool == 0) continue;
-      const double aff = std::min(nv, 3.14159 * (double)p.radius * (double)p.radius * b->density[m]);
-      t += 14.0 + 0.030 * aff;
-      all += aff;
+      const SgDabK &k = dabs[(size_t)s * b->M + m];
+      if (k.tool == 0) continue;
+      const double aff = std::min(nv, 3.14159 * (double)k.r * (double)k.r * b->density[m]);
+      const int more = k.tool == SG_TOOL_SMOOTH ? k.iters - 1 : 0;
+      t += 14.5 + 0.7 * more + (0.024 + 0.0038 * more) * aff;
+      all += (0.0004 + 0.00003 * more) * aff;
     }
     slowest = std::max(slowest, t);
   }
-  return slowest <= 45.0 * steps + 0.00045 * all;
+  return slowest <= (36.0 + 3.0 * std::max(maxk - 1, 0)) * steps + all;
 }
 
 // Upload a [steps][n_meshes] dab table (tool 0 = no dab for that mesh in that step)
@@ -959,7 +965,7 @@ int sg_batch_load(SgBatch *b, const SgDabParams *dabs, int steps) {
   b->maxk = maxk;
   b->learned = learned;
   b->odd_k = odd_k;
-  if (b->persistent_auto) b->persistent = persistent_pays(b, dabs, steps);
+  if (b->persistent_auto) b->persistent = persistent_pays(b, tab.data(), steps, maxk);
   // what the step graph depends on besides the table's contents
   const std::vector<int> cfg = {maxk, learned ? 1 : 0, odd_k ? 1 : 0, b->mlp ? 1 : 0, b->g_search, b->g_brush,
                                 b->g_smooth, b->g_post, b->g_learned, b->brush_threads, b->brush_vpl};

@@ -501,7 +501,8 @@ SgBatch *sg_batch_new(int n_meshes, const float *const *co, const int *const *tr
                       const int *tottri, int leaf_limit);
 void sg_batch_free(SgBatch *batch);
 /* out[0..4] = meshes, vertices, tris, leaves, search cuts; then the first vertex of
- * each mesh in the arena (n_meshes + 1 entries) while out_n allows. */
+ * each mesh in the arena (n_meshes + 1 entries), then 1 when graph launches of the loaded
+ * table take the persistent step (0: a step graph), while out_n allows. */
 int sg_batch_info(SgBatch *batch, long long *out, int out_n);
 /* dabs[step * n_meshes + mesh], sculpt_tool 0 = no dab for that mesh in that step.
  * load uploads the table and captures the step graph; launch runs the next `steps`
@@ -530,7 +531,7 @@ int sg_batch_get_launch(SgBatch *batch, int g[7]);
 int sg_batch_autotune(SgBatch *batch, const SgDabParams *dabs, int steps, double out_ms[2]);
 int sg_batch_set_learned(SgBatch *batch, SgMlp *mlp);
 /* Persistent step on or off (default: decided for each loaded table from the meshes'
- * vertex densities and the dabs' radii; the autotuner times both): graph launches (sg_batch_launch flags bit 0 clear) of a table
+ * vertex densities and the dabs' tools, radii and Smooth steps; the autotuner times both): graph launches (sg_batch_launch flags bit 0 clear) of a table
  * without learned Smooth dabs run every row in one kernel, a workgroup per mesh
  * advancing its own dabs with workgroup barriers only; otherwise one captured step
  * graph per row.  Both give the same bits.  Returns whether the batch fits the

@@ -17,19 +17,20 @@ def _table(sg, meshes, steps, rmin, rmax, seed, empty=()):
             for s in range(steps)]
 
 
-@pytest.mark.parametrize("levels,tables", [
-    ((3, 4), [(0.05, 0.2, ())]),
-    ((7,), [(0.4, 0.9, ()), (0.01, 0.03, ())]),
-    ((4, 7, 2), [(0.02, 0.1, (1,)), (0.5, 1.5, ()), (0.02, 0.05, (0, 2))]),
+@pytest.mark.parametrize("levels,tables", [  # per table: radii, meshes without dabs, the choice
+    ((3, 4), [(0.05, 0.2, (), True)]),
+    ((7,), [(0.4, 0.9, (), False), (0.01, 0.03, (), True), (0.5, 0.8, (), False)]),
+    ((4, 7, 2), [(0.02, 0.1, (1,), True), (0.5, 1.5, (), False), (0.02, 0.05, (0, 2), True)]),
 ])
 def test_default_choice_keeps_the_bits(sg, levels, tables):
     meshes = [sg.noisy_icosphere(lv, seed=50 + i, amplitude=0.02) for i, lv in enumerate(levels)]
     a, b = sg.Batch(meshes, leaf_limit=64), sg.Batch(meshes, leaf_limit=64)
     b.set_persistent(False)
-    for i, (rmin, rmax, empty) in enumerate(tables):
+    for i, (rmin, rmax, empty, persistent) in enumerate(tables):
         table = _table(sg, meshes, 6, rmin, rmax, i, empty)
         a.run(table)
         b.run(table)
+        assert a.info()["persistent"] == persistent and not b.info()["persistent"], i
         for m in range(len(meshes)):
             assert np.array_equal(a.positions(m).view(np.uint32), b.positions(m).view(np.uint32)), (i, m)
             assert np.array_equal(a.normals(m).view(np.uint32), b.normals(m).view(np.uint32)), (i, m)
@@ -58,3 +59,17 @@ def test_tables_of_other_step_counts_in_one_batch(sg, persistent):
     b.close()
     for p in alone:
         p.close()
+
+
+def test_choice_by_tool_and_steps(sg):
+    """A wide Draw dab on one mesh beside Smooth dabs on the other: with a few steps the graph
+    is the shorter one, with 64 it has 63 kernels more in every step."""
+    meshes = [sg.noisy_icosphere(7, seed=50, amplitude=0.02), sg.noisy_icosphere(4, seed=51, amplitude=0.02)]
+    b = sg.Batch(meshes, leaf_limit=64)
+    for k, persistent in ((2, False), (64, True), (1, False)):
+        b.load([[sg.make_dab(tool=1, location=meshes[0][0][9], radius=0.25, strength=0.5),
+                 sg.make_dab(tool=2, location=meshes[1][0][9], radius=0.04, strength=0.5, smooth_iterations=k)]] * 4)
+        assert b.info()["persistent"] == persistent, k
+    b.set_persistent(False)
+    assert not b.info()["persistent"]
+    b.close()
