@@ -99,6 +99,15 @@ __device__ __forceinline__ void chain_append(const SgDevView &d, int serial, int
   }
 }
 
+// Counter i (SG_CTR_*) of a chained dab: its lines summed.
+__device__ __forceinline__ long long chain_counter(const long long *lines, int i) {
+  const int f = i == SG_CTR_NAREA ? SG_CH_NAREA : i;
+  if (f > SG_CH_NAREA || i == SG_CH_NAREA) return 0;
+  long long t = 0;
+  for (int q = 0; q < SG_CH_SEG; q++) t += lines[q * SG_CH_CTR + f];
+  return t;
+}
+
 // Affected vertices of dab `ls`, staged by launch `ss`, into the mesh arrays: a wave per
 // leaf it gathered (its uniq range, entries of that launch only).
 __device__ __forceinline__ void chain_copy_back(const SgDevView &d, int ls, int ss, int gw, int nw) {
@@ -145,7 +154,9 @@ __device__ __forceinline__ void chain_copy_back(const SgDevView &d, int ls, int 
 //   leaf blocks       a thread per leaf: box test, then for passing leaves the records
 //                     load beside one slot reservation per wave
 //   [copy0, ...)      copy in the fused dab before (number serial - 1, launch copy_ss), when
-//                     its own launch had no next dab to leave that to (placed strokes)
+//                     its own launch had no next dab to leave that to (placed strokes, and
+//                     dabs that are not fused after one that is: a launch for the copy alone
+//                     cost a stroke that alternates the two 3 us in each pair)
 // No test waits on a subtree box: a leaf's own box decides, so a passing leaf's chain
 // is its box, then the reservation.
 __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long *log, int log_index,
@@ -200,13 +211,19 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
   // subtree waves
   const int c = (int)blockIdx.x * (blockDim.x / SG_WAVE) + threadIdx.x / SG_WAVE;
   if (c == nrefresh) {  // bookkeeping
+    // a fused dab before one that is not left its counters in the chain's lines
+    const bool chain_prev = copy0 < (int)gridDim.x && !k.fused;
+    long long *lines = d.ch_ctr + (size_t)((serial + 2) % 3) * SG_CH_SEG * SG_CH_CTR;
     if (lane < SG_CTR_COUNT) {
       if (log && log_index > 0) {
-        const long long prev = d.ctr_next[lane];  // the set the previous dab used
+        // the set the previous dab used
+        const long long prev = chain_prev ? chain_counter(lines, lane) : d.ctr_next[lane];
         log[(size_t)(log_index - 1) * SG_CTR_COUNT + lane] = lane == SG_CTR_NGATHER ? (prev & 0xffffffffll) : prev;
       }
       d.ctr_next[lane] = 0;
     }
+    if (chain_prev)
+      for (int i = lane; i < SG_CH_SEG * SG_CH_CTR; i += SG_WAVE) lines[i] = 0;
     if (lane < 2 * SG_LRN_LINES) d.lrn_next[(lane / 2) * SG_LRN_LINE + lane % 2] = 0;
     if (lane == 0 && d.seq) d.seq[0] += 1;  // this dab's stamp for the later kernels
     if (lane == 0 && undo_active(d)) atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], SG_NGATHER_UNDO);
@@ -995,15 +1012,6 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
   area_flush(sum, d.ch_ctr + ((size_t)((ls + 1) % 3) * SG_CH_SEG + b % SG_CH_AREA) * SG_CH_CTR);
 }
 
-// Counter i (SG_CTR_*) of a chained dab: its lines summed.
-__device__ __forceinline__ long long chain_counter(const long long *lines, int i) {
-  const int f = i == SG_CTR_NAREA ? SG_CH_NAREA : i;
-  if (f > SG_CH_NAREA || i == SG_CH_NAREA) return 0;
-  long long t = 0;
-  for (int q = 0; q < SG_CH_SEG; q++) t += lines[q * SG_CH_CTR + f];
-  return t;
-}
-
 // PLACED: the dab's centre comes from `place`, and its positions go to the mesh's (qx, qy, qz)
 // of this view as well (see sg_enqueue_dab).  An instance of its own: the same tests at run
 // time cost the strokes that are not placed 3 percent (k in vector registers).
@@ -1036,6 +1044,8 @@ __global__ __launch_bounds__(NT) void k_dab_chain(SgDevView d, SgDabK k, SgDabK 
         ca.log[(size_t)(ls - 1) * SG_CTR_COUNT + threadIdx.x] = chain_counter(ctr, threadIdx.x);
       __syncthreads();
       if (threadIdx.x < SG_CH_SEG * SG_CH_CTR) ctr[threadIdx.x] = 0;
+      // the search of the chain's first dab counted in its set, which a dab after the chain may use
+      if (threadIdx.x < SG_CTR_COUNT) d.ctr[threadIdx.x] = d.ctr_next[threadIdx.x] = 0;
       return;
     }
     g0 = o - ca.ns - ca.nc - 1 + ca.f0;
@@ -2066,16 +2076,15 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
   kk.fused = fs.lpt > 0 ? 1 : 0;
   const int leaf_blocks = std::max(1, (p->d.L + 255) / 256);
   const bool chained = kk.fused && p->chain_live;  // the previous dab's launch searched for this one
-  if (!kk.fused && p->fused_pending)
-    if (int rc = sg_enqueue_finish(p, serial - 1)) return rc;
   if (!chained) {
     {
       ProfScope ps(p, SG_K_SEARCH);
       const int nrefresh = place || k.stats ? p->d.C : 0;
       const int cut_blocks = (nrefresh + 1 + 3) / 4;  // a wave per subtree and one for the bookkeeping
-      const int copy_blocks = kk.fused && p->fused_pending ? 128 : 0;
+      const int copy_blocks = p->fused_pending ? 128 : 0;
       SG_LAUNCH(ps, k_search, dim3(leaf_blocks + cut_blocks + copy_blocks), dim3(256), 0, s, v, kk, log, log_index,
                 serial, place, cut_blocks, nrefresh, leaf_blocks + cut_blocks, p->ch_ss);
+      if (!kk.fused) p->fused_pending = false;
     }
     if (kk.fused && k.tool == SG_TOOL_DRAW) {
       ProfScope ps(p, SG_K_AREA);

@@ -255,3 +255,18 @@ def test_largest_fused_leaves(sg, nu, nv, leaf):
     p.stroke(dabs, graph=False)
     assert [v[1] for k, v in p.profile_read().items() if "post" in k] == [0]
     p.close()
+
+
+@pytest.mark.parametrize("breaks", ["orig", "elastic"])
+@pytest.mark.parametrize("run", [1, 2, 3, 4])
+@pytest.mark.parametrize("how", [{"graph": True}, {"graph": False}, {"refit_each": True}])
+def test_chains_between_dabs_that_are_not_fused(sg, breaks, run, how):
+    """Chains of 1 to 4 dabs before each Grab from the original coordinates or elastic deform,
+    whose search takes in the chain's results and counters."""
+    co, tris = sg.noisy_icosphere(5, seed=4, amplitude=0.02)
+    dabs = _path(sg, 15, 2, np.full(15, 0.25), (1, 2, 4, 5), (3, 6))
+    other = {"orig": dict(tool=5, flag=sg.DAB_ORIGINAL),
+             "elastic": dict(tool=sg.TOOL_ELASTIC_DEFORM, elastic_type=sg.ELASTIC_GRAB)}[breaks]
+    for i in range(run, 15, run + 1):
+        dabs[i] = sg.make_dab(location=dabs[i].location, radius=0.3, strength=0.5, grab_delta=(0.01, 0.02, 0), **other)
+    _check(sg, co, tris, dabs, **how)
