@@ -1099,8 +1099,13 @@ __global__ __launch_bounds__(NT) void k_dab_chain(SgDevView d, SgDabK k, SgDabK 
   }
   // the host reads the last dab's lists by gathered leaf: entries before this segment's
   int gbase = 0;
-  if (ca.last)
-    for (int q = 0; q < seg; q++) gbase += (int)lines[q * SG_CH_CTR];
+  if (ca.last) {  // every load ahead of the sum: up to the segment's number they were one after the other
+    int n[SG_CH_SEG];
+#pragma unroll
+    for (int q = 0; q < SG_CH_SEG; q++) n[q] = (int)lines[q * SG_CH_CTR];
+#pragma unroll
+    for (int q = 0; q < SG_CH_SEG; q++) gbase += q < seg ? n[q] : 0;
+  }
   const bool hide = d.vhide && d.respect_hide;
   for (int g = g0; g < ng; g += ca.nf / SG_CH_SEG) {
     const bool first = g == g0;
