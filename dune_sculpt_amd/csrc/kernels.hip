@@ -1016,9 +1016,12 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
 // of this view as well (see sg_enqueue_dab).  An instance of its own: the same tests at run
 // time cost the strokes that are not placed 3 percent (k in vector registers).
 // SMOOTH: a Smooth dab; the others have no Jacobi steps and load no neighbour rows.
+// Two locals a thread with Jacobi steps took 132 VGPRs, 4 past the step to 4 waves a SIMD, and
+// dabs over many leaves ran longer than on the kernel before the chain (Smooth(4) over all of
+// 2.6 M vertices 1.52 ms, 1.35 there): held to 128, without spills, 1.18.
 template <int NT, int LPT, bool SMOOTH, bool PLACED>
-__global__ __launch_bounds__(NT) void k_dab_chain(SgDevView d, SgDabK k, SgDabK kn, const float *curve,
-                                                            SgChainArgs ca, const float *place) {
+__global__ __launch_bounds__(NT, NT == 256 && LPT == 2 && SMOOTH ? 4 : 1) void k_dab_chain(
+    SgDevView d, SgDabK k, SgDabK kn, const float *curve, SgChainArgs ca, const float *place) {
   if (d.halt && d.halt[0]) return;
   if (PLACED) sg_place(k, place);
   extern __shared__ __align__(16) unsigned char fused_smem[];
