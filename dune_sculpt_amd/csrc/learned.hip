@@ -790,7 +790,7 @@ __global__ __launch_bounds__(256) void k_mlp_train(const float *w, const float *
                                                   int n_valid, int base, float inv_count, const float *norm,
                                                   float *grad_part, float *loss_part) {
   __shared__ float sX[TB][TRN_XP], sA1[TB][TRN_HP], sA2[TB][TRN_HP], sZ[TB][TRN_HP];
-  __shared__ float sD[TB][4];
+  __shared__ __align__(16) float sD[TB][4];  // rows read as float4
   __shared__ float sLoss[2];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 15, g = lane >> 4;
   const int j = wv * 16 + c;
