@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <vector>
 
@@ -633,6 +634,10 @@ __global__ __launch_bounds__(GR_THREADS) void kg_edges_verts(GView g) {
 #define DF_MAX_EPT 16   // passes over a face at most (the affected flags are a bit per pass)
 #define GR_LINES 16     // counter lines: [0] affected elements and, from bit 40, faces; [1] edges and vertices
 #define GR_LINE 16      // long longs per line
+// More faces than this and the tests of all faces and edges are bound by the lines that they
+// load, not by their chains: dabs of r 0.01 and 0.1 on 960 k faces (level 2) took 108 and 157 us
+// with a line per record, 65 and 124 with four records a line and the ranges of the hit ones.
+#define GR_SCAN_FACES 65536
 
 __device__ __forceinline__ bool face_gathered(const GView &g, const int4 &fl, int serial) {
   const int a = g.leaf_gmark[fl.x], b = g.leaf_gmark[fl.y], c = g.leaf_gmark[fl.z];
@@ -662,17 +667,27 @@ __global__ __launch_bounds__(DF_THREADS) void kg_dab_faces(GView g, SgDabK k, co
     oz = (az * k.r) * k.bstr;
   }
   if (tid == 0) s_naff = s_nface = 0;
+  const int grp = g.F > GR_SCAN_FACES ? 4 : 1;
   for (int base = 0; base < g.F; base += gridDim.x * DF_THREADS) {
     if (tid == 0) s_n = 0;
     __syncthreads();
-    // the workgroup's faces of this round (every gridDim-th), a thread each
-    const int f = base + (int)blockIdx.x + tid * (int)gridDim.x;
+    // the workgroup's faces of this round (every gridDim-th), a thread each; in large meshes
+    // four neighbours each time, whose records share a line, and the ranges of the hit ones only
+    const int f = base + (int)blockIdx.x * grp + tid / grp * grp * (int)gridDim.x + tid % grp;
     if (f < g.F) {
       const int4 fl = g.face_leaf[f];
-      const int g0 = g.face_gbeg[f], n = g.face_gbeg[f + 1] - g0;
+      int g0 = 0, n = 0;
+      if (grp == 1 || fl.w == -2) {
+        g0 = g.face_gbeg[f];
+        n = g.face_gbeg[f + 1] - g0;
+      }
       bool hit = face_gathered(g, fl, serial);
       if (fl.w == -2 && !hit)  // grids in more leaves than the record holds
         for (int c = 0; c < n && !hit; c++) hit = g.leaf_gmark[g.grid_pl[g0 + c].y] == serial;
+      if (hit && n == 0) {
+        g0 = g.face_gbeg[f];
+        n = g.face_gbeg[f + 1] - g0;
+      }
       if (hit) s_list[atomicAdd(&s_n, 1)] = make_int4(f, g0, n, 0);
     }
     __syncthreads();
@@ -885,7 +900,8 @@ __device__ __forceinline__ void avg_few(const GView &g, const int *els, int stri
 
 // The averages of kg_edges_verts for the edges and vertices the face kernel stamped: a lane
 // checks an item (every wave-count-th, so that neighbours go to different waves), the wave
-// then takes the stamped ones.
+// then takes the stamped ones.  In large meshes (GR_SCAN_FACES) a lane checks four, which lie
+// four to a line, ahead of any that it takes, and loads the ranges of the stamped ones only.
 __global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
   __shared__ int s_n;
   if (threadIdx.x == 0) s_n = 0;
@@ -896,18 +912,15 @@ __global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
   const int nw = gridDim.x * blockDim.x / SG_WAVE;
   const int n2 = 2 * g.gs, total = g.Ed + g.Vc;
   int cnt = 0;
-  for (int base = 0; base < total; base += nw * SG_WAVE) {
-    const int item = base + w + lane * nw;
-    bool hit = false;
-    int fb = 0, nf = 0;
-    if (item < total) {
-      const bool edge = item < g.Ed;
-      const int j = edge ? item : item - g.Ed;
-      const int *off = edge ? g.edge_foff : g.vert_foff;
-      hit = (edge ? g.edge_stamp[j] : g.vert_stamp[j]) == serial;
-      fb = off[j];
-      nf = off[j + 1] - fb;
-    }
+  auto stamp_of = [&](int item) { return item < g.Ed ? g.edge_stamp[item] : g.vert_stamp[item - g.Ed]; };
+  auto range_of = [&](int item, int &fb, int &nf) {
+    const bool edge = item < g.Ed;
+    const int j = edge ? item : item - g.Ed;
+    const int *off = edge ? g.edge_foff : g.vert_foff;
+    fb = off[j];
+    nf = off[j + 1] - fb;
+  };
+  auto take = [&](int item, bool hit, int fb, int nf) {
     unsigned long long m = __ballot(hit);
     cnt += __popcll(m);
     while (m) {
@@ -927,6 +940,34 @@ __global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
           avg_few(g, g.vert_el + b, 1, n, serial);
         else
           avg_list(g, g.vert_el + b, 1, n, serial);
+      }
+    }
+  };
+  if (g.F <= GR_SCAN_FACES) {
+    for (int base = 0; base < total; base += nw * SG_WAVE) {
+      const int item = base + w + lane * nw;
+      bool hit = false;
+      int fb = 0, nf = 0;
+      if (item < total) {
+        hit = stamp_of(item) == serial;
+        range_of(item, fb, nf);
+      }
+      take(item, hit, fb, nf);
+    }
+  } else {
+    for (int base = 0; base < total; base += 4 * nw * SG_WAVE) {
+      int item[4], st[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        item[u] = base + (u * SG_WAVE + lane / 4 * 4) * nw + 4 * w + lane % 4;
+        st[u] = stamp_of(min(item[u], total - 1));
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const bool hit = item[u] < total && st[u] == serial;
+        int fb = 0, nf = 0;
+        if (hit) range_of(item[u], fb, nf);
+        take(item[u], hit, fb, nf);
       }
     }
   }
@@ -1345,6 +1386,23 @@ int sg_grids_build_device(PBVH *p) {
       }
     }
   }
+  {  // leaves per unit of surface area, from up to 4096 grids (their corners' quads)
+    const int step = std::max(1, d.G / 4096), c[4] = {0, d.gs - 1, d.ga - 1, d.ga - d.gs};
+    double area = 0.0;
+    int n = 0;
+    for (int g = 0; g < d.G; g += step, n++) {
+      double u[2][3];
+      for (int i = 0; i < 2; i++) {
+        const size_t a = (size_t)g * d.ga + c[i], b = (size_t)g * d.ga + c[i + 2];
+        u[i][0] = (double)x[b] - x[a], u[i][1] = (double)y[b] - y[a], u[i][2] = (double)z[b] - z[a];
+      }
+      const double cx = u[0][1] * u[1][2] - u[0][2] * u[1][1], cy = u[0][2] * u[1][0] - u[0][0] * u[1][2],
+                   cz = u[0][0] * u[1][1] - u[0][1] * u[1][0];
+      area += 0.5 * std::sqrt(cx * cx + cy * cy + cz * cz);
+    }
+    if (n > 0) area *= (double)d.G / n;
+    p->leaf_density = area > 0.0 && area < 1e30 ? d.L / area : 0.0;
+  }
   // tree tables: leaf boxes, internal nodes by height
   std::vector<float> lbb((size_t)d.L * 8, 0.0f), lobb((size_t)d.L * 8, 0.0f), nbb((size_t)d.N * 8, 0.0f),
       nobb((size_t)d.N * 8, 0.0f);
@@ -1546,6 +1604,18 @@ int sg_grids_settle(PBVH *p) {
   return 0;
 }
 
+// Whether dab k runs per face.  Testing every face and edge costs a mesh of many faces more
+// than listing those of the gathered leaves does, unless the dab gathers many: the lists take
+// an atomic for each.  240 k faces (level 3, 100 to a leaf), per face / per leaf: r 0.01 53 / 44
+// us a dab, r 0.03 56 / 50, r 0.1 74 / 103; 277 to a leaf (level 2), r 0.01 53 / 66, r 0.1 65 /
+// 102; 540 k, r 0.01 57 / 49 and 56 / 61, r 0.1 96 / 156 and 85 / 152; 60 k, r 0.01 39 / 40.
+static bool grid_per_face(const SgGridDev &d, double leaf_density, const SgDabK &k) {
+  if (d.face_lds <= 0) return false;
+  if (d.F <= GR_SCAN_FACES) return true;
+  const double across = 1.0 + 2.0 * (double)k.r * std::sqrt(leaf_density);  // leaves, on a surface
+  return across * across * d.F / d.L >= 340.0;
+}
+
 static bool grid_tool(const SgDabK &k) {
   return k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_SMOOTH || k.tool == SG_TOOL_GRAB;
 }
@@ -1570,7 +1640,7 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   d.ctr_unclean = true;
   if (!searched) kg_search<<<(d.L + GR_THREADS - 1) / GR_THREADS, GR_THREADS, 0, p->stream>>>(g, k);
   if (k.tool == SG_TOOL_DRAW) kg_area<<<eb, GR_THREADS, 0, p->stream>>>(g, k, rh);
-  if (normals && d.face_lds > 0) {
+  if (normals && grid_per_face(d, p->leaf_density, k)) {
     const float *s[3] = {d.px, d.py, d.pz};
     if (k.tool == SG_TOOL_SMOOTH) {
       if (k.iters < 1) {

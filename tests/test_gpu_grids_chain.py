@@ -128,3 +128,23 @@ def test_stroke_with_a_refused_dab(sg, bad):
         got.append(_all(p))
         p.close()
     assert all(np.asarray(x).tobytes() == np.asarray(y).tobytes() for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("level,leaf_limit", [(2, 10000), (3, 2500)])
+def test_many_faces(sg, po, level, leaf_limit):
+    """A base of 66 k faces, past the line where faces and edges are tested four to a line and
+    small dabs run per leaf: both kinds of dab in one stroke, against the oracle."""
+    g, mesh = noisy_sphere_grids(sg, 105, level, seed=5)
+    o = oracle_of(po, g, mesh, leaf_limit)
+    p = gr.GridPBVH(g, leaf_limit=leaf_limit)
+    small, wide = stroke(sg, 3, 8, 0.01, 0.03), stroke(sg, 4, 8, 0.1, 0.4)
+    dabs = [d for i in range(8) for d in (small[i], wide[i], small[(i + 1) % 8])]
+    p.stroke(dabs)
+    for d in dabs:
+        o.dab(po.to_orc(d))
+    for x, y in zip(p.state()[:2], o.state()[:2]):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    for x, y in zip(p.boxes(), o.boxes()):
+        assert np.array_equal(x, y)
+    p.close()
+    o.close()
