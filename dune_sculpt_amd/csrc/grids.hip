@@ -644,6 +644,9 @@ __device__ __forceinline__ bool face_gathered(const GView &g, const int4 &fl, in
   return a == serial || b == serial || c == serial;
 }
 
+// MANY (more than GR_SCAN_FACES faces): an instance of its own, as is that of the edges; the
+// choice at run time cost the others 2 percent of a dab.
+template <bool MANY>
 __global__ __launch_bounds__(DF_THREADS) void kg_dab_faces(GView g, SgDabK k, const float *curve, int respect_hide,
                                                            const float *sx, const float *sy, const float *sz) {
   extern __shared__ float s_face[];
@@ -667,7 +670,7 @@ __global__ __launch_bounds__(DF_THREADS) void kg_dab_faces(GView g, SgDabK k, co
     oz = (az * k.r) * k.bstr;
   }
   if (tid == 0) s_naff = s_nface = 0;
-  const int grp = g.F > GR_SCAN_FACES ? 4 : 1;
+  constexpr int grp = MANY ? 4 : 1;
   for (int base = 0; base < g.F; base += gridDim.x * DF_THREADS) {
     if (tid == 0) s_n = 0;
     __syncthreads();
@@ -677,14 +680,14 @@ __global__ __launch_bounds__(DF_THREADS) void kg_dab_faces(GView g, SgDabK k, co
     if (f < g.F) {
       const int4 fl = g.face_leaf[f];
       int g0 = 0, n = 0;
-      if (grp == 1 || fl.w == -2) {
+      if (!MANY || fl.w == -2) {
         g0 = g.face_gbeg[f];
         n = g.face_gbeg[f + 1] - g0;
       }
       bool hit = face_gathered(g, fl, serial);
       if (fl.w == -2 && !hit)  // grids in more leaves than the record holds
         for (int c = 0; c < n && !hit; c++) hit = g.leaf_gmark[g.grid_pl[g0 + c].y] == serial;
-      if (hit && n == 0) {
+      if (MANY && hit && n == 0) {
         g0 = g.face_gbeg[f];
         n = g.face_gbeg[f + 1] - g0;
       }
@@ -902,6 +905,7 @@ __device__ __forceinline__ void avg_few(const GView &g, const int *els, int stri
 // checks an item (every wave-count-th, so that neighbours go to different waves), the wave
 // then takes the stamped ones.  In large meshes (GR_SCAN_FACES) a lane checks four, which lie
 // four to a line, ahead of any that it takes, and loads the ranges of the stamped ones only.
+template <bool MANY>
 __global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
   __shared__ int s_n;
   if (threadIdx.x == 0) s_n = 0;
@@ -943,7 +947,7 @@ __global__ __launch_bounds__(GR_THREADS) void kg_dab_edges(GView g) {
       }
     }
   };
-  if (g.F <= GR_SCAN_FACES) {
+  if (!MANY) {
     for (int base = 0; base < total; base += nw * SG_WAVE) {
       const int item = base + w + lane * nw;
       bool hit = false;
@@ -1656,9 +1660,11 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
         if (k.iters & 1) s[0] = d.qx, s[1] = d.qy, s[2] = d.qz;
       }
     }
-    kg_dab_faces<<<std::max(1, std::min(d.F, 2048)), DF_THREADS, d.face_lds, p->stream>>>(g, k, curve_dev, rh, s[0], s[1],
-                                                                                        s[2]);
-    kg_dab_edges<<<std::max(1, std::min((d.Ed + d.Vc + 3) / 4, 1024)), GR_THREADS, 0, p->stream>>>(g);
+    const bool many = d.F > GR_SCAN_FACES;
+    const dim3 gf(std::max(1, std::min(d.F, 2048))), ge(std::max(1, std::min((d.Ed + d.Vc + 3) / 4, 1024)));
+    (many ? kg_dab_faces<true> : kg_dab_faces<false>)<<<gf, DF_THREADS, d.face_lds, p->stream>>>(g, k, curve_dev, rh, s[0],
+                                                                                               s[1], s[2]);
+    (many ? kg_dab_edges<true> : kg_dab_edges<false>)<<<ge, GR_THREADS, 0, p->stream>>>(g);
     // one workgroup searches 256 leaves at a time: past a few rounds a launch of its own is
     // shorter; a dab that will be refused leaves no search behind
     const bool search = next && d.L <= 4 * GR_THREADS && grid_tool(*next) && !next->learned && !next->orig_co;
