@@ -1647,18 +1647,14 @@ int sg_grids_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long 
   if (normals && grid_per_face(d, p->leaf_density, k)) {
     const float *s[3] = {d.px, d.py, d.pz};
     if (k.tool == SG_TOOL_SMOOTH) {
-      if (k.iters < 1) {
-        kg_brush<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh, 0);
-      } else {
-        kg_smooth_first<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh);
-        for (int it = 1; it < k.iters; it++) {
-          if (it & 1)
-            kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.qx, d.qy, d.qz, d.px, d.py, d.pz);
-          else
-            kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.px, d.py, d.pz, d.qx, d.qy, d.qz);
-        }
-        if (k.iters & 1) s[0] = d.qx, s[1] = d.qy, s[2] = d.qz;
+      kg_smooth_first<<<eb, GR_THREADS, 0, p->stream>>>(g, k, curve_dev, rh);
+      for (int it = 1; it < k.iters; it++) {
+        if (it & 1)
+          kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.qx, d.qy, d.qz, d.px, d.py, d.pz);
+        else
+          kg_smooth<<<eb, GR_THREADS, 0, p->stream>>>(g, d.px, d.py, d.pz, d.qx, d.qy, d.qz);
       }
+      if (k.iters & 1) s[0] = d.qx, s[1] = d.qy, s[2] = d.qz;
     }
     const bool many = d.F > GR_SCAN_FACES;
     const dim3 gf(std::max(1, std::min(d.F, 2048))), ge(std::max(1, std::min((d.Ed + d.Vc + 3) / 4, 1024)));

@@ -860,8 +860,8 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 // so a dab waits for one kernel boundary instead of two (three for Draw) and for no
 // search.  Bound by the chain of dependent loads, not by bytes.  As search, area normal
 // and brush kernels 240 mixed dabs on a 2.6 M-vertex mesh took 3.47 ms with the draw
-// refill after them, now 2.24; 200 Draw dabs on 41 k vertices 2.67 and 1.58; 24 dabs over
-// about 1250 leaves each 0.94 and 0.76.  The first dab of a chain has its own search (and
+// refill after them, now 2.20; 200 Draw dabs on 41 k vertices 2.67 and 1.56; 24 dabs over
+// about 1250 leaves each 0.94 and 0.73.  The first dab of a chain has its own search (and
 // k_area).
 //
 // F works on the leaf's halo (its uniq vertices, ring 0 = its shared vertices and their
@@ -891,7 +891,8 @@ __global__ __launch_bounds__(256) void k_post(SgDevView d, int stats, int stamp,
 #define FUSED_LEAD 256  // F blocks started before the S and C blocks: more leaves than most dabs gather
 #define FUSED_ROW 8  // neighbour / incidence entries per local held in registers
 
-// F: one workgroup per gathered leaf; each thread holds LPT locals (local i = tid + j * 256).
+// F: one workgroup (NT threads) per gathered leaf; each thread holds LPT locals (local i = tid +
+// j * NT).
 // Global loads come in three dependent levels, each issued for every local at once:
 //   1  the counters and the workgroup's first gathered leaf (ranges, halo header)
 //   2  halo vertex ids, neighbour-row and incidence ranges, shared-vertex local ids
@@ -2032,7 +2033,7 @@ struct FusedShape {
 static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
   FusedShape f;
   const bool tool = k.tool == SG_TOOL_DRAW || k.tool == SG_TOOL_INFLATE || k.tool == SG_TOOL_GRAB ||
-                    (k.tool == SG_TOOL_SMOOTH && k.iters >= 1);
+                    k.tool == SG_TOOL_SMOOTH;
   if (!p->d.halo_ok || !p->fused_enabled || !tool || k.stats || k.orig_co || (k.learned && p->mlp)) return f;
   if (k.tool == SG_TOOL_SMOOTH) f.launches = (k.iters + SG_HALO_RINGS - 1) / SG_HALO_RINGS;
   const int steps = k.tool == SG_TOOL_SMOOTH ? (k.iters + f.launches - 1) / f.launches : 0;  // most in one launch
@@ -2041,8 +2042,8 @@ static FusedShape fused_shape(PBVH *p, const SgDabK &k) {
   f.lds = (size_t)f.cap * 2 * sizeof(float4) + (size_t)f.fcap * sizeof(float4) + (size_t)(p->d.leaf_maxsh + 2) * 2 + 16;
   // A Smooth dab's halo is two to three times its leaf, so 512 threads with a local each run
   // shorter than 256 with two, while every gathered leaf has a workgroup in flight: two of 512
-  // threads fit a CU, three of 256.  60 Smooth(8) dabs over some 60 leaves: 1.26 ms with 256,
-  // 1.18 with 512; 24 mixed ones over 700 to 4000: 0.76 and 0.78.
+  // threads fit a CU, four of 256.  60 Smooth(8) dabs over some 60 leaves: 1.32 ms with 256,
+  // 1.18 with 512; 24 mixed ones over 700 to 4000: 0.77 and 0.83.
   const double reach = (double)k.r + 0.5 / std::sqrt(std::max(p->leaf_density, 1e-30));
   const bool few = 3.14159 * reach * reach * p->leaf_density <= 512.0;  // leaves the dab gathers on a surface
   f.threads = k.tool == SG_TOOL_SMOOTH && f.cap > FUSED_THREADS && few ? 2 * FUSED_THREADS : FUSED_THREADS;

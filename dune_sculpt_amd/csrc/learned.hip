@@ -331,20 +331,21 @@ __global__ __launch_bounds__(LRN_THREADS) void k_mlp_predict(SgMlpView m, const 
 }
 
 // ---------------------------------------------------------------------------
-// Learned dab.  k_brush_learned: work items (gathered leaf, slot), the wave of slot t
-// takes the leaf's 16-vertex tiles t, t+4, ...: sphere test and factor as the plain
-// Smooth brush, then features -> MLP (MFMA, 16 rows) -> predicted position written to
-// the shadow copy; affected vertices get the dab's stamp.  The error estimate
-// sum((|d|/r)^2) (2^-32 fixed point), the out-of-range count and the affected count
-// are reduced per block and added once per block.
+// Learned dab.  k_brush_learned: work items (gathered leaf, slot), slot t of n takes the
+// leaf's 16-vertex tiles t, t+n, ...; a slot is a workgroup on a single mesh, a wave in
+// the batch (k_bbrush_learned).  Sphere test and factor as the plain Smooth brush, then
+// features -> MLP (MFMA, 16 rows) -> predicted position written to the shadow copy;
+// affected vertices get the dab's stamp.  The error estimate sum((|d|/r)^2) (2^-32 fixed
+// point), the out-of-range count and the affected count are added once per workgroup
+// (batch: once per item).
 // k_post_learned: accept (error estimate and range checks within tolerance): normals
 // and leaf bounds from the shadow copy, commit it to the positions; reject: undo the
 // shadow copy and raise the halt flag so the rest of the stroke stops and the host
 // runs this dab with the plain brush.  Both walk the gathered leaves' vertex ranges
 // and test the stamp (no per-vertex list, so no slot reservations).
 // ---------------------------------------------------------------------------
-#define LRN_SLOTS 4   // waves per gathered leaf (batch)
-#define LRN_DSLOTS 8  // waves per gathered leaf (single mesh): one 16-row tile each for leaves up to 128 uniq vertices
+#define LRN_SLOTS 4   // slots of a gathered leaf, a wave each (batch)
+#define LRN_DSLOTS 8  // slots of a gathered leaf, a workgroup each (single mesh): a tile each for leaves up to 128 uniq vertices
 
 // Evaluate one 16-vertex tile of a learned dab (every lane of the wave calls it; lanes
 // < 16 own a vertex).  Returns the Smooth factor of the lane's vertex.
@@ -401,7 +402,9 @@ __device__ __forceinline__ BrushIn learned_tile_load(const SgDevView &d, const S
 // each wave holds a quarter of the hidden columns, its weight fragments in registers.  Same
 // products and sums in the same order as learned_eval.  A wave per tile, a lane per vertex,
 // spent 5.8 us on the features and 3.0 on the network and the kernel took 14.7 us (1050
-// affected vertices, 37 leaves); now 8.7.
+// affected vertices, 37 leaves); now 8.7.  It stays the shorter one where the tiles are many
+// times the chip's: a learned dab took 381 us over 7900 leaves, now 278; 10 leaves 39 and 28.
+// The batch keeps the wave per tile: its meshes fill the chip with tiles of their own.
 __global__ __launch_bounds__(LRN_THREADS) void k_brush_learned(SgDevView d, SgDabK k, const float *curve,
                                                                SgMlpView m, const float *place) {
   __shared__ __align__(16) uint16_t bufA[LRN_ROWS * MLP_ST];

@@ -10,7 +10,7 @@ enum {
   SG_CTR_FA = 12,     // distinct tris incident to the affected set (stats mode)
   SG_CTR_VFA = 13,    // distinct vertices of those tris (stats mode)
   SG_CTR_SHARED = 14, // shared vertices read by the leaf refit
-  SG_CTR_LERR = 15,   // learned Smooth: sum (|d|/r)^2 in 2^-40 fixed point
+  SG_CTR_LERR = 15,   // learned Smooth: sum (|d|/r)^2 in 2^-32 fixed point
   SG_CTR_LOOD = 16,   // learned Smooth: vertices outside the trained range
   SG_CTR_LACC = 17,   // learned Smooth: 1 when the dab was accepted
 };

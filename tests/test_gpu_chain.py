@@ -62,7 +62,7 @@ def test_lengths(sg, n, graph):
 @pytest.mark.parametrize("tools,ks", [((1,), (1,)), ((1, 2), (4,)), ((2,), (1, 5, 4, 9)), ((4, 5, 1), (1,)),
                                       ((1, 2, 2), (3, 6))])
 def test_broken_chains(sg, tools, ks):
-    """Smooth with more steps than the halo covers runs the separate kernels in between."""
+    """Smooth with more steps than a launch covers, as several launches between dabs of one."""
     co, tris = sg.noisy_icosphere(5, seed=4, amplitude=0.02)
     _check(sg, co, tris, _path(sg, 24, 2, np.full(24, 0.15), tools, ks))
 
