@@ -168,7 +168,20 @@ int upload_host_leaf_verts(PBVH *p, const std::vector<int> &leaves) {
       if (int rc = sg_check_hip(hipMemcpy(dst[a] + b, src[a], n * 4, hipMemcpyHostToDevice), "copy")) return rc;
     i = j + 1;
   }
-  return 0;
+  // until they are refit, the boxes of the owners (among them leaves that only share a
+  // vertex with a listed one) lag
+  std::vector<int> owner;
+  for (int v : idx) {
+    const int l = (int)(std::upper_bound(p->leaf_vbeg.begin(), p->leaf_vbeg.end(), v) - p->leaf_vbeg.begin()) - 1;
+    if (owner.empty() || owner.back() != l) owner.push_back(l);  // (idx is sorted)
+  }
+  if (owner.empty()) return 0;
+  int *dl = (int *)stage(p, owner.size() * sizeof(int));
+  if (!dl) return -1;
+  int rc = sg_check_hip(hipMemcpyAsync(dl, owner.data(), owner.size() * sizeof(int), hipMemcpyHostToDevice, p->stream),
+                        "copy");
+  if (!rc) rc = sg_enqueue_box_lag(p, dl, (int)owner.size());
+  return rc ? rc : sg_check_hip(hipStreamSynchronize(p->stream), "upload");
 }
 
 std::vector<int> flagged_leaves(PBVH *p, int flag) {
@@ -1606,6 +1619,7 @@ void BKE_pbvh_update_bounds(PBVH *p, int flag) {  // pbvh.c:1401-1421
       r.ob[k] = n.orig_vb[k];
       r.ob[4 + k] = n.orig_vb[3 + k];
     }
+    r.vb[3] = 1.0f;  // taken to lag: UpdateOriginalBB alone brings no new box
     return r;
   };
   for (size_t i = 0; i < nl; i++) {  // pbvh_update_BB_redraw_task_cb (pbvh.c:1206-1227)

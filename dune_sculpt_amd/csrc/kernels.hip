@@ -949,17 +949,14 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
                                              int *s_nq) {
   const int lane = lane_id();
   if (threadIdx.x == 0) *s_nq = 0;
-  // Before a Draw dab a block takes a wave's leaves only, and all its waves share their
-  // vertices: with a leaf per thread a block could meet over a hundred new leaves, 30 to 40 of
-  // them after one another on each wave (240 mixed dabs on 2.6 M vertices 2.29 ms, now 2.23;
-  // 24 wide ones 0.82 and 0.81).
-  const int per = kn.tool == SG_TOOL_DRAW ? SG_WAVE : (int)blockDim.x;
-  const int l = b * per + threadIdx.x, lc = min(l, d.L - 1);
-  const BB6 bb = bb_load((kn.use_orig ? d.leaf_obb : d.leaf_bb) + 8 * (size_t)lc);
+  const int gstamp = d.dstamp[0] + ls, stamp = d.dstamp[0] + ss;
+  const int l = b * blockDim.x + threadIdx.x, lc = min(l, d.L - 1);
+  const float *box = (kn.use_orig ? d.leaf_obb : d.leaf_bb) + 8 * (size_t)lc;
+  const BB6 bb = bb_load(box);
+  const float lag = box[3];
   const int gs = d.ch_gstamp[(size_t)(ls & 1) * d.L + lc];
   const int fl = kn.hide_skip ? d.leaf_flags[lc] : 0;
-  const int gstamp = d.dstamp[0] + ls, stamp = d.dstamp[0] + ss;
-  const bool pass = (int)threadIdx.x < per && l < d.L && gs != gstamp && !(fl & kn.hide_skip) && sphere_box(bb, kn.cx, kn.cy, kn.cz, kn.r2);
+  const bool pass = l < d.L && gs != gstamp && !(fl & kn.hide_skip) && sphere_box(bb, kn.cx, kn.cy, kn.cz, kn.r2);
   const unsigned long long m = __ballot(pass);
   int4 r0 = make_int4(0, 0, 0, 0), r1 = make_int4(0, 0, 0, 0);
   if (m) {
@@ -968,12 +965,21 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
     chain_append(d, ls + 1, l, pass, m, r0, r1, gstamp + 1);
   }
   if (kn.tool != SG_TOOL_DRAW) return;
-  // The area normal's share of the new leaves, two leaves a wave at a time.  Every vertex is
-  // tested, as k_area does: a leaf's box does not always hold its vertices (a host edit without
-  // a bounds update, a fold over a NaN).  The normals load only where a vertex lies in the
-  // sphere (usually none: the dab before covered it).
+  // The area normal's share of the new leaves that reach into its sphere (usually none: the dab
+  // before covered it), two leaves a wave at a time; the normals load only where a vertex lies
+  // in it.  A vertex with d2 <= nr2 lies in its leaf's box, whose distance, rounded the same
+  // way, is not larger, unless the box lags its vertices (bb_store): then every vertex is
+  // tested, as k_area does.  Testing them always cost 1000 mixed dabs on 10.5 M vertices 11.5
+  // ms, where the boxes' test takes 10.7.
+  float t2 = 0.0f;
+  {
+    const float cc[3] = {kn.cx, kn.cy, kn.cz};
+    float t[3];
+    for (int i = 0; i < 3; i++) t[i] = cc[i] - (bb.mn[i] > cc[i] ? bb.mn[i] : (bb.mx[i] < cc[i] ? bb.mx[i] : cc[i]));
+    t2 = t[0] * t[0] + t[1] * t[1] + t[2] * t[2];
+  }
   __syncthreads();
-  if (pass) s_q[atomicAdd(s_nq, 1)] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
+  if (pass && (lag != 0.0f || t2 <= kn.nr2)) s_q[atomicAdd(s_nq, 1)] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
   __syncthreads();
   const int nq = *s_nq, nw = blockDim.x / SG_WAVE;
   if (nq == 0) return;
@@ -1343,17 +1349,20 @@ __global__ __launch_bounds__(NT, NT == 256 && LPT == 2 && SMOOTH ? 4 : 1) void k
       const int tot = nu + ns, per = (tot + SG_WAVE - 1) / SG_WAVE;
       BB6 acc;
       bb_reset(acc);
+      bool nan = false;
       for (int c = 0; c < per; c++) {
         const int i = lane * per + c;
         if (i < tot) {
           const float4 pu = F[i < nu ? i : Sshl[i - nu]];
           bb_add_point(acc, pu.x, pu.y, pu.z);
+          nan = nan || pu.x != pu.x || pu.y != pu.y || pu.z != pu.z;
         }
       }
+      nan = __any(nan);
       acc = bb_wave_scan(acc);
       if (lane == SG_WAVE - 1) {
-        bb_store(d.leaf_bb + 8 * (size_t)leaf, acc);
-        bb_store(d.leaf_obb + 8 * (size_t)leaf, acc);
+        bb_store(d.leaf_bb + 8 * (size_t)leaf, acc, nan);
+        bb_store(d.leaf_obb + 8 * (size_t)leaf, acc, nan);
         d.cut_dirty[cut] = 1;
         d.draw_dirty[cut] = 1;  // the subtree's leaves need new draw records (UpdateDrawBuffers)
         if (ca.last) d.gathered[gbase + g] = leaf;
@@ -1767,9 +1776,10 @@ __global__ __launch_bounds__(256) void k_leaf_boxes(SgDevView d, const int *leav
   const int nw = gridDim.x * blockDim.x / SG_WAVE;
   for (int g = gw; g < n; g += nw) {
     const int leaf = leaves[g];
+    bool lag;
     const BB6 b = leaf_box(d, make_int2(d.leaf_vbeg[leaf], d.leaf_vbeg[leaf + 1]),
-                           make_int2(d.leaf_sh_off[leaf], d.leaf_sh_off[leaf + 1]));
-    if (lane_id() == 0) bb_store(out + 8 * (size_t)g, b);
+                           make_int2(d.leaf_sh_off[leaf], d.leaf_sh_off[leaf + 1]), lag);
+    if (lane_id() == 0) bb_store(out + 8 * (size_t)g, b, lag);
   }
 }
 
@@ -1791,6 +1801,12 @@ __global__ __launch_bounds__(256) void k_scatter_boxes(SgDevView d, const SgBoxR
     else
       ob[8 * (size_t)r.idx + k - 8] = r.ob[k - 8];
   }
+}
+
+// The boxes of the leaves that own uploaded vertices lag until they are refit (bb_store).
+__global__ __launch_bounds__(256) void k_box_lag(SgDevView d, const int *leaves, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    d.leaf_bb[8 * (size_t)leaves[i] + 3] = 1.0f;
 }
 
 // Host marks (BKE_pbvh_vert_mark_update) join the device's marks: list of new ids.
@@ -2133,8 +2149,7 @@ int sg_enqueue_dab(PBVH *p, const SgDabK &k, const float *curve_dev, long long *
       ca.has_next = has_next && !ca.cont_out ? 1 : 0;
       ca.has_prev = prev && !ca.cont_in ? 1 : 0;
       ca.last = !has_next && !ca.cont_out ? 1 : 0;
-      const int per = kn.tool == SG_TOOL_DRAW ? SG_WAVE : fs.threads;  // leaves of an S block
-      ca.ns = ca.has_next ? std::max(1, (p->d.L + per - 1) / per) : 0;
+      ca.ns = ca.has_next ? std::max(1, (p->d.L + fs.threads - 1) / fs.threads) : 0;
       ca.nc = chained && !ca.cont_in ? 128 * FUSED_THREADS / fs.threads : 0;
       ProfScope ps(p, SG_K_BRUSH);
       const dim3 gf(ca.nf + ca.ns + ca.nc + 1), bf(fs.threads);
@@ -2305,6 +2320,12 @@ int sg_enqueue_leaf_boxes(PBVH *p, const int *leaves_dev, int n, float *out_dev)
   if (n > 0) hipLaunchKernelGGL(k_leaf_boxes, dim3(std::max(1, std::min(p->grid_wg, (n + 3) / 4))), dim3(256), 0,
                                 p->stream, v, leaves_dev, n, out_dev);
   return sg_check_hip(hipGetLastError(), "leaf boxes launch");
+}
+
+int sg_enqueue_box_lag(PBVH *p, const int *leaves_dev, int n) {
+  const SgDevView v = sg_view(p);
+  hipLaunchKernelGGL(k_box_lag, dim3(std::max(1, std::min((n + 255) / 256, 1024))), dim3(256), 0, p->stream, v, leaves_dev, n);
+  return sg_check_hip(hipGetLastError(), "box launch");
 }
 
 int sg_enqueue_scatter_boxes(PBVH *p, const void *recs_dev, int n) {

@@ -890,6 +890,11 @@ void sg_build_device(PBVH *p, const float *co) {
     if (n > 0) area *= (double)T / n;
     p->leaf_density = area > 0.0 && area < 1e30 ? L / area : 0.0;
   }
+  {  // a box folded over a NaN need not hold its leaf's vertices (bb_store's lag)
+    bool nan = false;
+    for (int v = 0; v < V; v++) nan |= h.x[v] != h.x[v] || h.y[v] != h.y[v] || h.z[v] != h.z[v];
+    for (int l = 0; l < L && nan; l++) h.leaf_bb[8 * (size_t)l + 3] = 1.0f;
+  }
   upload(&d.px, h.x.data(), V, s);
   upload(&d.py, h.y.data(), V, s);
   upload(&d.pz, h.z.data(), V, s);

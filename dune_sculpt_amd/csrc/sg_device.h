@@ -152,8 +152,12 @@ __device__ __forceinline__ BB6 bb_load(const float *p) {
   r.mx[2] = b.z;
   return r;
 }
-__device__ __forceinline__ void bb_store(float *p, const BB6 &b) {
-  *(float4 *)p = make_float4(b.mn[0], b.mn[1], b.mn[2], 0.0f);
+// lag (word 3 of a box): not 0 when the box need not hold every vertex of its leaf: one is a
+// NaN, which the fold's comparisons lose the values before it by, or a host edit moved one and
+// no refit followed.  The dab search decides by the box all the same, as the reference does;
+// what would only skip work by it must look.
+__device__ __forceinline__ void bb_store(float *p, const BB6 &b, bool lag = false) {
+  *(float4 *)p = make_float4(b.mn[0], b.mn[1], b.mn[2], lag ? 1.0f : 0.0f);
   *(float4 *)(p + 4) = make_float4(b.mx[0], b.mx[1], b.mx[2], 0.0f);
 }
 // wave-ordered reduction: lane i's box covers elements before lane i+1's.
@@ -576,24 +580,26 @@ __device__ __forceinline__ void vertex_normal(const SgDevView &d, int v, int b, 
 // Leaf bounds over ALL its vertices, uniq then shared (update_node_vb pbvh.c:108-128,
 // BB_expand in vert_indices order).  Each lane folds a contiguous chunk, then the
 // wave combines lanes in order.  Writes vb and orig_vb (UpdateOriginalBB).
-__device__ __forceinline__ BB6 leaf_box(const SgDevView &d, int2 vr, int2 sr);
+__device__ __forceinline__ BB6 leaf_box(const SgDevView &d, int2 vr, int2 sr, bool &lag);
 __device__ __forceinline__ void leaf_refit(const SgDevView &d, int leaf, int2 vr, int2 sr, long long &nsh) {
-  const BB6 acc = leaf_box(d, vr, sr);
+  bool lag;
+  const BB6 acc = leaf_box(d, vr, sr, lag);
   if (lane_id() == 0) {
-    bb_store(d.leaf_bb + 8 * (size_t)leaf, acc);
-    bb_store(d.leaf_obb + 8 * (size_t)leaf, acc);
+    bb_store(d.leaf_bb + 8 * (size_t)leaf, acc, lag);
+    bb_store(d.leaf_obb + 8 * (size_t)leaf, acc, lag);
     nsh += sr.y - sr.x;
   }
 }
 
 // The box over a leaf's vertices (uniq range vr, then its shared vertices sr) in
-// vert_indices order; lane 0 holds the result.
-__device__ __forceinline__ BB6 leaf_box(const SgDevView &d, int2 vr, int2 sr) {
+// vert_indices order; lane 0 holds the result.  lag (every lane): a vertex is a NaN.
+__device__ __forceinline__ BB6 leaf_box(const SgDevView &d, int2 vr, int2 sr, bool &lag) {
   const int nu = vr.y - vr.x, ns = sr.y - sr.x, tot = nu + ns;
   const int per = (tot + SG_WAVE - 1) / SG_WAVE;
   const int lane = lane_id();
   BB6 acc;
   bb_reset(acc);
+  bool nan = false;
   for (int q0 = 0; q0 < per; q0 += 8) {
     int vid[8];
 #pragma unroll
@@ -613,9 +619,13 @@ __device__ __forceinline__ BB6 leaf_box(const SgDevView &d, int2 vr, int2 sr) {
     }
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-      if (vid[j] >= 0) bb_add_point(acc, x[j], y[j], z[j]);
+      if (vid[j] >= 0) {
+        bb_add_point(acc, x[j], y[j], z[j]);
+        nan = nan || x[j] != x[j] || y[j] != y[j] || z[j] != z[j];
+      }
     }
   }
+  lag = __any(nan);
   return bb_wave_reduce(acc);
 }
 

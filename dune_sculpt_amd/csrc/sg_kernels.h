@@ -133,6 +133,7 @@ int sg_enqueue_normals_list(PBVH *p, const int *leaves_dev, int n);
 int sg_enqueue_coords_apply(PBVH *p, const float *src_dev);
 int sg_enqueue_leaf_boxes(PBVH *p, const int *leaves_dev, int n, float *out_dev);
 int sg_enqueue_scatter_boxes(PBVH *p, const void *recs_dev, int n);
+int sg_enqueue_box_lag(PBVH *p, const int *leaves_dev, int n);
 int sg_enqueue_set_marks(PBVH *p, const int *verts_dev, int n);
 int sg_enqueue_finish(PBVH *p, int serial_last);
 int sg_enqueue_gather(PBVH *p, int which, float *out_dev);
