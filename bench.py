@@ -36,11 +36,11 @@ sys.path.insert(0, str(ROOT))
 from dune_sculpt_amd.workloads import batch_meshes, batch_table, plain_stroke, smooth_stroke  # noqa: E402
 
 HBM_PEAK_GBPS = 8000.0
-# HBM bytes per dab of the 1000-dab stroke on the 10.5M-vertex mesh (fused dabs), from
+# HBM bytes per dab of the 1000-dab stroke on the 10.5M-vertex mesh (chained fused dabs), from
 # two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE) summed over the dab kernels,
 # FETCH_SIZE scaled by 2.00 and WRITE_SIZE by 1.00 (what they read for a 1 GiB device
 # copy); profiles/dab_step_c2.md holds the commands and the per-kernel figures.
-TRAFFIC_BYTES_PER_DAB = 11_878_502
+TRAFFIC_BYTES_PER_DAB = 13_807_583
 METRIC = "vertex-updates/s + HBM GB/s; learned vs plain Smooth dabs/s at ≤1e-3 RMS"
 NO_PERSISTENT = False  # set from --no-persistent
 
@@ -976,7 +976,7 @@ def main():
     gbps = timed_bytes / elapsed / 1e9
 
     # Roofline of the dab step: the stroke graph is one dependent chain of small kernels
-    # (k_search -> [k_area] -> k_dab_fused per dab), so
+    # (a k_dab_chain launch per dab, after the first dab's k_search and k_area), so
     # its unit is the dab: algorithmic bytes per dab over event time per dab.
     us_per_dab_ev = event_s / (K * args.dabs) * 1e6
     bytes_per_dab = stroke_bytes / args.dabs

@@ -298,9 +298,10 @@ int sg_pbvh_set_grid(PBVH *pbvh, int workgroups);
 /* Workgroups of the brush / post / smooth-step kernels (0 = the common grid). */
 int sg_pbvh_set_kernel_grids(PBVH *pbvh, int brush, int post, int smooth);
 int sg_pbvh_get_kernel_grids(PBVH *pbvh, int out[4]);
-/* Fused dabs: on (default) a plain Draw / Inflate / Grab / Smooth(k <= 4) dab on a
- * triangle mesh runs as the search plus one kernel per gathered leaf over the leaf's
- * halo; off, the separate brush / Smooth-step / normals-and-bounds kernels.  Both give
+/* Fused dabs: on (default) a plain Draw / Inflate / Grab / Smooth dab on a mesh of
+ * triangles and quads runs as one launch (Smooth(k): one per four steps) over its gathered
+ * leaves' halos, which also searches for the next dab of a stroke; off, the separate
+ * search / brush / Smooth-step / normals-and-bounds kernels.  Both give
  * the same bits.  Returns whether the mesh has the halo tables the fused path needs. */
 int sg_pbvh_set_fused(PBVH *pbvh, int on);
 /* Halo tables of the fused dabs: {built, most locals of a leaf (all rings), most
