@@ -80,16 +80,20 @@ __device__ __forceinline__ int aff_count_sum(const SgDevView &d, const CountPref
 // l = lane modulo SG_CH_SEG).  The list is SG_CH_SEG segments by leaf number, each with
 // its own counter line and room for its share of all leaves: one counter took a returning
 // atomic per gathered leaf, 12 ns each (a dab over 1250 leaves waited 15 us on it).
-__device__ __forceinline__ void chain_append(const SgDevView &d, int serial, int l, bool pass, unsigned long long m,
-                                             const int4 &r0, const int4 &r1, int stamp) {
-  const int lane = lane_id(), seg = lane % SG_CH_SEG;
-  // this lane's segment: every SG_CH_SEG-th lane
-  const unsigned long long ms = m & (0x0001000100010001ull << seg);
+__device__ __forceinline__ int chain_reserve(const SgDevView &d, int serial, unsigned long long m) {
+  const int lane = lane_id();
+  const unsigned long long ms = m & (0x0001000100010001ull << lane % SG_CH_SEG);  // the segment's lanes
   int base = 0;
   if (lane < SG_CH_SEG && ms)
-    base = (int)atomicAdd((unsigned long long *)&d.ch_ctr[((size_t)(serial % 3) * SG_CH_SEG + seg) * SG_CH_CTR],
+    base = (int)atomicAdd((unsigned long long *)&d.ch_ctr[((size_t)(serial % 3) * SG_CH_SEG + lane) * SG_CH_CTR],
                           (unsigned long long)__popcll(ms));
-  base = __shfl(base, seg);
+  return base;  // of segment `lane`
+}
+__device__ __forceinline__ void chain_append(const SgDevView &d, int serial, int l, bool pass, unsigned long long m,
+                                             int reserved, const int4 &r0, const int4 &r1, int stamp) {
+  const int seg = lane_id() % SG_CH_SEG;
+  const unsigned long long ms = m & (0x0001000100010001ull << seg);
+  const int base = __shfl(reserved, seg);
   if (pass) {
     const size_t q = (size_t)(serial % 3) * d.ch_cap * SG_CH_SEG + (size_t)seg * d.ch_cap + (size_t)(base + mask_prefix(ms));
     d.ch_leaf[q] = l;
@@ -192,20 +196,27 @@ __global__ __launch_bounds__(256) void k_search(SgDevView d, SgDabK k, long long
     }
     const int cut = d.leaf_cut[lc];
     const int stamp = d.dstamp ? d.dstamp[0] + serial : 0;
+    // a fused dab (the first of a chain) has the chain's list; its area normal, and every
+    // dab that is not fused, reads the plain one.  Both reservations before either's use.
+    const bool plain = !k.fused || k.tool == SG_TOOL_DRAW;
+    const int cbase = k.fused ? chain_reserve(d, serial, m) : 0;
     int wbase = 0;
-    if (lane == 0) wbase = (int)atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], (unsigned long long)__popcll(m));
+    if (plain && lane == 0)
+      wbase = (int)atomicAdd((unsigned long long *)&d.ctr[SG_CTR_NGATHER], (unsigned long long)__popcll(m));
+    if (k.fused) chain_append(d, serial, l, pass, m, cbase, r0, r1, stamp);
     wbase = __shfl(wbase, 0);
     if (pass) {
-      const int pos = wbase + mask_prefix(m);
-      d.gathered[pos] = l;
-      d.gl_v[pos] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
-      d.gl_s[pos] = make_int2(r0.y, r0.y + (r1.x >> 16));
+      if (plain) {
+        const int pos = wbase + mask_prefix(m);
+        d.gathered[pos] = l;
+        d.gl_v[pos] = make_int2(r0.x, r0.x + (r1.x & 0xffff));
+        d.gl_s[pos] = make_int2(r0.y, r0.y + (r1.x >> 16));
+      }
       // the subtree's flags (every passing leaf of it writes the same values)
       d.cut_touch[cut] = serial;
       d.cut_dirty[cut] = 1;
       d.draw_dirty[cut] = 1;  // the subtree's leaves need new draw records (UpdateDrawBuffers)
     }
-    if (k.fused) chain_append(d, serial, l, pass, m, r0, r1, stamp);  // the first dab of a chain
     return;
   }
   // subtree waves
@@ -962,7 +973,7 @@ __device__ __forceinline__ void chain_search(const SgDevView &d, const SgDabK &k
   if (m) {
     r0 = d.hl_rec[2 * (size_t)lc];
     r1 = d.hl_rec[2 * (size_t)lc + 1];
-    chain_append(d, ls + 1, l, pass, m, r0, r1, gstamp + 1);
+    chain_append(d, ls + 1, l, pass, m, chain_reserve(d, ls + 1, m), r0, r1, gstamp + 1);
   }
   if (kn.tool != SG_TOOL_DRAW) return;
   // The area normal's share of the new leaves that reach into its sphere (usually none: the dab
